@@ -209,8 +209,13 @@ struct InteriorLaunch {
     int x_chunk;
 };
 
+// Tile of the x sweeps (sweep.h): rows along y, and the number of tiles along z.
+struct SweepTile {
+    int rows = 0, ntz = 0;
+};
+
 // Up to four (x, y) boxes of interior rows, all of z, that one launch of the
-// pair sweeps covers, blocks numbered box by box (the launch fills first,
+// x sweeps covers, blocks numbered box by box (the launch fills first,
 // tyn and xc from the tile shape).  The whole interior is one box; the
 // rows around the fused step's box are four.
 struct Boxes {
@@ -235,19 +240,26 @@ struct Boxes {
 //             literal coefficients (constant media).
 // Values, term order and fma accumulation equal bc_point's, so the fields
 // are those of the boundary launches bit for bit.
-// coefficient block in device memory, staged into LDS once per block
+// coefficient block in device memory
 struct ZCoef {
-    float rc[2][2][9];     // recompute literals [low, high][Txx, Tyy][term]
+    float rc[9][2];        // recompute literals [term][Txx, Tyy], the same at both faces
     float zc[2][3][MAXM];  // image coefficients [low, high][Tzz, Tyz, Txz][k]
 };
 constexpr int ZCOEF_WORDS = (int)(sizeof(ZCoef) / 4);
 static_assert(sizeof(ZCoef) % 4 == 0, "ZCoef is copied as 32-bit words");
+// the recompute literals in the form the sweep keeps in scalar registers:
+// sum along x  -x[1] U(x-2) - x[0] U(x-1) + x[0] U(x) + x[1] U(x+1), the same
+// along y with V, then 1 T(t0) (the host checks that the nine terms are these)
+struct ZRecompute {
+    float x[2][2], y[2][2];   // [k][Txx, Tyy]
+};
 // scalar part, passed by value
 struct ZFaceArgs {
     int F = 0;        // 0: off
     int rec = 0;      // recompute statements present
     int n1 = 0, npts = 0;
     const ZCoef* coef = nullptr;
+    ZRecompute rc = {};
 };
 
 // `boxes` (x0..y1 and n set) restricts the update to those rows; it needs
@@ -255,6 +267,12 @@ struct ZFaceArgs {
 hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                          const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
                          const ZFaceArgs* zf = nullptr, const void* pool = nullptr, const Boxes* boxes = nullptr);
+// the flat-tile stress sweep (stress.hip) and whether it takes these
+// coefficients
+hipError_t launch_stress_sweep(const Geom& g, int real_bytes, int storage, bool het, const void* fields,
+                               const void* media, const void* coefs, int t0, int t1, const InteriorLaunch& cfg,
+                               hipStream_t s, const ZFaceArgs* zf, const Boxes* boxes);
+bool stress_sweep_applies(int real_bytes, bool het, const void* coefs, int m);
 // whether launch_stress applies ZFaceArgs for this configuration
 bool stress_applies_zfaces(int real_bytes, bool het, const InteriorLaunch& cfg);
 hipError_t launch_velocity(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,

@@ -19,10 +19,12 @@
 // the read path.  Arithmetic in the compute type R (float or double); fields
 // stored as S (float, double, _Float16, bf16).
 //
-// Three implementations (kernel_variant):
-//  * 0, pair sweep (default for FP32 arithmetic, any storage): the sweep below
-//    with two z points per lane and 128(z) x TY(y) tiles; FP64 uses 2.
-//  * 2, sweep: a block owns a 64(z) x TY(y) column tile and sweeps x.
+// Implementations (kernel_variant):
+//  * stress, 0 and 2: the flat-tile sweep of stress.hip (2 leaves the z-face
+//    statements to their own launch).
+//  * velocity, 0 (FP32 arithmetic): a sweep with two z points per lane and
+//    128(z) x TY(y) tiles; 2, and every FP64 sweep: one point per lane, 64(z) x
+//    TY(y) tiles.
 //    Fields differentiated along x live in per-thread register queues, the
 //    current x plane of fields differentiated along y or z is staged with its
 //    halo in LDS, so every field is read from HBM once per sweep.  Blocks are
@@ -31,8 +33,9 @@
 //    store are non-temporal (streamed once); only the stencil operands, whose
 //    halo lines neighbouring tiles re-read, are ordinary cached loads.
 //  * 1, gather: one thread per (y,z) column, every stencil operand loaded from
-//    global memory (caches only); kept as the simple reference form.
-// All three keep one accumulation order, so their results agree bit for bit.
+//    global memory (caches only); kept as the simple reference form, and the
+//    stress kernel of models whose off-axis normal coefficients differ.
+// All keep one accumulation order, so their results agree bit for bit.
 #include "common.h"
 
 #include <algorithm>
@@ -263,133 +266,6 @@ struct Staged {
 };
 
 template <typename R, typename S, int M, int TY, bool HET>
-__global__ __launch_bounds__(64 * TY) void stress_sweep(Geom g, FieldPtrs<S> F, MediaPtrs<R> md, Coefs<R> c,
-                                                        int t0, int t1, int tz, int ty, int xchunk, int nblocks) {
-    using P = Plane<M, TY>;
-    using C = Conv<S, R>;
-    __shared__ R sU[2][P::H * P::W], sV[2][P::H * P::W], sW[2][P::H * P::W];
-    const int l = logical_block(nblocks);
-    if (l < 0) return;
-    const int bz = l % tz, by = (l / tz) % ty, bx = l / (tz * ty);
-    const int lz = threadIdx.x & 63, ly = threadIdx.x >> 6;
-    const int z0 = M + bz * 64, y0 = M + by * TY;
-    const int z = z0 + lz, y = y0 + ly;
-    const bool active = z < g.nz - M && y < g.ny - M;
-    const int64_t col = (int64_t)min(y, g.ny - 1) * g.sy + min(z, g.nz - 1);
-    const int xb = M + bx * xchunk, xe = min(xb + xchunk, g.nx - M);
-    const S* U0 = F.f[0][t0];
-    const S* V0 = F.f[1][t0];
-    const S* W0 = F.f[2][t0];
-    HaloSlots<M, TY> hs;
-    hs.init(g, y0, z0);
-    // register queues along x: qU[i] = U(x+i-M), qV[i] = V(x+i-M+1), qW[i] = W(x+i-M+1)
-    R qU[2 * M], qV[2 * M], qW[2 * M];
-#pragma unroll
-    for (int i = 1; i < 2 * M; ++i) {
-        qU[i] = C::ld(U0 + (int64_t)(xb - M - 1 + i) * g.sx + col);
-        qV[i] = C::ld(V0 + (int64_t)(xb - M + i) * g.sx + col);
-        qW[i] = C::ld(W0 + (int64_t)(xb - M + i) * g.sx + col);
-    }
-    // values of the next plane, fetched one iteration ahead
-    R nU, nV, nW, nT[6];
-    Staged<R, M, TY, true, true> nhU, nhV, nhW;
-    auto fetch = [&](int x) {
-        const int64_t px = (int64_t)x * g.sx;
-        nU = C::ld(U0 + px + (int64_t)(M - 1) * g.sx + col);
-        nV = C::ld(V0 + px + (int64_t)M * g.sx + col);
-        nW = C::ld(W0 + px + (int64_t)M * g.sx + col);
-#pragma unroll
-        for (int f = 0; f < 6; ++f) nT[f] = C::ldnt(F.f[3 + f][t0] + px + col);
-        nhU.fetch(U0, px, hs);
-        nhV.fetch(V0, px, hs);
-        nhW.fetch(W0, px, hs);
-    };
-    fetch(xb);
-    for (int x = xb; x < xe; ++x) {
-        const int b = (x - xb) & 1;
-#pragma unroll
-        for (int i = 0; i < 2 * M - 1; ++i) {
-            qU[i] = qU[i + 1];
-            qV[i] = qV[i + 1];
-            qW[i] = qW[i + 1];
-        }
-        qU[2 * M - 1] = nU;
-        qV[2 * M - 1] = nV;
-        qW[2 * M - 1] = nW;
-        R T0[6];
-#pragma unroll
-        for (int f = 0; f < 6; ++f) T0[f] = nT[f];
-        R* LU = sU[b];
-        R* LV = sV[b];
-        R* LW = sW[b];
-        const int me = (ly + M) * P::W + lz + M;
-        LU[me] = qU[M];
-        LV[me] = qV[M - 1];
-        LW[me] = qW[M - 1];
-        nhU.put(LU, hs);
-        nhV.put(LV, hs);
-        nhW.put(LW, hs);
-        if (x + 1 < xe) fetch(x + 1);
-        __syncthreads();
-        if (active) {
-            const int64_t q = (int64_t)x * g.sx + col;
-            R dx[M], dy[M], dz[M];
-#pragma unroll
-            for (int k = 0; k < M; ++k) {
-                dx[k] = qU[M + k] - qU[M - 1 - k];
-                dy[k] = LV[me + k * P::W] - LV[me - (1 + k) * P::W];
-                dz[k] = LW[me + k] - LW[me - 1 - k];
-            }
-            R lam = 0, l2m = 0;
-            if (HET) {
-                lam = __builtin_nontemporal_load(md.m[OPESCI_M_LAMBDA] + q);
-                l2m = lam + (R)2 * __builtin_nontemporal_load(md.m[OPESCI_M_MU] + q);
-            }
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                R acc = T0[i];
-                R s = 0;
-#pragma unroll
-                for (int k = 0; k < M; ++k) s = fmac(c.cn[i][0][k], dx[k], s);
-                acc = HET ? fmac(i == 0 ? l2m : lam, s, acc) : acc + s;
-                s = 0;
-#pragma unroll
-                for (int k = 0; k < M; ++k) s = fmac(c.cn[i][1][k], dy[k], s);
-                acc = HET ? fmac(i == 1 ? l2m : lam, s, acc) : acc + s;
-                s = 0;
-#pragma unroll
-                for (int k = 0; k < M; ++k) s = fmac(c.cn[i][2][k], dz[k], s);
-                acc = HET ? fmac(i == 2 ? l2m : lam, s, acc) : acc + s;
-                C::stnt(F.f[3 + i][t1] + q, acc);
-            }
-            // Txy: dU/dy then dV/dx;  Tyz: dV/dz then dW/dy;  Txz: dU/dz then dW/dx
-            R sxy = 0, syz = 0, sxz = 0;
-#pragma unroll
-            for (int k = 0; k < M; ++k) sxy = fmac(c.cs[0][0][k], LU[me + (1 + k) * P::W] - LU[me - k * P::W], sxy);
-#pragma unroll
-            for (int k = 0; k < M; ++k) sxy = fmac(c.cs[0][1][k], qV[M + k] - qV[M - 1 - k], sxy);
-#pragma unroll
-            for (int k = 0; k < M; ++k) syz = fmac(c.cs[1][0][k], LV[me + 1 + k] - LV[me - k], syz);
-#pragma unroll
-            for (int k = 0; k < M; ++k) syz = fmac(c.cs[1][1][k], LW[me + (1 + k) * P::W] - LW[me - k * P::W], syz);
-#pragma unroll
-            for (int k = 0; k < M; ++k) sxz = fmac(c.cs[2][0][k], LU[me + 1 + k] - LU[me - k], sxz);
-#pragma unroll
-            for (int k = 0; k < M; ++k) sxz = fmac(c.cs[2][1][k], qW[M + k] - qW[M - 1 - k], sxz);
-            if (HET) {
-                C::stnt(F.f[6][t1] + q, fmac(__builtin_nontemporal_load(md.m[OPESCI_M_MU12] + q), sxy, T0[3]));
-                C::stnt(F.f[7][t1] + q, fmac(__builtin_nontemporal_load(md.m[OPESCI_M_MU23] + q), syz, T0[4]));
-                C::stnt(F.f[8][t1] + q, fmac(__builtin_nontemporal_load(md.m[OPESCI_M_MU13] + q), sxz, T0[5]));
-            } else {
-                C::stnt(F.f[6][t1] + q, T0[3] + sxy);
-                C::stnt(F.f[7][t1] + q, T0[4] + syz);
-                C::stnt(F.f[8][t1] + q, T0[5] + sxz);
-            }
-        }
-    }
-}
-
-template <typename R, typename S, int M, int TY, bool HET>
 __global__ __launch_bounds__(64 * TY) void velocity_sweep(Geom g, FieldPtrs<S> F, MediaPtrs<R> md, Coefs<R> c,
                                                           int t0, int t1, int tz, int ty, int xchunk, int nblocks) {
     using P = Plane<M, TY>;
@@ -617,256 +493,6 @@ template <typename S>
 __device__ __forceinline__ float lane_read(float v, int lane) {
     const float r = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
     return Conv<S, float>::from(Conv<S, float>::to(r));
-}
-
-template <typename S, int M, int TY, bool HET, bool ZF>
-__global__ __launch_bounds__(64 * TY) void stress_sweep2(Geom g, FieldPtrs<S> F, MediaPtrs<float> md,
-                                                         Coefs<float> c, int t0, int t1, int tz, int nblocks,
-                                                         Boxes B, ZFaceArgs zf) {
-    using R = float;
-    using P = Plane2<M, TY>;
-    __shared__ R sU[2][P::H * P::W], sV[2][P::H * P::W], sW[2][P::H * P::W];
-    const int l = logical_block(nblocks);
-    if (l < 0) return;
-    const TileOrigin o = tile_of<TY>(B, l, tz, M);
-    const int lz = threadIdx.x & 63, ly = threadIdx.x >> 6;
-    const int z0 = o.z0, y0 = o.y0;
-    const int z = z0 + 2 * lz, y = y0 + ly;
-    const bool act0 = z < g.nz - M && y < o.yend, act1 = z + 1 < g.nz - M && y < o.yend;
-    const int64_t col = (int64_t)min(y, g.ny - 1) * g.sy + pair_start(g, z);
-    const int xb = o.xb, xe = o.xe;
-    const S* U0 = F.f[0][t0];
-    const S* V0 = F.f[1][t0];
-    const S* W0 = F.f[2][t0];
-    HaloSlots2<M, TY> hs;
-    hs.init(g, y0, z0);
-    static_assert(!(ZF && HET), "in-sweep z faces are built for constant media");
-    // z-face statements: coefficient block staged in LDS once per block (kept
-    // out of the kernel arguments, whose scalar registers it would exhaust)
-    __shared__ ZCoef zl;
-    const int zrh = g.nz - M - 1 - z0;                 // high face relative to the tile
-    const bool zlo = z0 == M, zhi = zrh >= 0 && zrh < 128;
-    const int zlane = zlo && (threadIdx.x & 63) == 0 ? 0 : (zhi && (int)(threadIdx.x & 63) == (zrh >> 1) ? 1 : -1);
-    if constexpr (ZF) {
-        for (int w = threadIdx.x; w < ZCOEF_WORDS; w += blockDim.x)
-            reinterpret_cast<int*>(&zl)[w] = reinterpret_cast<const int*>(zf.coef)[w];
-        __syncthreads();
-    }
-    // per point v: qU[v][i] = U(x+i-M), qV[v][i] = V(x+i-M+1), qW[v][i] = W(x+i-M+1)
-    R qU[2][2 * M], qV[2][2 * M], qW[2][2 * M];
-#pragma unroll
-    for (int i = 1; i < 2 * M; ++i) {
-        ld2(U0 + (int64_t)(xb - M - 1 + i) * g.sx + col, qU[0][i], qU[1][i]);
-        ld2(V0 + (int64_t)(xb - M + i) * g.sx + col, qV[0][i], qV[1][i]);
-        ld2(W0 + (int64_t)(xb - M + i) * g.sx + col, qW[0][i], qW[1][i]);
-    }
-    R nU[2], nV[2], nW[2], nT[6][2];
-    Staged2<M, TY, true, true> nhU, nhV, nhW;
-    auto fetch = [&](int x) {
-        const int64_t px = (int64_t)x * g.sx;
-        ld2(U0 + px + (int64_t)(M - 1) * g.sx + col, nU[0], nU[1]);
-        ld2(V0 + px + (int64_t)M * g.sx + col, nV[0], nV[1]);
-        ld2(W0 + px + (int64_t)M * g.sx + col, nW[0], nW[1]);
-#pragma unroll
-        for (int f = 0; f < 6; ++f) ldnt2(F.f[3 + f][t0] + px + col, nT[f][0], nT[f][1]);
-        nhU.fetch(U0, px, hs);
-        nhV.fetch(V0, px, hs);
-        nhW.fetch(W0, px, hs);
-    };
-    fetch(xb);
-    for (int x = xb; x < xe; ++x) {
-        const int b = (x - xb) & 1;
-#pragma unroll
-        for (int v = 0; v < 2; ++v) {
-#pragma unroll
-            for (int i = 0; i < 2 * M - 1; ++i) {
-                qU[v][i] = qU[v][i + 1];
-                qV[v][i] = qV[v][i + 1];
-                qW[v][i] = qW[v][i + 1];
-            }
-            qU[v][2 * M - 1] = nU[v];
-            qV[v][2 * M - 1] = nV[v];
-            qW[v][2 * M - 1] = nW[v];
-        }
-        R T0[6][2];
-#pragma unroll
-        for (int f = 0; f < 6; ++f) {
-            T0[f][0] = nT[f][0];
-            T0[f][1] = nT[f][1];
-        }
-        R* LU = sU[b];
-        R* LV = sV[b];
-        R* LW = sW[b];
-        const int me0 = (ly + M) * P::W + 2 * lz + M;
-#pragma unroll
-        for (int v = 0; v < 2; ++v) {
-            LU[me0 + v] = qU[v][M];
-            LV[me0 + v] = qV[v][M - 1];
-            LW[me0 + v] = qW[v][M - 1];
-        }
-        nhU.put(LU, hs);
-        nhV.put(LV, hs);
-        nhW.put(LW, hs);
-        if (x + 1 < xe) fetch(x + 1);
-        __syncthreads();
-        if (act0) {
-            const int64_t q = (int64_t)x * g.sx + col;
-            R out[6][2];
-            mpair_t mlam, mmu, m12, m23, m13;
-            if (HET) {
-                mlam = media2(md.m[OPESCI_M_LAMBDA] + q);
-                mmu = media2(md.m[OPESCI_M_MU] + q);
-                m12 = media2(md.m[OPESCI_M_MU12] + q);
-                m23 = media2(md.m[OPESCI_M_MU23] + q);
-                m13 = media2(md.m[OPESCI_M_MU13] + q);
-            }
-#pragma unroll
-            for (int v = 0; v < 2; ++v) {
-                const int me = me0 + v;
-                R dx[M], dy[M], dz[M];
-#pragma unroll
-                for (int k = 0; k < M; ++k) {
-                    dx[k] = qU[v][M + k] - qU[v][M - 1 - k];
-                    dy[k] = LV[me + k * P::W] - LV[me - (1 + k) * P::W];
-                    dz[k] = LW[me + k] - LW[me - 1 - k];
-                }
-                R lam = 0, l2m = 0;
-                if (HET) {
-                    lam = mlam[v];
-                    l2m = lam + (R)2 * mmu[v];
-                }
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    R acc = T0[i][v];
-                    R s = 0;
-#pragma unroll
-                    for (int k = 0; k < M; ++k) s = fmac(c.cn[i][0][k], dx[k], s);
-                    acc = HET ? fmac(i == 0 ? l2m : lam, s, acc) : acc + s;
-                    s = 0;
-#pragma unroll
-                    for (int k = 0; k < M; ++k) s = fmac(c.cn[i][1][k], dy[k], s);
-                    acc = HET ? fmac(i == 1 ? l2m : lam, s, acc) : acc + s;
-                    s = 0;
-#pragma unroll
-                    for (int k = 0; k < M; ++k) s = fmac(c.cn[i][2][k], dz[k], s);
-                    acc = HET ? fmac(i == 2 ? l2m : lam, s, acc) : acc + s;
-                    out[i][v] = acc;
-                }
-                R sxy = 0, syz = 0, sxz = 0;
-#pragma unroll
-                for (int k = 0; k < M; ++k) sxy = fmac(c.cs[0][0][k], LU[me + (1 + k) * P::W] - LU[me - k * P::W], sxy);
-#pragma unroll
-                for (int k = 0; k < M; ++k) sxy = fmac(c.cs[0][1][k], qV[v][M + k] - qV[v][M - 1 - k], sxy);
-#pragma unroll
-                for (int k = 0; k < M; ++k) syz = fmac(c.cs[1][0][k], LV[me + 1 + k] - LV[me - k], syz);
-#pragma unroll
-                for (int k = 0; k < M; ++k) syz = fmac(c.cs[1][1][k], LW[me + (1 + k) * P::W] - LW[me - k * P::W], syz);
-#pragma unroll
-                for (int k = 0; k < M; ++k) sxz = fmac(c.cs[2][0][k], LU[me + 1 + k] - LU[me - k], sxz);
-#pragma unroll
-                for (int k = 0; k < M; ++k) sxz = fmac(c.cs[2][1][k], qW[v][M + k] - qW[v][M - 1 - k], sxz);
-                if (HET) {
-                    out[3][v] = fmac(m12[v], sxy, T0[3][v]);
-                    out[4][v] = fmac(m23[v], syz, T0[4][v]);
-                    out[5][v] = fmac(m13[v], sxz, T0[5][v]);
-                } else {
-                    out[3][v] = T0[3][v] + sxy;
-                    out[4][v] = T0[4][v] + syz;
-                    out[5][v] = T0[5][v] + sxz;
-                }
-            }
-            if constexpr (ZF) {
-                // free-surface statements of the z faces on the deep rows (the
-                // wave is one row: x and y are wave-uniform)
-                if (x >= zf.F && x < g.nx - zf.F && y >= zf.F && y < g.ny - zf.F) {
-                    const int64_t row = (int64_t)x * g.sx + (int64_t)y * g.sy;
-                    const int rh = zrh;
-                    // image sources [face][Tzz, Tyz, Txz][k] (interior values,
-                    // before any replacement), read from the lanes holding
-                    // them while every interior lane is active
-                    float src[2][3][M];
-#pragma unroll
-                    for (int k = 0; k < M; ++k) {
-                        if (zlo) {
-                            src[0][0][k] = k >= 1 ? lane_read<S>(out[2][k & 1], k >> 1) : 0.0f;
-                            src[0][1][k] = lane_read<S>(out[4][k & 1], k >> 1);
-                            src[0][2][k] = lane_read<S>(out[5][k & 1], k >> 1);
-                        }
-                        if (zhi) {
-                            const int r0 = rh - k, r1 = rh - 1 - k;
-                            src[1][0][k] = k >= 1 ? lane_read<S>((r0 & 1) ? out[2][1] : out[2][0], r0 >> 1) : 0.0f;
-                            src[1][1][k] = lane_read<S>((r1 & 1) ? out[4][1] : out[4][0], r1 >> 1);
-                            src[1][2][k] = lane_read<S>((r1 & 1) ? out[5][1] : out[5][0], r1 >> 1);
-                        }
-                    }
-                    // the lane holding a surface point: its face's Levander
-                    // recompute of Txx and Tyy (one pass over the nine terms,
-                    // point element e), surface values and ghost cells
-                    if (zlane >= 0) {
-                        const int face = zlane, e = face ? (rh & 1) : 0;
-                        float rxx = 0.0f, ryy = 0.0f;
-                        if constexpr (M == 2) {
-                            if (zf.rec) {
-#pragma unroll
-                                for (int k = 0; k < 8; ++k) {
-                                    const float v = k < 4 ? (e ? qU[1][k] : qU[0][k]) : LV[me0 + e + (k - 6) * P::W];
-                                    rxx = fmac(zl.rc[face][0][k], v, rxx);
-                                    ryy = fmac(zl.rc[face][1][k], v, ryy);
-                                }
-                                rxx = fmac(zl.rc[face][0][8], e ? T0[0][1] : T0[0][0], rxx);
-                                ryy = fmac(zl.rc[face][1][8], e ? T0[1][1] : T0[1][0], ryy);
-                            }
-                        }
-                        float sv[3][M];
-#pragma unroll
-                        for (int f = 0; f < 3; ++f)
-#pragma unroll
-                            for (int k = 0; k < M; ++k) sv[f][k] = face ? src[1][f][k] : src[0][f][k];
-                        // ghost cells: ordinary stores, so the few cells of
-                        // each face line merge in L2 before they reach HBM
-                        using CS = Conv<S, float>;
-                        if (face == 0) {
-#pragma unroll
-                            for (int k = 0; k < M; ++k) {
-                                if (k >= 1) CS::st(F.f[5][t1] + row + M - k, fmac(zl.zc[0][0][k], sv[0][k], 0.0f));
-                                CS::st(F.f[7][t1] + row + M - 1 - k, fmac(zl.zc[0][1][k], sv[1][k], 0.0f));
-                                CS::st(F.f[8][t1] + row + M - 1 - k, fmac(zl.zc[0][2][k], sv[2][k], 0.0f));
-                            }
-                            if (zf.rec) {
-                                out[0][0] = rxx;
-                                out[1][0] = ryy;
-                            }
-                            out[2][0] = 0.0f;
-                        } else {
-                            const int bhi = g.nz - M - 1;
-#pragma unroll
-                            for (int k = 1; k < M; ++k) {
-                                CS::st(F.f[5][t1] + row + bhi + k, fmac(zl.zc[1][0][k], sv[0][k], 0.0f));
-                                CS::st(F.f[7][t1] + row + bhi + k, fmac(zl.zc[1][1][k], sv[1][k], 0.0f));
-                                CS::st(F.f[8][t1] + row + bhi + k, fmac(zl.zc[1][2][k], sv[2][k], 0.0f));
-                            }
-                            const float tyz = fmac(zl.zc[1][1][0], sv[1][0], 0.0f);
-                            const float txz = fmac(zl.zc[1][2][0], sv[2][0], 0.0f);
-#pragma unroll
-                            for (int v = 0; v < 2; ++v)
-                                if (v == e) {
-                                    if (zf.rec) {
-                                        out[0][v] = rxx;
-                                        out[1][v] = ryy;
-                                    }
-                                    out[2][v] = 0.0f;
-                                    out[4][v] = tyz;
-                                    out[5][v] = txz;
-                                }
-                        }
-                    }
-                }
-            }
-#pragma unroll
-            for (int f = 0; f < 6; ++f)
-                store_points(F.f[3 + f][t1] + q, out[f][0], out[f][1], act0, act1);
-        }
-    }
 }
 
 template <typename S, int M, int TY, bool HET>
@@ -1354,11 +980,11 @@ __global__ __launch_bounds__(64 * (TY + 2 * M)) void step_sweep2(Geom g, StepPtr
                         const float v = k < 4 ? (eh ? qU[1][k] : qU[0][k])
                                               : (k < 8 ? vV[vme0 + eh + (k - 6) * T::VW] : 0.0f);
                         if (k < 8) {
-                            rxx = fmac(zl.rc[face][0][k], v, rxx);
-                            ryy = fmac(zl.rc[face][1][k], v, ryy);
+                            rxx = fmac(zl.rc[k][0], v, rxx);
+                            ryy = fmac(zl.rc[k][1], v, ryy);
                         } else {
-                            rxx = fmac(zl.rc[face][0][k], eh ? T0[0][1] : T0[0][0], rxx);
-                            ryy = fmac(zl.rc[face][1][k], eh ? T0[1][1] : T0[1][0], ryy);
+                            rxx = fmac(zl.rc[k][0], eh ? T0[0][1] : T0[0][0], rxx);
+                            ryy = fmac(zl.rc[k][1], eh ? T0[1][1] : T0[1][0], ryy);
                         }
                     }
                 }
@@ -1651,8 +1277,7 @@ static int default_tile_y() {
 
 template <typename R, typename S, int M, bool HET, bool VEL>
 static hipError_t run_interior(const Geom& g, void* fields, const void* media, const void* coefs, int t0, int t1,
-                               const InteriorLaunch& cfg, hipStream_t s, const ZFaceArgs* zf, const void* pool,
-                               const Boxes* boxes) {
+                               const InteriorLaunch& cfg, hipStream_t s, const Boxes* boxes) {
     const FieldPtrs<S>& F = *static_cast<const FieldPtrs<S>*>(fields);
     const MediaPtrs<R>& md = *static_cast<const MediaPtrs<R>*>(media);
     const Coefs<R>& c = *static_cast<const Coefs<R>*>(coefs);
@@ -1668,6 +1293,9 @@ static hipError_t run_interior(const Geom& g, void* fields, const void* media, c
                                t.tz, t.tyn, t.xchunk, t.nb);
         return hipGetLastError();
     }
+    if constexpr (!VEL) {
+        return hipErrorInvalidValue;   // the stress sweeps are launch_stress_sweep's
+    } else {
     if constexpr (sizeof(R) == 4) {
         if (cfg.variant == 0) {
             // FP32 arithmetic: the pair sweeps (two z points per lane, 128-wide
@@ -1700,15 +1328,8 @@ static hipError_t run_interior(const Geom& g, void* fields, const void* media, c
             const int grid = ((nb + 7) / 8) * 8;
 #define OPESCI_PAIR(TYV)                                                                                        \
     if (ty == TYV) {                                                                                            \
-        if (VEL)                                                                                                \
-            hipLaunchKernelGGL((velocity_sweep2<S, M, TYV, HET>), dim3(grid), dim3(64 * TYV), 0, s, g, F, md, c,   \
-                               t0, t1, tz, nb, B);                                                              \
-        else if (zf && zf->F > 0)                                                                               \
-            hipLaunchKernelGGL((stress_sweep2<S, M, TYV, false, true>), dim3(grid), dim3(64 * TYV), 0, s, g, F,     \
-                               md, c, t0, t1, tz, nb, B, *zf);                                                  \
-        else                                                                                                    \
-            hipLaunchKernelGGL((stress_sweep2<S, M, TYV, HET, false>), dim3(grid), dim3(64 * TYV), 0, s, g, F, md, \
-                               c, t0, t1, tz, nb, B, ZFaceArgs());                                              \
+        hipLaunchKernelGGL((velocity_sweep2<S, M, TYV, HET>), dim3(grid), dim3(64 * TYV), 0, s, g, F, md, c,       \
+                           t0, t1, tz, nb, B);                                                                  \
         return hipGetLastError();                                                                               \
     }
             OPESCI_PAIR(4)
@@ -1727,42 +1348,30 @@ static hipError_t run_interior(const Geom& g, void* fields, const void* media, c
     const int tile_y = cfg.tile_y ? cfg.tile_y : default_tile_y<R, S, HET>();
     if (tile_y == 16) {
         const Tiling t = tiling<M>(g, cfg, 16);
-        if (VEL)
-            hipLaunchKernelGGL((velocity_sweep<R, S, M, 16, HET>), dim3(t.grid), dim3(1024), 0, s, g, F, md, c, t0, t1,
-                               t.tz, t.tyn, t.xchunk, t.nb);
-        else
-            hipLaunchKernelGGL((stress_sweep<R, S, M, 16, HET>), dim3(t.grid), dim3(1024), 0, s, g, F, md, c, t0, t1,
-                               t.tz, t.tyn, t.xchunk, t.nb);
+        hipLaunchKernelGGL((velocity_sweep<R, S, M, 16, HET>), dim3(t.grid), dim3(1024), 0, s, g, F, md, c, t0, t1,
+                           t.tz, t.tyn, t.xchunk, t.nb);
         return hipGetLastError();
     }
     if (tile_y == 4) {
         const Tiling t = tiling<M>(g, cfg, 4);
-        if (VEL)
-            hipLaunchKernelGGL((velocity_sweep<R, S, M, 4, HET>), dim3(t.grid), dim3(256), 0, s, g, F, md, c, t0, t1,
-                               t.tz, t.tyn, t.xchunk, t.nb);
-        else
-            hipLaunchKernelGGL((stress_sweep<R, S, M, 4, HET>), dim3(t.grid), dim3(256), 0, s, g, F, md, c, t0, t1,
-                               t.tz, t.tyn, t.xchunk, t.nb);
+        hipLaunchKernelGGL((velocity_sweep<R, S, M, 4, HET>), dim3(t.grid), dim3(256), 0, s, g, F, md, c, t0, t1,
+                           t.tz, t.tyn, t.xchunk, t.nb);
         return hipGetLastError();
     }
     const Tiling t = tiling<M>(g, cfg, 8);
-    if (VEL)
-        hipLaunchKernelGGL((velocity_sweep<R, S, M, 8, HET>), dim3(t.grid), dim3(512), 0, s, g, F, md, c, t0, t1,
-                           t.tz, t.tyn, t.xchunk, t.nb);
-    else
-        hipLaunchKernelGGL((stress_sweep<R, S, M, 8, HET>), dim3(t.grid), dim3(512), 0, s, g, F, md, c, t0, t1,
-                           t.tz, t.tyn, t.xchunk, t.nb);
+    hipLaunchKernelGGL((velocity_sweep<R, S, M, 8, HET>), dim3(t.grid), dim3(512), 0, s, g, F, md, c, t0, t1,
+                       t.tz, t.tyn, t.xchunk, t.nb);
     return hipGetLastError();
+    }
 }
 
 template <typename R, typename S, bool VEL>
 static hipError_t dispatch_m(const Geom& g, bool het, void* fields, const void* media, const void* coefs, int t0,
-                             int t1, const InteriorLaunch& cfg, hipStream_t s, const ZFaceArgs* zf,
-                             const void* pool, const Boxes* boxes) {
+                             int t1, const InteriorLaunch& cfg, hipStream_t s, const Boxes* boxes) {
 #define OPESCI_CASE(MM)                                                                                          \
     case MM:                                                                                                     \
-        return het ? run_interior<R, S, MM, true, VEL>(g, fields, media, coefs, t0, t1, cfg, s, zf, pool, boxes) \
-                   : run_interior<R, S, MM, false, VEL>(g, fields, media, coefs, t0, t1, cfg, s, zf, pool, boxes);
+        return het ? run_interior<R, S, MM, true, VEL>(g, fields, media, coefs, t0, t1, cfg, s, boxes)           \
+                   : run_interior<R, S, MM, false, VEL>(g, fields, media, coefs, t0, t1, cfg, s, boxes);
     switch (g.m) {
         OPESCI_CASE(1)
         OPESCI_CASE(2)
@@ -1777,14 +1386,14 @@ static hipError_t dispatch_m(const Geom& g, bool het, void* fields, const void* 
 template <bool VEL>
 static hipError_t dispatch(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                            const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
-                           const ZFaceArgs* zf, const void* pool, const Boxes* boxes) {
+                           const Boxes* boxes) {
     if (real_bytes == 8)
-        return dispatch_m<double, double, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, nullptr, nullptr, boxes);
+        return dispatch_m<double, double, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
     if (storage == OPESCI_STORE_F16)
-        return dispatch_m<float, _Float16, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, zf, pool, boxes);
+        return dispatch_m<float, _Float16, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
     if (storage == OPESCI_STORE_BF16)
-        return dispatch_m<float, bf16_t, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, zf, pool, boxes);
-    return dispatch_m<float, float, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, zf, pool, boxes);
+        return dispatch_m<float, bf16_t, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
+    return dispatch_m<float, float, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
 }
 
 // ------------------------------------------------------------------ fused step launch
@@ -1860,14 +1469,22 @@ bool stress_applies_zfaces(int real_bytes, bool het, const InteriorLaunch& cfg) 
 hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                          const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
                          const ZFaceArgs* zf, const void* pool, const Boxes* boxes) {
-    if (zf && zf->F > 0 && !stress_applies_zfaces(real_bytes, het, cfg)) return hipErrorInvalidValue;
-    return dispatch<false>(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, zf, pool, boxes);
+    (void)pool;
+    const bool sweep = cfg.variant != 1 && stress_sweep_applies(real_bytes, het, coefs, g.m);
+    if (zf && zf->F > 0 && !(sweep && stress_applies_zfaces(real_bytes, het, cfg))) return hipErrorInvalidValue;
+    if (boxes && !(sweep && real_bytes == 4 && cfg.variant == 0)) return hipErrorInvalidValue;
+    if (sweep)
+        return launch_stress_sweep(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, zf, boxes);
+    // sums not shared by the normal stresses: the gather kernel takes any coefficients
+    InteriorLaunch gather = cfg;
+    gather.variant = 1;
+    return dispatch<false>(g, real_bytes, storage, het, fields, media, coefs, t0, t1, gather, s, nullptr);
 }
 
 hipError_t launch_velocity(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                            const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
                            const Boxes* boxes) {
-    return dispatch<true>(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, nullptr, nullptr, boxes);
+    return dispatch<true>(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, boxes);
 }
 
 }  // namespace opesci

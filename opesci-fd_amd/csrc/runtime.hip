@@ -450,7 +450,7 @@ int build_zfaces(OpesciContext* c) {
     c->zf = ZFaceArgs();
     const Geom& g = c->g;
     const int M = g.m;
-    if (c->levels[4].size() != 1) return 0;
+    if (c->levels[4].size() != 1 || !stress_sweep_applies(c->real_bytes, c->het, c->coefs(), M)) return 0;
     const int blo = M, bhi = g.nz - M - 1;
     // image sources within the wave that holds the face: 2M interior points
     // on either side, and the high face at least M points into its tile
@@ -501,7 +501,8 @@ int build_zfaces(OpesciContext* c) {
                 const int64_t want_disp = k < 4 ? (k - 2) * g.sx : (k < 8 ? (k - 6) * g.sy : 0);
                 // literal coefficients only (constant media)
                 if (t.fl != want_fl || t.disp != want_disp || t.cslot >= 0) return 0;
-                zc.rc[face][f - 3][k] = t.coef;
+                if (face == 1 && rec[0][f - 3] && zc.rc[k][f - 3] != t.coef) return 0;
+                zc.rc[k][f - 3] = t.coef;
             }
             rec[face][f - 3] = true;
         } else {
@@ -516,6 +517,21 @@ int build_zfaces(OpesciContext* c) {
     const int nrec = rec[0][0] + rec[0][1] + rec[1][0] + rec[1][1];
     if (nrec != 0 && nrec != 4) return 0;
     z.rec = nrec == 4;
+    // the forms the sweep keeps in scalar registers: images negate, the
+    // recompute's sums are antisymmetric and add T(t0) itself
+    for (int face = 0; face < 2; ++face)
+        for (int fi = 0; fi < 3; ++fi)
+            for (int k = fi == 0 ? 1 : 0; k < M; ++k)
+                if (zc.zc[face][fi][k] != -1.0f) return 0;
+    if (z.rec)
+        for (int i = 0; i < 2; ++i) {
+            for (int k = 0; k < 2; ++k) {
+                z.rc.x[k][i] = zc.rc[2 + k][i];
+                z.rc.y[k][i] = zc.rc[6 + k][i];
+                if (zc.rc[1 - k][i] != -z.rc.x[k][i] || zc.rc[5 - k][i] != -z.rc.y[k][i]) return 0;
+            }
+            if (zc.rc[8][i] != 1.0f) return 0;
+        }
     z.F = F;
     z.n1 = g.ny - 2 * F;
     z.npts = (g.nx - 2 * F) * z.n1;

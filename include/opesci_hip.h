@@ -187,9 +187,8 @@ typedef struct OpesciModelDesc {
     /* launch tuning (0 = library default) */
     int32_t tile_y;
     int32_t x_chunk;
-    int32_t kernel_variant;     /* 0 default (LDS/register-queue sweep, two z points per lane
-                                   for FP32 arithmetic), 1 plain gather, 2 sweep with one
-                                   point per lane (the FP64 default) */
+    int32_t kernel_variant;     /* 0 default (LDS/register-queue sweep), 1 plain gather, 2 sweep
+                                   without the z-face statements in the stress kernel */
     int32_t use_graph;          /* capture the time loop in a hipGraph */
     /* adjoint: derivative programs of the media-dependent boundary
      * coefficients (may be 0 / null when no gradient is asked for) */
@@ -273,17 +272,15 @@ int opesci_ctx_kernel_times(OpesciContext* ctx, int32_t nsteps, double out_ms[3]
 /* Execution plan of a context: out[0] = boundary launches per time step,
  * out[1] = phase-4 statements (deep z-face rows of the stress phase),
  * out[2] = launches they take (0 or 1), out[3] = 1 when the stress sweep
- * applies them in place (FP32 pair sweeps), else 0, out[4] = the fused
+ * applies them in place (FP32 sweeps), else 0, out[4] = the fused
  * step's margin F (its box is [F, dim - F) in x and y; 0: separate stress
  * and velocity launches).  No reference counterpart. */
 int opesci_ctx_stats(OpesciContext* ctx, int32_t out[5]);
 
-/* Launch configuration of the interior kernels: kernel_variant 0 = sweep (the
- * FP32 velocity kernel with two z points per lane), 1 = gather, 2 = sweep
- * without the z-face statements in the stress kernel and with one point per
- * lane in the velocity kernel; tile_y 0 (the kernels' own choice) | 4 | 8 | 16
- * rows of a tile at most; x_chunk 0 = chosen from the grid.  Used by the
- * autotuner.  Results do not depend on it (same arithmetic in every
+/* Launch configuration of the interior kernels: kernel_variant 0 = sweep, 1 =
+ * gather, 2 = sweep with the z-face statements of the stress phase left to
+ * their own launch; tile_y 0 (the kernels' own choice) | 4 | 8 | 16 rows of a
+ * tile at most; x_chunk 0 = chosen from the grid.  Used by the autotuner.  Results do not depend on it (same arithmetic in every
  * configuration).  No reference counterpart. */
 int opesci_ctx_configure(OpesciContext* ctx, int32_t kernel_variant, int32_t tile_y, int32_t x_chunk);
 

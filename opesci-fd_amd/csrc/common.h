@@ -202,7 +202,7 @@ int fail(int code, const std::string& msg);
     } while (0)
 
 // ---------------------------------------------------------------- launch wrappers
-// interior kernels (interior.hip); variant 0 = LDS/register-queue sweep, 1 = plain gather
+// interior kernels; variant 0, 2 = flat-tile sweep, 1 = plain gather
 struct InteriorLaunch {
     int variant;
     int tile_y;
@@ -227,7 +227,7 @@ struct Boxes {
 
 
 // Free-surface statements of the stress phase on the z faces, applied by the
-// FP32 pair stress sweep in place, for the deep rows x, y in [F, dim - F)
+// FP32 stress sweep in place, for the deep rows x, y in [F, dim - F)
 // (where they commute with every other statement of the phase, so they may
 // follow the interior update directly).  Per face (b = m low, dim - m - 1
 // high) the statements have three fixed forms, which the host checks
@@ -262,8 +262,7 @@ struct ZFaceArgs {
     ZRecompute rc = {};
 };
 
-// `boxes` (x0..y1 and n set) restricts the update to those rows; it needs
-// the pair sweeps (FP32 arithmetic, kernel variant 0)
+// `boxes` (x0..y1 and n set) restricts the update to those rows (sweeps only)
 hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                          const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
                          const ZFaceArgs* zf = nullptr, const void* pool = nullptr, const Boxes* boxes = nullptr);
@@ -273,6 +272,10 @@ hipError_t launch_stress_sweep(const Geom& g, int real_bytes, int storage, bool 
                                const void* media, const void* coefs, int t0, int t1, const InteriorLaunch& cfg,
                                hipStream_t s, const ZFaceArgs* zf, const Boxes* boxes);
 bool stress_sweep_applies(int real_bytes, bool het, const void* coefs, int m);
+// the flat-tile velocity sweep (velocity.hip)
+hipError_t launch_velocity_sweep(const Geom& g, int real_bytes, int storage, bool het, const void* fields,
+                                 const void* media, const void* coefs, int t0, int t1, const InteriorLaunch& cfg,
+                                 hipStream_t s, const Boxes* boxes);
 // whether launch_stress applies ZFaceArgs for this configuration
 bool stress_applies_zfaces(int real_bytes, bool het, const InteriorLaunch& cfg);
 hipError_t launch_velocity(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,

@@ -20,22 +20,15 @@
 // stored as S (float, double, _Float16, bf16).
 //
 // Implementations (kernel_variant):
-//  * stress, 0 and 2: the flat-tile sweep of stress.hip (2 leaves the z-face
-//    statements to their own launch).
-//  * velocity, 0 (FP32 arithmetic): a sweep with two z points per lane and
-//    128(z) x TY(y) tiles; 2, and every FP64 sweep: one point per lane, 64(z) x
-//    TY(y) tiles.
-//    Fields differentiated along x live in per-thread register queues, the
-//    current x plane of fields differentiated along y or z is staged with its
-//    halo in LDS, so every field is read from HBM once per sweep.  Blocks are
-//    remapped so that the tiles of one XCD form a contiguous slab and share
-//    halo lines in that XCD's L2.  The cell's own previous value and every
-//    store are non-temporal (streamed once); only the stencil operands, whose
-//    halo lines neighbouring tiles re-read, are ordinary cached loads.
-//  * 1, gather: one thread per (y,z) column, every stencil operand loaded from
-//    global memory (caches only); kept as the simple reference form, and the
-//    stress kernel of models whose off-axis normal coefficients differ.
+//  * 0 and 2: the flat-tile sweeps of stress.hip and velocity.hip (sweep.h has
+//    what they share); 2 leaves the z-face statements of the stress phase to
+//    their own launch.
+//  * 1, gather (here): one thread per (y,z) column, every stencil operand
+//    loaded from global memory (caches only); the simple reference form, and
+//    the stress kernel of models whose off-axis normal coefficients differ.
 // All keep one accumulation order, so their results agree bit for bit.
+//
+// Also here: the opt-in fused step.
 #include "common.h"
 
 #include <algorithm>
@@ -178,307 +171,13 @@ __global__ __launch_bounds__(256) void velocity_gather(Geom g, FieldPtrs<S> F, M
     }
 }
 
-// ------------------------------------------------------------------ sweep
-// LDS plane of a 64 x TY tile with an M-cell halo.  Halo cells: the y-halo
-// (M rows above and below, tile columns only) and the z-halo (M columns left
-// and right, tile rows only); corners are never read.
-template <int M, int TY>
-struct Plane {
-    static constexpr int W = 64 + 2 * M;
-    static constexpr int H = TY + 2 * M;
-    static constexpr int NT = 64 * TY;
-    static constexpr int NY = 2 * M * 64;   // y-halo cells
-    static constexpr int NZ = TY * 2 * M;   // z-halo cells
-    static constexpr int JY = (NY + NT - 1) / NT;
-    static_assert(NZ <= NT, "z halo larger than the block");
-    __device__ __forceinline__ static void yhalo(int h, int& row, int& col) {
-        const int r = h / 64;
-        row = r < M ? r : r + TY;
-        col = M + h % 64;
-    }
-    __device__ __forceinline__ static void zhalo(int h, int& row, int& col) {
-        row = M + h / (2 * M);
-        const int c = h % (2 * M);
-        col = c < M ? c : 64 + c;
-    }
-};
-
-// Per-thread halo slots: LDS offset and in-plane global offset of every halo
-// cell this thread stages (-1 = none).
-template <int M, int TY>
-struct HaloSlots {
-    using P = Plane<M, TY>;
-    int ly[P::JY], gy[P::JY];
-    int lz, gz;
-    __device__ void init(const Geom& g, int y0, int z0) {
-        const int t = threadIdx.x;
-#pragma unroll
-        for (int j = 0; j < P::JY; ++j) {
-            const int h = t + j * P::NT;
-            if (h < P::NY) {
-                int row, cl;
-                P::yhalo(h, row, cl);
-                const int yy = min(max(y0 - M + row, 0), g.ny - 1), zz = min(max(z0 - M + cl, 0), g.nz - 1);
-                ly[j] = row * P::W + cl;
-                gy[j] = yy * (int)g.sy + zz;
-            } else {
-                ly[j] = -1;
-                gy[j] = 0;
-            }
-        }
-        if (t < P::NZ) {
-            int row, cl;
-            P::zhalo(t, row, cl);
-            const int yy = min(max(y0 - M + row, 0), g.ny - 1), zz = min(max(z0 - M + cl, 0), g.nz - 1);
-            lz = row * P::W + cl;
-            gz = yy * (int)g.sy + zz;
-        } else {
-            lz = -1;
-            gz = 0;
-        }
-    }
-};
-
-// Values staged for one plane: y-halo and z-halo registers.
-template <typename R, int M, int TY, bool HY, bool HZ>
-struct Staged {
-    using P = Plane<M, TY>;
-    R y[HY ? P::JY : 1];
-    R z;
-    template <typename S>
-    __device__ __forceinline__ void fetch(const S* base, int64_t px, const HaloSlots<M, TY>& hs) {
-        using C = Conv<S, R>;
-        if (HY) {
-#pragma unroll
-            for (int j = 0; j < P::JY; ++j)
-                if (hs.ly[j] >= 0) y[j] = C::ld(base + px + hs.gy[j]);
-        }
-        if (HZ && hs.lz >= 0) z = C::ld(base + px + hs.gz);
-    }
-    __device__ __forceinline__ void put(R* lds, const HaloSlots<M, TY>& hs) const {
-        if (HY) {
-#pragma unroll
-            for (int j = 0; j < P::JY; ++j)
-                if (hs.ly[j] >= 0) lds[hs.ly[j]] = y[j];
-        }
-        if (HZ && hs.lz >= 0) lds[hs.lz] = z;
-    }
-};
-
-template <typename R, typename S, int M, int TY, bool HET>
-__global__ __launch_bounds__(64 * TY) void velocity_sweep(Geom g, FieldPtrs<S> F, MediaPtrs<R> md, Coefs<R> c,
-                                                          int t0, int t1, int tz, int ty, int xchunk, int nblocks) {
-    using P = Plane<M, TY>;
-    using C = Conv<S, R>;
-    __shared__ R sYY[2][P::H * P::W], sZZ[2][P::H * P::W], sXY[2][P::H * P::W], sYZ[2][P::H * P::W],
-        sXZ[2][P::H * P::W];
-    const int l = logical_block(nblocks);
-    if (l < 0) return;
-    const int bz = l % tz, by = (l / tz) % ty, bx = l / (tz * ty);
-    const int lz = threadIdx.x & 63, ly = threadIdx.x >> 6;
-    const int z0 = M + bz * 64, y0 = M + by * TY;
-    const int z = z0 + lz, y = y0 + ly;
-    const bool active = z < g.nz - M && y < g.ny - M;
-    const int64_t col = (int64_t)min(y, g.ny - 1) * g.sy + min(z, g.nz - 1);
-    const int xb = M + bx * xchunk, xe = min(xb + xchunk, g.nx - M);
-    const S* TXX = F.f[3][t1];
-    const S* TYY = F.f[4][t1];
-    const S* TZZ = F.f[5][t1];
-    const S* TXY = F.f[6][t1];
-    const S* TYZ = F.f[7][t1];
-    const S* TXZ = F.f[8][t1];
-    HaloSlots<M, TY> hs;
-    hs.init(g, y0, z0);
-    // qXX[i] = Txx(x+i-M+1) (a = 1), qXY[i] = Txy(x+i-M), qXZ[i] = Txz(x+i-M) (a = 0)
-    R qXX[2 * M], qXY[2 * M], qXZ[2 * M];
-#pragma unroll
-    for (int i = 1; i < 2 * M; ++i) {
-        qXX[i] = C::ldnt(TXX + (int64_t)(xb - M + i) * g.sx + col);
-        qXY[i] = C::ld(TXY + (int64_t)(xb - M - 1 + i) * g.sx + col);
-        qXZ[i] = C::ld(TXZ + (int64_t)(xb - M - 1 + i) * g.sx + col);
-    }
-    R nXX, nXY, nXZ, nYY, nZZ, nYZ, nU, nV, nW;
-    Staged<R, M, TY, true, false> hYY, hXY;
-    Staged<R, M, TY, false, true> hZZ, hXZ;
-    Staged<R, M, TY, true, true> hYZ;
-    auto fetch = [&](int x) {
-        const int64_t px = (int64_t)x * g.sx;
-        nXX = C::ldnt(TXX + px + (int64_t)M * g.sx + col);   // read along x only: streamed once
-        nXY = C::ld(TXY + px + (int64_t)(M - 1) * g.sx + col);
-        nXZ = C::ld(TXZ + px + (int64_t)(M - 1) * g.sx + col);
-        nYY = C::ld(TYY + px + col);
-        nZZ = C::ld(TZZ + px + col);
-        nYZ = C::ld(TYZ + px + col);
-        nU = C::ldnt(F.f[0][t0] + px + col);
-        nV = C::ldnt(F.f[1][t0] + px + col);
-        nW = C::ldnt(F.f[2][t0] + px + col);
-        hYY.fetch(TYY, px, hs);
-        hXY.fetch(TXY, px, hs);
-        hZZ.fetch(TZZ, px, hs);
-        hXZ.fetch(TXZ, px, hs);
-        hYZ.fetch(TYZ, px, hs);
-    };
-    fetch(xb);
-    for (int x = xb; x < xe; ++x) {
-        const int b = (x - xb) & 1;
-#pragma unroll
-        for (int i = 0; i < 2 * M - 1; ++i) {
-            qXX[i] = qXX[i + 1];
-            qXY[i] = qXY[i + 1];
-            qXZ[i] = qXZ[i + 1];
-        }
-        qXX[2 * M - 1] = nXX;
-        qXY[2 * M - 1] = nXY;
-        qXZ[2 * M - 1] = nXZ;
-        const R u0 = nU, v0 = nV, w0 = nW;
-        R* LYY = sYY[b];
-        R* LZZ = sZZ[b];
-        R* LXY = sXY[b];
-        R* LYZ = sYZ[b];
-        R* LXZ = sXZ[b];
-        const int me = (ly + M) * P::W + lz + M;
-        LYY[me] = nYY;
-        LZZ[me] = nZZ;
-        LYZ[me] = nYZ;
-        LXY[me] = qXY[M];
-        LXZ[me] = qXZ[M];
-        hYY.put(LYY, hs);
-        hXY.put(LXY, hs);
-        hZZ.put(LZZ, hs);
-        hXZ.put(LXZ, hs);
-        hYZ.put(LYZ, hs);
-        if (x + 1 < xe) fetch(x + 1);
-        __syncthreads();
-        if (active) {
-            const int64_t q = (int64_t)x * g.sx + col;
-            R su = 0, sv = 0, sw = 0;
-#pragma unroll
-            for (int k = 0; k < M; ++k) su = fmac(c.cv[0][0][k], qXX[M + k] - qXX[M - 1 - k], su);
-#pragma unroll
-            for (int k = 0; k < M; ++k) su = fmac(c.cv[0][1][k], LXY[me + k * P::W] - LXY[me - (1 + k) * P::W], su);
-#pragma unroll
-            for (int k = 0; k < M; ++k) su = fmac(c.cv[0][2][k], LXZ[me + k] - LXZ[me - 1 - k], su);
-#pragma unroll
-            for (int k = 0; k < M; ++k) sv = fmac(c.cv[1][0][k], qXY[M + k] - qXY[M - 1 - k], sv);
-#pragma unroll
-            for (int k = 0; k < M; ++k) sv = fmac(c.cv[1][1][k], LYY[me + (1 + k) * P::W] - LYY[me - k * P::W], sv);
-#pragma unroll
-            for (int k = 0; k < M; ++k) sv = fmac(c.cv[1][2][k], LYZ[me + k] - LYZ[me - 1 - k], sv);
-#pragma unroll
-            for (int k = 0; k < M; ++k) sw = fmac(c.cv[2][0][k], qXZ[M + k] - qXZ[M - 1 - k], sw);
-#pragma unroll
-            for (int k = 0; k < M; ++k) sw = fmac(c.cv[2][1][k], LYZ[me + k * P::W] - LYZ[me - (1 + k) * P::W], sw);
-#pragma unroll
-            for (int k = 0; k < M; ++k) sw = fmac(c.cv[2][2][k], LZZ[me + 1 + k] - LZZ[me - k], sw);
-            if (HET) {
-                C::stnt(F.f[0][t1] + q, fmac(__builtin_nontemporal_load(md.m[OPESCI_M_BETA1] + q), su, u0));
-                C::stnt(F.f[1][t1] + q, fmac(__builtin_nontemporal_load(md.m[OPESCI_M_BETA2] + q), sv, v0));
-                C::stnt(F.f[2][t1] + q, fmac(__builtin_nontemporal_load(md.m[OPESCI_M_BETA3] + q), sw, w0));
-            } else {
-                C::stnt(F.f[0][t1] + q, u0 + su);
-                C::stnt(F.f[1][t1] + q, v0 + sv);
-                C::stnt(F.f[2][t1] + q, w0 + sw);
-            }
-        }
-    }
-}
-
-// ------------------------------------------------------------------ pair sweeps (FP32 arithmetic)
-// The same sweeps with two z points per lane: a tile is 128 (z) x TY (y),
-// lane lz owns z0 + 2 lz and z0 + 2 lz + 1, and every own-column value and
-// y-halo row is moved as one pair (32 bits for FP16/BF16 storage, 64 bits
-// for FP32; tiles start at z = m, which the layout aligns to 128 bytes, so
-// pairs are aligned; the row padding holds the partner of the last point).
-// Twice the bytes per load instruction and half the blocks' z halos: at
-// 256^3 the FP32 read path runs 11 % faster than with one point per lane.
-// Per point the arithmetic is the single-point sweeps' and the gather
-// kernels'.
-template <int M, int TY>
-struct Plane2 {
-    static constexpr int W = 128 + 2 * M;
-    static constexpr int H = TY + 2 * M;
-    static constexpr int NT = 64 * TY;
-    static constexpr int NY = 2 * M * 64;   // y-halo pairs
-    static constexpr int NZ = TY * 2 * M;   // z-halo cells
-    static constexpr int JY = (NY + NT - 1) / NT;
-    static_assert(NZ <= NT, "z halo larger than the block");
-};
-
 // first z of the aligned pair holding z (z - m even), kept inside the row
 __device__ __forceinline__ int pair_start(const Geom& g, int z) {
     z = min(max(z, 0), g.nz - 1);
     return z - ((z - g.m) & 1);
 }
 
-template <int M, int TY>
-struct HaloSlots2 {
-    using P = Plane2<M, TY>;
-    int ly[P::JY], gy[P::JY];
-    int lz, gz;
-    __device__ void init(const Geom& g, int y0, int z0) {
-        const int t = threadIdx.x;
-#pragma unroll
-        for (int j = 0; j < P::JY; ++j) {
-            const int h = t + j * P::NT;
-            if (h < P::NY) {
-                const int r = h / 64, row = r < M ? r : r + TY, cl = M + 2 * (h % 64);
-                const int yy = min(max(y0 - M + row, 0), g.ny - 1), zz = pair_start(g, z0 - M + cl);
-                ly[j] = row * P::W + cl;
-                gy[j] = yy * (int)g.sy + zz;
-            } else {
-                ly[j] = -1;
-                gy[j] = 0;
-            }
-        }
-        if (t < P::NZ) {
-            const int row = M + t / (2 * M), c = t % (2 * M), cl = c < M ? c : 128 + c;
-            const int yy = min(max(y0 - M + row, 0), g.ny - 1), zz = min(max(z0 - M + cl, 0), g.nz - 1);
-            lz = row * P::W + cl;
-            gz = yy * (int)g.sy + zz;
-        } else {
-            lz = -1;
-            gz = 0;
-        }
-    }
-};
-
-template <int M, int TY, bool HY, bool HZ>
-struct Staged2 {
-    using P = Plane2<M, TY>;
-    float y0[HY ? P::JY : 1], y1[HY ? P::JY : 1];
-    float z;
-    template <typename S>
-    __device__ __forceinline__ void fetch(const S* base, int64_t px, const HaloSlots2<M, TY>& hs) {
-        if (HY) {
-#pragma unroll
-            for (int j = 0; j < P::JY; ++j)
-                if (hs.ly[j] >= 0) ld2(base + px + hs.gy[j], y0[j], y1[j]);
-        }
-        if (HZ && hs.lz >= 0) z = Conv<S, float>::ld(base + px + hs.gz);
-    }
-    __device__ __forceinline__ void put(float* lds, const HaloSlots2<M, TY>& hs) const {
-        if (HY) {
-#pragma unroll
-            for (int j = 0; j < P::JY; ++j)
-                if (hs.ly[j] >= 0) {
-                    lds[hs.ly[j]] = y0[j];
-                    lds[hs.ly[j] + 1] = y1[j];
-                }
-        }
-        if (HZ && hs.lz >= 0) lds[hs.lz] = z;
-    }
-};
-
-// FP32 media of a lane's two points as one 8-byte load (the media use the
-// fields' element layout, so z - m even is 8-byte aligned for them)
-typedef float mpair_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ mpair_t media2(const float* p) {
-    return __builtin_nontemporal_load(reinterpret_cast<const mpair_t*>(p));
-}
-
-// one or two of a lane's points, as one pair or a single value (non-temporal:
-// ordinary stores, which leave the fields in the memory-side cache for the
-// next launch, measured slower for both sweeps at 256^3)
+// one or two of a lane's points, as one pair or a single value
 template <typename S>
 __device__ __forceinline__ void store_points(S* p, float a, float b, bool act0, bool act1) {
     if (act1)
@@ -493,145 +192,6 @@ template <typename S>
 __device__ __forceinline__ float lane_read(float v, int lane) {
     const float r = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
     return Conv<S, float>::from(Conv<S, float>::to(r));
-}
-
-template <typename S, int M, int TY, bool HET>
-__global__ __launch_bounds__(64 * TY) void velocity_sweep2(Geom g, FieldPtrs<S> F, MediaPtrs<float> md,
-                                                           Coefs<float> c, int t0, int t1, int tz, int nblocks,
-                                                           Boxes B) {
-    using R = float;
-    using P = Plane2<M, TY>;
-    __shared__ R sYY[2][P::H * P::W], sZZ[2][P::H * P::W], sXY[2][P::H * P::W], sYZ[2][P::H * P::W],
-        sXZ[2][P::H * P::W];
-    const int l = logical_block(nblocks);
-    if (l < 0) return;
-    const TileOrigin o = tile_of<TY>(B, l, tz, M);
-    const int lz = threadIdx.x & 63, ly = threadIdx.x >> 6;
-    const int z0 = o.z0, y0 = o.y0;
-    const int z = z0 + 2 * lz, y = y0 + ly;
-    const bool act0 = z < g.nz - M && y < o.yend, act1 = z + 1 < g.nz - M && y < o.yend;
-    const int64_t col = (int64_t)min(y, g.ny - 1) * g.sy + pair_start(g, z);
-    const int xb = o.xb, xe = o.xe;
-    const S* TXX = F.f[3][t1];
-    const S* TYY = F.f[4][t1];
-    const S* TZZ = F.f[5][t1];
-    const S* TXY = F.f[6][t1];
-    const S* TYZ = F.f[7][t1];
-    const S* TXZ = F.f[8][t1];
-    HaloSlots2<M, TY> hs;
-    hs.init(g, y0, z0);
-    // per point v: qXX[v][i] = Txx(x+i-M+1), qXY[v][i] = Txy(x+i-M), qXZ[v][i] = Txz(x+i-M)
-    R qXX[2][2 * M], qXY[2][2 * M], qXZ[2][2 * M];
-#pragma unroll
-    for (int i = 1; i < 2 * M; ++i) {
-        ldnt2(TXX + (int64_t)(xb - M + i) * g.sx + col, qXX[0][i], qXX[1][i]);
-        ld2(TXY + (int64_t)(xb - M - 1 + i) * g.sx + col, qXY[0][i], qXY[1][i]);
-        ld2(TXZ + (int64_t)(xb - M - 1 + i) * g.sx + col, qXZ[0][i], qXZ[1][i]);
-    }
-    R nXX[2], nXY[2], nXZ[2], nYY[2], nZZ[2], nYZ[2], nU[2], nV[2], nW[2];
-    Staged2<M, TY, true, false> hYY, hXY;
-    Staged2<M, TY, false, true> hZZ, hXZ;
-    Staged2<M, TY, true, true> hYZ;
-    auto fetch = [&](int x) {
-        const int64_t px = (int64_t)x * g.sx;
-        ldnt2(TXX + px + (int64_t)M * g.sx + col, nXX[0], nXX[1]);
-        ld2(TXY + px + (int64_t)(M - 1) * g.sx + col, nXY[0], nXY[1]);
-        ld2(TXZ + px + (int64_t)(M - 1) * g.sx + col, nXZ[0], nXZ[1]);
-        ld2(TYY + px + col, nYY[0], nYY[1]);
-        ld2(TZZ + px + col, nZZ[0], nZZ[1]);
-        ld2(TYZ + px + col, nYZ[0], nYZ[1]);
-        ldnt2(F.f[0][t0] + px + col, nU[0], nU[1]);
-        ldnt2(F.f[1][t0] + px + col, nV[0], nV[1]);
-        ldnt2(F.f[2][t0] + px + col, nW[0], nW[1]);
-        hYY.fetch(TYY, px, hs);
-        hXY.fetch(TXY, px, hs);
-        hZZ.fetch(TZZ, px, hs);
-        hXZ.fetch(TXZ, px, hs);
-        hYZ.fetch(TYZ, px, hs);
-    };
-    fetch(xb);
-    for (int x = xb; x < xe; ++x) {
-        const int b = (x - xb) & 1;
-#pragma unroll
-        for (int v = 0; v < 2; ++v) {
-#pragma unroll
-            for (int i = 0; i < 2 * M - 1; ++i) {
-                qXX[v][i] = qXX[v][i + 1];
-                qXY[v][i] = qXY[v][i + 1];
-                qXZ[v][i] = qXZ[v][i + 1];
-            }
-            qXX[v][2 * M - 1] = nXX[v];
-            qXY[v][2 * M - 1] = nXY[v];
-            qXZ[v][2 * M - 1] = nXZ[v];
-        }
-        const R u0[2] = {nU[0], nU[1]}, v0[2] = {nV[0], nV[1]}, w0[2] = {nW[0], nW[1]};
-        R* LYY = sYY[b];
-        R* LZZ = sZZ[b];
-        R* LXY = sXY[b];
-        R* LYZ = sYZ[b];
-        R* LXZ = sXZ[b];
-        const int me0 = (ly + M) * P::W + 2 * lz + M;
-#pragma unroll
-        for (int v = 0; v < 2; ++v) {
-            LYY[me0 + v] = nYY[v];
-            LZZ[me0 + v] = nZZ[v];
-            LYZ[me0 + v] = nYZ[v];
-            LXY[me0 + v] = qXY[v][M];
-            LXZ[me0 + v] = qXZ[v][M];
-        }
-        hYY.put(LYY, hs);
-        hXY.put(LXY, hs);
-        hZZ.put(LZZ, hs);
-        hXZ.put(LXZ, hs);
-        hYZ.put(LYZ, hs);
-        if (x + 1 < xe) fetch(x + 1);
-        __syncthreads();
-        if (act0) {
-            const int64_t q = (int64_t)x * g.sx + col;
-            R ou[2], ov[2], ow[2];
-            mpair_t b1, b2, b3;
-            if (HET) {
-                b1 = media2(md.m[OPESCI_M_BETA1] + q);
-                b2 = media2(md.m[OPESCI_M_BETA2] + q);
-                b3 = media2(md.m[OPESCI_M_BETA3] + q);
-            }
-#pragma unroll
-            for (int v = 0; v < 2; ++v) {
-                const int me = me0 + v;
-                R su = 0, sv = 0, sw = 0;
-#pragma unroll
-                for (int k = 0; k < M; ++k) su = fmac(c.cv[0][0][k], qXX[v][M + k] - qXX[v][M - 1 - k], su);
-#pragma unroll
-                for (int k = 0; k < M; ++k) su = fmac(c.cv[0][1][k], LXY[me + k * P::W] - LXY[me - (1 + k) * P::W], su);
-#pragma unroll
-                for (int k = 0; k < M; ++k) su = fmac(c.cv[0][2][k], LXZ[me + k] - LXZ[me - 1 - k], su);
-#pragma unroll
-                for (int k = 0; k < M; ++k) sv = fmac(c.cv[1][0][k], qXY[v][M + k] - qXY[v][M - 1 - k], sv);
-#pragma unroll
-                for (int k = 0; k < M; ++k) sv = fmac(c.cv[1][1][k], LYY[me + (1 + k) * P::W] - LYY[me - k * P::W], sv);
-#pragma unroll
-                for (int k = 0; k < M; ++k) sv = fmac(c.cv[1][2][k], LYZ[me + k] - LYZ[me - 1 - k], sv);
-#pragma unroll
-                for (int k = 0; k < M; ++k) sw = fmac(c.cv[2][0][k], qXZ[v][M + k] - qXZ[v][M - 1 - k], sw);
-#pragma unroll
-                for (int k = 0; k < M; ++k) sw = fmac(c.cv[2][1][k], LYZ[me + k * P::W] - LYZ[me - (1 + k) * P::W], sw);
-#pragma unroll
-                for (int k = 0; k < M; ++k) sw = fmac(c.cv[2][2][k], LZZ[me + 1 + k] - LZZ[me - k], sw);
-                if (HET) {
-                    ou[v] = fmac(b1[v], su, u0[v]);
-                    ov[v] = fmac(b2[v], sv, v0[v]);
-                    ow[v] = fmac(b3[v], sw, w0[v]);
-                } else {
-                    ou[v] = u0[v] + su;
-                    ov[v] = v0[v] + sv;
-                    ow[v] = w0[v] + sw;
-                }
-            }
-            store_points(F.f[0][t1] + q, ou[0], ou[1], act0, act1);
-            store_points(F.f[1][t1] + q, ov[0], ov[1], act0, act1);
-            store_points(F.f[2][t1] + q, ow[0], ow[1], act0, act1);
-        }
-    }
 }
 
 // ------------------------------------------------------------------ fused step
@@ -1212,28 +772,22 @@ __global__ __launch_bounds__(64 * (TY + 2 * M)) void step_sweep2(Geom g, StepPtr
 
 // ------------------------------------------------------------------ dispatch
 struct Tiling {
-    int ty, tz, tyn, tx, xchunk, nb, grid;
+    int tz, tyn, xchunk, nb, grid;
 };
 
 template <int M>
-static Tiling tiling(const Geom& g, const InteriorLaunch& cfg, int ty, int tzw = 64) {
+static Tiling tiling(const Geom& g, int x_chunk) {
     Tiling t;
     const int ni[3] = {g.nx - 2 * M, g.ny - 2 * M, g.nz - 2 * M};
-    t.ty = ty;
-    t.tz = (ni[2] + tzw - 1) / tzw;
-    t.tyn = (ni[1] + ty - 1) / ty;
-    int xc = cfg.x_chunk;
+    t.tz = (ni[2] + 63) / 64;
+    t.tyn = (ni[1] + 3) / 4;
+    int xc = x_chunk;
     if (xc <= 0) {
-        // about 512 blocks of 512 threads (256 of 1024): two per CU.  Long x
-        // sweeps load fewer x halos and measured fastest at 256^3 (x chunks
-        // 8..128 timed); 8..64 planes
-        const int cols = t.tz * t.tyn, target = ty >= 16 ? 256 : 512;
-        xc = (ni[0] * cols + target - 1) / target;
+        xc = (ni[0] * t.tz * t.tyn + 511) / 512;   // about 512 blocks
         xc = xc < 8 ? 8 : (xc > 64 ? 64 : xc);
     }
     t.xchunk = xc;
-    t.tx = (ni[0] + xc - 1) / xc;
-    t.nb = t.tz * t.tyn * t.tx;
+    t.nb = t.tz * t.tyn * ((ni[0] + xc - 1) / xc);
     t.grid = ((t.nb + 7) / 8) * 8;
     return t;
 }
@@ -1266,112 +820,29 @@ static Boxes fill_boxes(const Geom& g, Boxes B, int ty, int xc0, int& tz) {
     return B;
 }
 
-// Rows per tile of the single-point sweeps when the caller leaves it open: 16
-// for FP32 on constant media (fewer y-halo rows; measured 2-3 % faster at
-// 256^3), else 8 (the media streams and the 16-bit conversions favour the
-// smaller tile).
-template <typename R, typename S, bool HET>
-static int default_tile_y() {
-    return (!HET && sizeof(R) == 4 && sizeof(S) == 4) ? 16 : 8;
-}
-
 template <typename R, typename S, int M, bool HET, bool VEL>
-static hipError_t run_interior(const Geom& g, void* fields, const void* media, const void* coefs, int t0, int t1,
-                               const InteriorLaunch& cfg, hipStream_t s, const Boxes* boxes) {
+static hipError_t run_gather(const Geom& g, void* fields, const void* media, const void* coefs, int t0, int t1,
+                             int x_chunk, hipStream_t s) {
     const FieldPtrs<S>& F = *static_cast<const FieldPtrs<S>*>(fields);
     const MediaPtrs<R>& md = *static_cast<const MediaPtrs<R>*>(media);
     const Coefs<R>& c = *static_cast<const Coefs<R>*>(coefs);
-    // box lists run on the pair sweeps only
-    if (boxes && (sizeof(R) != 4 || cfg.variant != 0)) return hipErrorInvalidValue;
-    if (cfg.variant == 1) {
-        const Tiling t = tiling<M>(g, cfg, 4);
-        if (VEL)
-            hipLaunchKernelGGL((velocity_gather<R, S, M, HET>), dim3(t.grid), dim3(256), 0, s, g, F, md, c, t0, t1,
-                               t.tz, t.tyn, t.xchunk, t.nb);
-        else
-            hipLaunchKernelGGL((stress_gather<R, S, M, HET>), dim3(t.grid), dim3(256), 0, s, g, F, md, c, t0, t1,
-                               t.tz, t.tyn, t.xchunk, t.nb);
-        return hipGetLastError();
-    }
-    if constexpr (!VEL) {
-        return hipErrorInvalidValue;   // the stress sweeps are launch_stress_sweep's
-    } else {
-    if constexpr (sizeof(R) == 4) {
-        if (cfg.variant == 0) {
-            // FP32 arithmetic: the pair sweeps (two z points per lane, 128-wide
-            // z tiles).  Stress tiles have 4 or 8 rows (default 8), as
-            // 1024-thread blocks would spill the doubled register queues; the
-            // velocity kernel, with fewer of them, takes 16 rows at orders 2
-            // and 4 (the default for FP32 storage: fewer y-halo rows, 2-5 %
-            // faster at 256^3)
-            int ty = cfg.tile_y == 4 ? 4 : 8;
-            if constexpr (VEL && M <= 2)
-                if (cfg.tile_y == 16 || (cfg.tile_y == 0 && sizeof(S) == 4)) ty = 16;
-            Boxes B;
-            int tz = 0;
-            if (boxes) {
-                B = fill_boxes<M>(g, *boxes, ty, cfg.x_chunk, tz);
-            } else {
-                const Tiling t = tiling<M>(g, cfg, ty, 128);
-                B.n = 1;
-                B.x0[0] = M;
-                B.x1[0] = g.nx - M;
-                B.y0[0] = M;
-                B.y1[0] = g.ny - M;
-                B.tyn[0] = t.tyn;
-                B.xc[0] = t.xchunk;
-                B.first[1] = t.nb;
-                tz = t.tz;
-            }
-            const int nb = B.first[B.n];
-            if (nb == 0) return hipSuccess;
-            const int grid = ((nb + 7) / 8) * 8;
-#define OPESCI_PAIR(TYV)                                                                                        \
-    if (ty == TYV) {                                                                                            \
-        hipLaunchKernelGGL((velocity_sweep2<S, M, TYV, HET>), dim3(grid), dim3(64 * TYV), 0, s, g, F, md, c,       \
-                           t0, t1, tz, nb, B);                                                                  \
-        return hipGetLastError();                                                                               \
-    }
-            OPESCI_PAIR(4)
-            OPESCI_PAIR(8)
-#undef OPESCI_PAIR
-            if constexpr (VEL && M <= 2) {
-                if (ty == 16) {
-                    hipLaunchKernelGGL((velocity_sweep2<S, M, 16, HET>), dim3(grid), dim3(1024), 0, s, g, F, md, c,
-                                       t0, t1, tz, nb, B);
-                    return hipGetLastError();
-                }
-            }
-        }
-    }
-    // one point per lane: kernel_variant 2, and every FP64 sweep
-    const int tile_y = cfg.tile_y ? cfg.tile_y : default_tile_y<R, S, HET>();
-    if (tile_y == 16) {
-        const Tiling t = tiling<M>(g, cfg, 16);
-        hipLaunchKernelGGL((velocity_sweep<R, S, M, 16, HET>), dim3(t.grid), dim3(1024), 0, s, g, F, md, c, t0, t1,
-                           t.tz, t.tyn, t.xchunk, t.nb);
-        return hipGetLastError();
-    }
-    if (tile_y == 4) {
-        const Tiling t = tiling<M>(g, cfg, 4);
-        hipLaunchKernelGGL((velocity_sweep<R, S, M, 4, HET>), dim3(t.grid), dim3(256), 0, s, g, F, md, c, t0, t1,
-                           t.tz, t.tyn, t.xchunk, t.nb);
-        return hipGetLastError();
-    }
-    const Tiling t = tiling<M>(g, cfg, 8);
-    hipLaunchKernelGGL((velocity_sweep<R, S, M, 8, HET>), dim3(t.grid), dim3(512), 0, s, g, F, md, c, t0, t1,
-                       t.tz, t.tyn, t.xchunk, t.nb);
+    const Tiling t = tiling<M>(g, x_chunk);
+    if (VEL)
+        hipLaunchKernelGGL((velocity_gather<R, S, M, HET>), dim3(t.grid), dim3(256), 0, s, g, F, md, c, t0, t1, t.tz,
+                           t.tyn, t.xchunk, t.nb);
+    else
+        hipLaunchKernelGGL((stress_gather<R, S, M, HET>), dim3(t.grid), dim3(256), 0, s, g, F, md, c, t0, t1, t.tz,
+                           t.tyn, t.xchunk, t.nb);
     return hipGetLastError();
-    }
 }
 
 template <typename R, typename S, bool VEL>
-static hipError_t dispatch_m(const Geom& g, bool het, void* fields, const void* media, const void* coefs, int t0,
-                             int t1, const InteriorLaunch& cfg, hipStream_t s, const Boxes* boxes) {
-#define OPESCI_CASE(MM)                                                                                          \
-    case MM:                                                                                                     \
-        return het ? run_interior<R, S, MM, true, VEL>(g, fields, media, coefs, t0, t1, cfg, s, boxes)           \
-                   : run_interior<R, S, MM, false, VEL>(g, fields, media, coefs, t0, t1, cfg, s, boxes);
+static hipError_t gather_m(const Geom& g, bool het, void* fields, const void* media, const void* coefs, int t0, int t1,
+                           int x_chunk, hipStream_t s) {
+#define OPESCI_CASE(MM)                                                                               \
+    case MM:                                                                                          \
+        return het ? run_gather<R, S, MM, true, VEL>(g, fields, media, coefs, t0, t1, x_chunk, s)     \
+                   : run_gather<R, S, MM, false, VEL>(g, fields, media, coefs, t0, t1, x_chunk, s);
     switch (g.m) {
         OPESCI_CASE(1)
         OPESCI_CASE(2)
@@ -1384,16 +855,14 @@ static hipError_t dispatch_m(const Geom& g, bool het, void* fields, const void* 
 }
 
 template <bool VEL>
-static hipError_t dispatch(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
-                           const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
-                           const Boxes* boxes) {
-    if (real_bytes == 8)
-        return dispatch_m<double, double, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
+static hipError_t launch_gather(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
+                                const void* coefs, int t0, int t1, int x_chunk, hipStream_t s) {
+    if (real_bytes == 8) return gather_m<double, double, VEL>(g, het, fields, media, coefs, t0, t1, x_chunk, s);
     if (storage == OPESCI_STORE_F16)
-        return dispatch_m<float, _Float16, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
+        return gather_m<float, _Float16, VEL>(g, het, fields, media, coefs, t0, t1, x_chunk, s);
     if (storage == OPESCI_STORE_BF16)
-        return dispatch_m<float, bf16_t, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
-    return dispatch_m<float, float, VEL>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
+        return gather_m<float, bf16_t, VEL>(g, het, fields, media, coefs, t0, t1, x_chunk, s);
+    return gather_m<float, float, VEL>(g, het, fields, media, coefs, t0, t1, x_chunk, s);
 }
 
 // ------------------------------------------------------------------ fused step launch
@@ -1459,10 +928,8 @@ hipError_t launch_step_fused(const Geom& g, int storage, void* fields, const voi
 }
 
 bool stress_applies_zfaces(int real_bytes, bool het, const InteriorLaunch& cfg) {
-    // the pair sweeps (FP32 arithmetic, variant 0) with their 4- or 8-row
-    // stress tiles, constant media (on the read path the surface recompute
-    // takes per-point coefficients, whose prefetch costs the sweep more
-    // occupancy than the separate launch costs time)
+    // FP32 arithmetic on constant media (on the read path the surface
+    // recompute takes per-point coefficients)
     return real_bytes == 4 && !het && cfg.variant == 0;
 }
 
@@ -1472,19 +939,20 @@ hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, v
     (void)pool;
     const bool sweep = cfg.variant != 1 && stress_sweep_applies(real_bytes, het, coefs, g.m);
     if (zf && zf->F > 0 && !(sweep && stress_applies_zfaces(real_bytes, het, cfg))) return hipErrorInvalidValue;
-    if (boxes && !(sweep && real_bytes == 4 && cfg.variant == 0)) return hipErrorInvalidValue;
     if (sweep)
         return launch_stress_sweep(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, zf, boxes);
+    if (boxes) return hipErrorInvalidValue;
     // sums not shared by the normal stresses: the gather kernel takes any coefficients
-    InteriorLaunch gather = cfg;
-    gather.variant = 1;
-    return dispatch<false>(g, real_bytes, storage, het, fields, media, coefs, t0, t1, gather, s, nullptr);
+    return launch_gather<false>(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg.x_chunk, s);
 }
 
 hipError_t launch_velocity(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                            const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
                            const Boxes* boxes) {
-    return dispatch<true>(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, boxes);
+    if (cfg.variant != 1)
+        return launch_velocity_sweep(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, boxes);
+    if (boxes) return hipErrorInvalidValue;
+    return launch_gather<true>(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg.x_chunk, s);
 }
 
 }  // namespace opesci

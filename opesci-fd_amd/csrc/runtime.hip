@@ -98,7 +98,7 @@ struct OpesciContext {
     bool initialised = false;
     size_t field_bytes = 0;
     InteriorLaunch cfg{0, 0, 0};
-    ZFaceArgs zf;                   // deep z-face statements the pair stress sweep applies (F = 0: none)
+    ZFaceArgs zf;                   // deep z-face statements the stress sweep applies (F = 0: none)
     std::vector<OpesciBcTerm> h_terms;  // boundary terms as given (host)
     int fused_F = 0;                // fused step: box [F, dim - F) in x and y (0: off)
     Boxes fbox, frame;              // its box and the four boxes of rows around it
@@ -442,7 +442,7 @@ int alloc_zero(OpesciContext* c, void** p, size_t bytes) {
 }
 
 // The deep z-face statements (phase 4, one launch level) when they have the
-// fixed forms the pair stress sweep applies in place: zero and images of
+// fixed forms the stress sweep applies in place: zero and images of
 // Tzz, images of Tyz/Txz, and the Levander recompute of Txx/Tyy with its
 // terms in the canonical order.  Anything else leaves zf.F = 0 and the
 // statements run as their own launch.
@@ -620,7 +620,7 @@ int build_fused(OpesciContext* c) {
     return 0;
 }
 
-// whether steps run the fused kernel (FP32 pair sweeps with the z faces in place)
+// whether steps run the fused kernel (FP32 sweeps with the z faces in place)
 bool fused_step(const OpesciContext* c) {
     return c->fused_F > 0 && c->cfg.variant == 0 && zfaces_in_sweep(c);
 }

@@ -10,14 +10,14 @@
 // addresses from shared 32-bit offsets, rotates the queues by name and sums
 // the off-axis normal terms once: 184 instructions per plane and wave of 64
 // points at 4th order, against 271 per 64 points for the sweep of two points
-// per lane that it replaces.  Two points per lane in this form (131 instead
-// of 84 KiB of registers a block, two blocks per CU) measured 248 us against
-// 239 on the 256^3 read path and 147 against 128 us for FP16; loads two
-// planes ahead instead of one, and blocks of 256 or 1024 threads, gained
-// nothing.  Measured before -> after (events, us): 256^3 4th order FP32 with
-// the z faces 223 -> 204, read path 253 -> 239, FP16 278 -> 128; 512-byte
-// FP64 rows, 128^3 4th order read path 82 -> 57; 160^3 FP32 107 -> 61; 161 x
-// 129 x 193 8th order BF16 read path 103 -> 79; 16^3 26 -> 7.
+// per lane that it replaces.  Two points per lane in this form (two blocks
+// per CU) measured 248 us against 239 on the 256^3 read path and 147 against
+// 128 us for FP16; loads two planes ahead instead of one, and blocks of 256
+// or 1024 threads, gained nothing; z tiles that do not start on a line cost
+// 81 us against 58 at 160^3.  Measured before -> after (events, us): 256^3
+// 4th order FP32 with the z faces 223 -> 204, read path 253 -> 239, FP16 278
+// -> 128; 128^3 4th order FP64 read path 82 -> 57; 160^3 FP32 107 -> 61; 161
+// x 129 x 193 8th order BF16 read path 103 -> 79; 16^3 26 -> 7.
 #include "sweep.h"
 
 namespace opesci {
@@ -75,7 +75,8 @@ __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void str
         for (int k = 0; k < 3; ++k) bm[2 + k] = P.ms[k] + x0;
     }
     const uint32_t plane = (uint32_t)g.sx * sizeof(S);
-    uint32_t own = s.own * sizeof(S), oy = s.gy * sizeof(S), oz = s.gz * sizeof(S), ox = s.gx * sizeof(S), om = s.own * sizeof(R);
+    uint32_t own = s.own * sizeof(S), oy = s.gy * sizeof(S), oz = s.gz * sizeof(S), ox = s.gx * sizeof(S),
+             om = s.own * sizeof(R);
     // register queues, logical element i at slot (phase + i) % Q:
     // U(x + i - M), V(x + i - M + 1), W(x + i - M + 1)
     R qU[Q], qV[Q], qW[Q];

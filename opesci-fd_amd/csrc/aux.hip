@@ -82,8 +82,17 @@ __device__ __forceinline__ const double* stage_tables(const SolProg& sol, int f,
 // Field f's analytic values at z on K rows (x[k], y[k]) of a block: the K
 // points of a shallow program in one pass over its ops, the others one
 // point at a time.
+// Bound by the doubles of the programs' sin, cos, sqrt and divide and by their
+// decoding.  A program whose factors mix media with two axes reaches depth 4
+// or 5 after its tables are split off, and the one-point evaluator's indexed
+// stack then goes through scratch, so the several-points form takes depth 5
+// (initial state with 3-D media, FP32: 512^3 45.1 -> 12.4 ms, 256^3 5.6 ->
+// 1.54 ms; L2 norms at 101^3 217 -> 110 us).
+// GENERAL: some field's program needs the one-point evaluator or holds POWC,
+// EXP or LOG; the plain form leaves both out of the kernel and so keeps four
+// waves per SIMD instead of two.
 constexpr int SOL_ROWS = 4;
-template <typename R>
+template <typename R, bool GENERAL>
 __device__ __forceinline__ void sol_points(const SolProg& sol, const OpesciExprOp* __restrict__ code, int f,
                                            const SolTable& tab, const MediaPtrs<R>& md, const Geom& g,
                                            const int x[SOL_ROWS], const int y[SOL_ROWS], int z,
@@ -96,8 +105,8 @@ __device__ __forceinline__ void sol_points(const SolProg& sol, const OpesciExprO
         cy[k] = coord_of<R>(tab.dx[1], y[k], m, stag(f, 1));
     }
     const double cz = coord_of<R>(tab.dx[2], z, m, stag(f, 2));
-    if (sol.shallow[f]) {
-        vm_eval_k<R, SOL_ROWS>(code + sol.off[f], sol.len[f], cx, cy, cz, tab.t[f], md, g, x, y, z, tabs, v);
+    if (!GENERAL || sol.shallow[f]) {
+        vm_eval_k<R, SOL_ROWS, GENERAL>(code + sol.off[f], sol.len[f], cx, cy, cz, tab.t[f], md, g, x, y, z, tabs, v);
     } else {
         for (int k = 0; k < SOL_ROWS; ++k) {
             const double c[3] = {cx[k], cy[k], cz};
@@ -121,7 +130,7 @@ __device__ __forceinline__ void sol_rows(int r0, int rows, int ny, int m, int x[
 
 // StaggeredGrid.initialise (opesci/staggeredgrid.py:612-659): level 0,
 // ranges [m, dim-m) or [m, dim-m-1) when staggered, t = dt/2 for velocities.
-template <typename R, typename S>
+template <typename R, typename S, bool GENERAL>
 __global__ __launch_bounds__(256) void initial_kernel(Geom g, FieldPtrs<S> F, MediaPtrs<R> md, SolProg sol,
                                                       const OpesciExprOp* __restrict__ code, SolTable tab,
                                                       int lds_cap) {
@@ -138,7 +147,7 @@ __global__ __launch_bounds__(256) void initial_kernel(Geom g, FieldPtrs<S> F, Me
         sol_rows(r0, rows, ny, m, x, y, ok);
         for (int z = m + (int)threadIdx.x; z < m + nz; z += blockDim.x) {
             double v[SOL_ROWS];
-            sol_points<R>(sol, code, f, tab, md, g, x, y, z, tabs, v);
+            sol_points<R, GENERAL>(sol, code, f, tab, md, g, x, y, z, tabs, v);
 #pragma unroll
             for (int k = 0; k < SOL_ROWS; ++k)
                 if (ok[k]) C::st(F.f[f][0] + g.at(x[k], y[k], z), (R)v[k]);
@@ -154,7 +163,7 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-template <typename R, typename S>
+template <typename R, typename S, bool GENERAL>
 __global__ __launch_bounds__(256) void l2_kernel(Geom g, FieldPtrs<S> F, MediaPtrs<R> md, SolProg sol,
                                                  const OpesciExprOp* __restrict__ code, SolTable tab, int level,
                                                  double* __restrict__ partial, int lds_cap) {
@@ -172,7 +181,7 @@ __global__ __launch_bounds__(256) void l2_kernel(Geom g, FieldPtrs<S> F, MediaPt
         sol_rows(r0, rows, ny, m, x, y, ok);
         for (int z = m + (int)threadIdx.x; z < m + nz; z += blockDim.x) {
             double v[SOL_ROWS];
-            sol_points<R>(sol, code, f, tab, md, g, x, y, z, tabs, v);
+            sol_points<R, GENERAL>(sol, code, f, tab, md, g, x, y, z, tabs, v);
 #pragma unroll
             for (int k = 0; k < SOL_ROWS; ++k)
                 if (ok[k]) {
@@ -380,7 +389,8 @@ static hipError_t init_t(const Geom& g, void* fields, const void* media, const S
                          hipStream_t s) {
     if (hipError_t e = sol_tables_t<R>(g, media, sol, tab, s)) return e;
     const int cap = sol_lds(sol);
-    hipLaunchKernelGGL((initial_kernel<R, S>), dim3(512, NF), dim3(256), cap * sizeof(double), s, g,
+    auto kernel = sol.general ? initial_kernel<R, S, true> : initial_kernel<R, S, false>;
+    hipLaunchKernelGGL(kernel, dim3(512, NF), dim3(256), cap * sizeof(double), s, g,
                        *static_cast<const FieldPtrs<S>*>(fields), *static_cast<const MediaPtrs<R>*>(media), sol,
                        sol.code, tab, cap);
     return hipGetLastError();
@@ -401,7 +411,8 @@ static hipError_t l2_t(const Geom& g, void* fields, const void* media, const Sol
                        int level, double* partial, int nblk, hipStream_t s) {
     if (hipError_t e = sol_tables_t<R>(g, media, sol, tab, s)) return e;
     const int cap = sol_lds(sol);
-    hipLaunchKernelGGL((l2_kernel<R, S>), dim3(nblk, NF), dim3(256), cap * sizeof(double), s, g,
+    auto kernel = sol.general ? l2_kernel<R, S, true> : l2_kernel<R, S, false>;
+    hipLaunchKernelGGL(kernel, dim3(nblk, NF), dim3(256), cap * sizeof(double), s, g,
                        *static_cast<const FieldPtrs<S>*>(fields), *static_cast<const MediaPtrs<R>*>(media), sol,
                        sol.code, tab, level, partial, cap);
     return hipGetLastError();

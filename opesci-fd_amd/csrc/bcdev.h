@@ -101,64 +101,86 @@ __device__ double vm_eval_tos(const OpesciExprOp* code, int n, const double coor
 }
 
 // K points of one program at once (the same ops, decoded once for all K),
-// for programs whose stack never exceeds depth 3: t0/t1/t2 are the top
-// three entries of each point's stack.  Per point, the same double
-// operations in the same order as vm_eval.
-template <typename R, int K>
+// for programs whose stack never exceeds depth SOL_DEPTH: t[0] is the top of
+// each point's stack, kept in registers.  Per point, the same double
+// operations in the same order as vm_eval.  ELEM: the program may hold
+// POWC, EXP or LOG, whose inlined code takes twice the registers.
+template <typename R, int K, bool ELEM>
 __device__ __forceinline__ void vm_eval_k(const OpesciExprOp* __restrict__ code, int n, const double cx[K],
                                           const double cy[K], double cz, double t, const MediaPtrs<R>& md,
                                           const Geom& g, const int ax[K], const int ay[K], int az,
                                           const double* __restrict__ tabs, double out[K]) {
-    double t0[K], t1[K], t2[K];
+    double s[SOL_DEPTH][K];
 #pragma unroll
-    for (int k = 0; k < K; ++k) t0[k] = t1[k] = t2[k] = 0.0;
+    for (int d = 0; d < SOL_DEPTH; ++d)
+#pragma unroll
+        for (int k = 0; k < K; ++k) s[d][k] = 0.0;
     for (int i = 0; i < n; ++i) {
         const OpesciExprOp o = code[i];
         const int op = o.op;
         if (op <= OPESCI_OP_MEDIA || op == OPX_TABLE) {
+            double v[K];
+            if (op == OPX_TABLE) {
+#pragma unroll
+                for (int k = 0; k < K; ++k) v[k] = tabs[o.a[0] + (o.a[1] == 0 ? ax[k] : (o.a[1] == 1 ? ay[k] : az))];
+            } else if (op == OPESCI_OP_CONST || op == OPESCI_OP_TIME) {
+#pragma unroll
+                for (int k = 0; k < K; ++k) v[k] = op == OPESCI_OP_CONST ? o.val : t;
+            } else if (op == OPESCI_OP_COORD) {
+#pragma unroll
+                for (int k = 0; k < K; ++k) v[k] = o.a[0] == 0 ? cx[k] : (o.a[0] == 1 ? cy[k] : cz);
+            } else {
+                const R* p = md.m[o.a[0]];
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    v[k] = p ? (double)p[g.at(ax[k] + o.a[1], ay[k] + o.a[2], az + o.a[3])] : 0.0;
+            }
 #pragma unroll
             for (int k = 0; k < K; ++k) {
-                double v;
-                if (op == OPX_TABLE)
-                    v = tabs[o.a[0] + (o.a[1] == 0 ? ax[k] : (o.a[1] == 1 ? ay[k] : az))];
-                else if (op == OPESCI_OP_CONST)
-                    v = o.val;
-                else if (op == OPESCI_OP_COORD)
-                    v = o.a[0] == 0 ? cx[k] : (o.a[0] == 1 ? cy[k] : cz);
-                else if (op == OPESCI_OP_TIME)
-                    v = t;
-                else {
-                    const R* p = md.m[o.a[0]];
-                    v = p ? (double)p[g.at(ax[k] + o.a[1], ay[k] + o.a[2], az + o.a[3])] : 0.0;
-                }
-                t2[k] = t1[k];
-                t1[k] = t0[k];
-                t0[k] = v;
+#pragma unroll
+                for (int d = SOL_DEPTH - 1; d > 0; --d) s[d][k] = s[d - 1][k];
+                s[0][k] = v[k];
+            }
+        } else if (op <= OPESCI_OP_DIV) {
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const double a = s[1][k], b = s[0][k];
+                if (op == OPESCI_OP_MUL)
+                    s[0][k] = a * b;
+                else if (op == OPESCI_OP_ADD)
+                    s[0][k] = a + b;
+                else if (op == OPESCI_OP_SUB)
+                    s[0][k] = a - b;
+                else
+                    s[0][k] = a / b;
+#pragma unroll
+                for (int d = 1; d < SOL_DEPTH - 1; ++d) s[d][k] = s[d + 1][k];
             }
         } else {
             switch (op) {
-#define OPESCI_K_LOOP(expr) _Pragma("unroll") for (int k = 0; k < K; ++k) t0[k] = (expr); break
-#define OPESCI_K_POP(expr) _Pragma("unroll") for (int k = 0; k < K; ++k) { t0[k] = (expr); t1[k] = t2[k]; } break
-                case OPESCI_OP_ADD: OPESCI_K_POP(t1[k] + t0[k]);
-                case OPESCI_OP_SUB: OPESCI_K_POP(t1[k] - t0[k]);
-                case OPESCI_OP_MUL: OPESCI_K_POP(t1[k] * t0[k]);
-                case OPESCI_OP_DIV: OPESCI_K_POP(t1[k] / t0[k]);
-                case OPESCI_OP_NEG: OPESCI_K_LOOP(-t0[k]);
-                case OPESCI_OP_POWC: OPESCI_K_LOOP(pow(t0[k], o.val));
-                case OPESCI_OP_SQRT: OPESCI_K_LOOP(sqrt(t0[k]));
-                case OPESCI_OP_SIN: OPESCI_K_LOOP(sin(t0[k]));
-                case OPESCI_OP_COS: OPESCI_K_LOOP(cos(t0[k]));
-                case OPESCI_OP_EXP: OPESCI_K_LOOP(exp(t0[k]));
-                case OPESCI_OP_LOG: OPESCI_K_LOOP(log(t0[k]));
-                case OPESCI_OP_ROUNDF: OPESCI_K_LOOP((double)(float)t0[k]);
+#define OPESCI_K_LOOP(expr) _Pragma("unroll") for (int k = 0; k < K; ++k) s[0][k] = (expr); break
+                case OPESCI_OP_NEG: OPESCI_K_LOOP(-s[0][k]);
+                case OPESCI_OP_SQRT: OPESCI_K_LOOP(sqrt(s[0][k]));
+                case OPESCI_OP_SIN: OPESCI_K_LOOP(sin(s[0][k]));
+                case OPESCI_OP_COS: OPESCI_K_LOOP(cos(s[0][k]));
+                case OPESCI_OP_ROUNDF: OPESCI_K_LOOP((double)(float)s[0][k]);
+                default:
+                    if (ELEM) {
+                        if (op == OPESCI_OP_POWC) {
+                            _Pragma("unroll") for (int k = 0; k < K; ++k) s[0][k] = pow(s[0][k], o.val);
+                        } else if (op == OPESCI_OP_EXP) {
+                            _Pragma("unroll") for (int k = 0; k < K; ++k) s[0][k] = exp(s[0][k]);
+                        } else if (op == OPESCI_OP_LOG) {
+                            _Pragma("unroll") for (int k = 0; k < K; ++k) s[0][k] = log(s[0][k]);
+                        }
+                    }
+                    break;
 #undef OPESCI_K_LOOP
-#undef OPESCI_K_POP
-                default: break;
             }
         }
     }
 #pragma unroll
-    for (int k = 0; k < K; ++k) out[k] = t0[k];
+    for (int k = 0; k < K; ++k) out[k] = s[0][k];
 }
 
 // One boundary statement at point p of its loop: dst = sum_k coef_k * src_k,

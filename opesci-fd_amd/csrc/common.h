@@ -394,6 +394,7 @@ hipError_t launch_src_cells(const Geom& g, int real_bytes, void* fields, int t, 
 // reads it back through OPX_TABLE.  The same double operations run in the
 // same order, so the values equal per-point evaluation bit for bit.
 constexpr int OPX_TABLE = 64;
+constexpr int SOL_DEPTH = 5;   // stack depth of the several-points evaluator
 struct SolSlot {
     int32_t field, axis, prog, len, tab;
 };
@@ -401,7 +402,8 @@ struct SolProg {
     const OpesciExprOp* code = nullptr;  // per-point programs, then the slots' programs
     int off[NF] = {}, len[NF] = {};
     int tab_base[NF] = {}, tab_len[NF] = {};  // field f's tables: tab[tab_base[f] ..], OPX_TABLE offsets relative to it
-    int shallow[NF] = {};                      // field f's point program never exceeds stack depth 3
+    int shallow[NF] = {};                      // field f's point program fits the several-points evaluator
+    int general = 0;                           // some field's does not, or holds POWC, EXP or LOG
     const SolSlot* slots = nullptr;
     int nslots = 0;
     int maxdim = 0;

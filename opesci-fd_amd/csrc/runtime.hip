@@ -419,8 +419,10 @@ int build_solution(OpesciContext* c, const OpesciModelDesc* d) {
             const int op = pc[i].op;
             depth += (op <= OPESCI_OP_MEDIA || op == OPX_TABLE) ? 1 : (op <= OPESCI_OP_DIV ? -1 : 0);
             maxd = std::max(maxd, depth);
+            if (op == OPESCI_OP_POWC || op == OPESCI_OP_EXP || op == OPESCI_OP_LOG) c->sol.general = 1;
         }
-        c->sol.shallow[f] = maxd <= 3;
+        c->sol.shallow[f] = maxd <= SOL_DEPTH;
+        if (!c->sol.shallow[f]) c->sol.general = 1;
     }
     for (SolSlot& s : slots) s.prog += (int32_t)pc.size();
     pc.insert(pc.end(), tc.begin(), tc.end());

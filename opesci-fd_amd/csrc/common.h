@@ -1,11 +1,15 @@
 // Internal definitions shared by the libopesci_hip translation units.
 //
 // Device layout of one field time level: F[x][y][zoff + z], x slowest,
-// z contiguous, rows padded to `pitch` elements so that the first interior
-// z (= m) of every row starts on a 128-byte boundary for 4-byte storage.
+// z contiguous, rows `pitch` elements apart, a whole number of 128-byte lines,
+// so that the first interior z (= m) of every row starts a line.
 // Pointers handed to kernels are pre-offset by zoff, so element (x,y,z) is
-// p[(x*ny + y)*pitch + z] for z in [0, nz); the padding in front of z = 0
-// keeps every stencil read (|offset| <= m) inside the allocation.
+// p[(x*ny + y)*pitch + z] for z in [0, nz).  pitch is nz rounded up: the low
+// ghosts end the line that the previous row's high ghosts begin.  The z faces
+// are bound by lines touched, and the sweeps read both ends of a row, so the
+// shared line is worth a line of ten at 256 floats.  The padding before the
+// first row and the line after the last keep every read within m of a row
+// inside the allocation.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -168,6 +172,7 @@ struct Geom {
     int pitch;        // row pitch in elements
     int zoff;         // elements in front of z = 0
     int64_t sy, sx;   // strides (sy = pitch, sx = ny*pitch)
+    int64_t total;    // elements of an allocation (all rows and one line)
     __host__ __device__ int64_t at(int x, int y, int z) const { return (int64_t)x * sx + (int64_t)y * sy + z; }
 };
 

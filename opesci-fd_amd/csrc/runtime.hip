@@ -734,10 +734,14 @@ int create(const OpesciModelDesc* d, OpesciContext** out) {
     g.m = d->space_order / 2;
     const int align = 128 / c->elem;  // first interior z on a 128-byte boundary
     g.zoff = (align - g.m % align) % align;
-    g.pitch = ((g.zoff + g.nz + g.m + align - 1) / align) * align;
+    // A row's high ghosts and the next row's low ghosts share a line: rows of
+    // 256 + 2m floats take 9 lines instead of 10.  One line past the last row
+    // holds its high ghosts and the reads of up to m past them.
+    g.pitch = ((g.nz + align - 1) / align) * align;
     g.sy = g.pitch;
     g.sx = (int64_t)g.ny * g.pitch;
-    c->field_bytes = (size_t)g.nx * g.sx * c->elem;
+    g.total = (int64_t)g.nx * g.sx + align;
+    c->field_bytes = (size_t)g.total * c->elem;
     for (int f = 0; f < NF; ++f)
         for (int l = 0; l < 2; ++l) {
             if (int e = alloc_zero(c.get(), &c->base[f][l], c->field_bytes)) return e;
@@ -747,7 +751,7 @@ int create(const OpesciModelDesc* d, OpesciContext** out) {
     const size_t dense = (size_t)g.nx * g.ny * g.nz;
     OPESCI_HIP_TRY(hipMalloc(&c->d_stage, dense * std::max(rb, sizeof(float) * 3)));
     if (c->het) {
-        const size_t mbytes = (size_t)g.nx * g.sx * rb;
+        const size_t mbytes = (size_t)g.total * rb;
         for (int i = 0; i < OPESCI_M_COUNT; ++i) {
             if (int e = alloc_zero(c.get(), &c->mbase[i], mbytes)) return e;
             c->mptr[i] = (char*)c->mbase[i] + (size_t)g.zoff * rb;
@@ -1438,7 +1442,7 @@ static int adj_alloc(OpesciContext* c, int ckpt, size_t seg_bytes, int log_steps
                 if (int e = alloc_zero(c, &c->abase[f][l], c->field_bytes)) return e;
                 c->aptr[f][l] = (char*)c->abase[f][l] + (size_t)g.zoff * rb;
             }
-        const size_t mbytes = (size_t)g.nx * g.sx * rb;
+        const size_t mbytes = (size_t)g.total * rb;
         for (int i = 0; i < OPESCI_M_COUNT; ++i) {
             if (int e = alloc_zero(c, &c->gbase[i], mbytes)) return e;
             c->gptr[i] = (char*)c->gbase[i] + (size_t)g.zoff * rb;
@@ -1708,7 +1712,7 @@ int opesci_ctx_gradient_reverse(OpesciContext* c) {
         // reverse sweep, segment by segment
         for (int f = 0; f < NF; ++f)
             for (int l = 0; l < 2; ++l) OPESCI_HIP_TRY(launch_zero(c->abase[f][l], c->field_bytes, c->stream));
-        const size_t mbytes = (size_t)c->g.nx * c->g.sx * c->real_bytes;
+        const size_t mbytes = (size_t)c->g.total * c->real_bytes;
         for (int i = 0; i < OPESCI_M_COUNT; ++i) OPESCI_HIP_TRY(launch_zero(c->gbase[i], mbytes, c->stream));
         if (c->d_gpool)
             OPESCI_HIP_TRY(launch_zero(c->d_gpool, ((size_t)c->pool_elems * c->real_bytes + 15) & ~size_t(15), c->stream));

@@ -277,15 +277,16 @@ hipError_t launch_stress_sweep(const Geom& g, int real_bytes, int storage, bool 
                                const void* media, const void* coefs, int t0, int t1, const InteriorLaunch& cfg,
                                hipStream_t s, const ZFaceArgs* zf, const Boxes* boxes);
 bool stress_sweep_applies(int real_bytes, bool het, const void* coefs, int m);
-// the flat-tile velocity sweep (velocity.hip)
+// the flat-tile velocity sweep (velocity.hip); zero_last: bit a stores zeros
+// on the last interior plane of axis a for the velocity along it
 hipError_t launch_velocity_sweep(const Geom& g, int real_bytes, int storage, bool het, const void* fields,
                                  const void* media, const void* coefs, int t0, int t1, const InteriorLaunch& cfg,
-                                 hipStream_t s, const Boxes* boxes);
+                                 hipStream_t s, const Boxes* boxes, int zero_last);
 // whether launch_stress applies ZFaceArgs for this configuration
 bool stress_applies_zfaces(int real_bytes, bool het, const InteriorLaunch& cfg);
 hipError_t launch_velocity(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                            const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
-                           const Boxes* boxes = nullptr);
+                           const Boxes* boxes = nullptr, int zero_last = 0);
 // Fused step (both half steps in one x sweep) over the rows of box (one box,
 // x0..y1 set) for FP32 arithmetic on constant media with the deep z faces
 // in the sweep; x_chunk 0 picks the chunk.  fused_step_builds(m): whether

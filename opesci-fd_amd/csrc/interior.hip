@@ -948,10 +948,11 @@ hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, v
 
 hipError_t launch_velocity(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                            const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
-                           const Boxes* boxes) {
+                           const Boxes* boxes, int zero_last) {
     if (cfg.variant != 1)
-        return launch_velocity_sweep(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, boxes);
-    if (boxes) return hipErrorInvalidValue;
+        return launch_velocity_sweep(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, boxes,
+                                     zero_last);
+    if (boxes || zero_last) return hipErrorInvalidValue;
     return launch_gather<true>(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg.x_chunk, s);
 }
 

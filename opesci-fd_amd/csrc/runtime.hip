@@ -51,6 +51,11 @@ struct OpesciContext {
     Coefs<double> cd;
     std::vector<OpesciBcStmt> stmts;  // sorted by (phase, sched, axis, ranges)
     std::vector<BcLevel> levels[5];    // phases 0..3 + 4 (deep z-face rows of the stress phase, one launch)
+    // launches of a step's phases 2 and 3 (build_step_launches), and those
+    // left beside a velocity sweep that stores the zero_last planes
+    std::vector<BcLevel> runs[4], runs_sweep[4];
+    int zero_last = 0;
+    int full_steps = 0;                // steps that still run every statement (after an upload)
     BcDesc* d_desc = nullptr;
     std::vector<BcDesc> h_desc;       // host copy of the descriptors (adjoint cell lists)
     void* d_pool = nullptr;           // precomputed media-dependent boundary coefficients (compute type)
@@ -282,6 +287,131 @@ int validate(const OpesciModelDesc* d) {
 // Sort statements by (phase, launch), build one self-contained descriptor
 // per statement with the linear displacements the device uses (all indices
 // were validated against the grid; the grid is checked to fit int32 offsets).
+
+// Cells of one time level of one field that a statement writes or a term reads.
+struct CellBox {
+    int fl;
+    int lo[3], hi[3];
+    bool meets(const CellBox& o) const {
+        if (fl != o.fl) return false;
+        for (int a = 0; a < 3; ++a)
+            if (lo[a] >= o.hi[a] || o.lo[a] >= hi[a]) return false;
+        return true;
+    }
+};
+CellBox stmt_box(const OpesciBcStmt& s, int fl, int plane, int off0, int off1) {
+    CellBox b;
+    b.fl = fl;
+    b.lo[s.axis] = plane;
+    b.hi[s.axis] = plane + 1;
+    const int o[2] = {s.axis == 0 ? 1 : 0, s.axis == 2 ? 1 : 2}, off[2] = {off0, off1};
+    for (int k = 0; k < 2; ++k) {
+        b.lo[o[k]] = s.lo[k] + off[k];
+        b.hi[o[k]] = s.hi[k] + off[k];
+    }
+    return b;
+}
+CellBox written_by(const OpesciBcStmt& s) { return stmt_box(s, s.field * 2 + s.level, s.plane, 0, 0); }
+CellBox read_by(const OpesciBcStmt& s, const OpesciBcTerm& t) {
+    return stmt_box(s, t.field * 2 + t.level, t.plane, t.off[0], t.off[1]);
+}
+
+// The launches of a step: the hazard levels without the statements that write
+// what is already there, and levels that no hazard separates any more joined.
+//   * A statement without terms writes zeros.  In ghost cells that nothing
+//     else writes, those cells hold zeros from the second step after an init
+//     (which clears both levels) or an upload (whose two next steps run every
+//     statement) on: dead.  At orders 2, 6 and 8 these are all velocity
+//     statements but the ones of the next item.
+//   * When every velocity statement is of that kind, those on the staggered
+//     field's last interior plane (U at x = nx - m - 1, V and W alike) are the
+//     only writers of non-ghost cells, and the velocity sweep stores the zero
+//     itself (zero_last, one bit per axis).
+// A boundary launch takes 4 to 5 us at any size, and a z plane's lanes are a
+// line apart: velocity boundary launches per step 3 -> 0 at orders 6 and 8
+// (step of 256^3 order 8 with media 546 -> 488 us, 117x93x131 order 6 86 ->
+// 72, 61x47x53 order 8 FP64 42 -> 32), 1 -> 0 at order 2 (64^3 FP64 28.7 ->
+// 25.4).
+bool zero_stays(const OpesciContext* c, const OpesciBcStmt& s, bool last_plane) {
+    const Geom& g = c->g;
+    const int n[3] = {g.nx, g.ny, g.nz}, m = g.m;
+    const CellBox w = written_by(s);
+    if (s.nterms != 0) return false;
+    CellBox inner = w;
+    for (int a = 0; a < 3; ++a) {
+        inner.lo[a] = m;
+        inner.hi[a] = n[a] - m;
+    }
+    if (!last_plane && w.meets(inner)) return false;
+    for (const OpesciBcStmt& o : c->stmts)
+        for (int l = 0; l < 2; ++l)
+            if (o.nterms > 0 && o.field == s.field && stmt_box(o, s.field * 2 + s.level, o.plane, 0, 0).meets(w))
+                return false;
+    return s.field < 3;   // (a source may add to any stress cell)
+}
+
+int build_step_launches(OpesciContext* c, const std::vector<const OpesciBcStmt*>& src, std::vector<BcDesc>& descs) {
+    const Geom& g = c->g;
+    const int n[3] = {g.nx, g.ny, g.nz}, m = g.m;
+    bool zeros = true;                    // every velocity statement stores constant zeros
+    bool last[3] = {false, false, false};
+    auto on_last = [&](const OpesciBcStmt& s) {
+        if (s.field >= 3 || s.axis != s.field || s.plane != n[s.axis] - m - 1) return false;
+        const CellBox w = written_by(s);
+        for (int a = 0; a < 3; ++a)
+            if (a != s.axis && (w.lo[a] > m || w.hi[a] < n[a] - m)) return false;
+        return s.level == 1 && zero_stays(c, s, true);
+    };
+    for (const BcLevel& lv : c->levels[3])
+        for (int i = lv.first; i < lv.first + lv.count; ++i) {
+            if (on_last(*src[i]))
+                last[src[i]->axis] = true;
+            else if (!zero_stays(c, *src[i], false))
+                zeros = false;
+        }
+    for (int a = 0; a < 3; ++a)
+        if (zeros && last[a]) c->zero_last |= 1 << a;
+    for (int ph = 2; ph < 4; ++ph)
+        for (int sweep = 0; sweep < 2; ++sweep) {
+            // sweep 1: the launches beside a velocity sweep that stores zero_last
+            std::vector<BcLevel>& out = sweep ? c->runs_sweep[ph] : c->runs[ph];
+            std::vector<const OpesciBcStmt*> prev;
+            for (const BcLevel& lv : c->levels[ph]) {
+                BcLevel r{(int)descs.size(), 0, 0};
+                std::vector<const OpesciBcStmt*> live;
+                for (int i = lv.first; i < lv.first + lv.count; ++i) {
+                    if (zero_stays(c, *src[i], false) || (sweep && c->zero_last && on_last(*src[i]))) continue;
+                    live.push_back(src[i]);
+                    descs.push_back(BcDesc(descs[i]));
+                    r.maxpts = std::max(r.maxpts, descs.back().npts);
+                }
+                r.count = (int)descs.size() - r.first;
+                if (r.count == 0) continue;
+                // joined with the launch before when neither reads or writes
+                // what the other writes
+                bool join = !out.empty() && out.back().count + r.count <= 65535;
+                for (const OpesciBcStmt* a : prev)
+                    for (const OpesciBcStmt* b : live) {
+                        if (!join) break;
+                        join = !written_by(*a).meets(written_by(*b));
+                        for (int k = 0; join && k < b->nterms; ++k)
+                            join = !written_by(*a).meets(read_by(*b, c->h_terms[b->term0 + k]));
+                        for (int k = 0; join && k < a->nterms; ++k)
+                            join = !written_by(*b).meets(read_by(*a, c->h_terms[a->term0 + k]));
+                    }
+                if (join) {
+                    out.back().count += r.count;
+                    out.back().maxpts = std::max(out.back().maxpts, r.maxpts);
+                    prev.insert(prev.end(), live.begin(), live.end());
+                } else {
+                    out.push_back(r);
+                    prev = live;
+                }
+            }
+        }
+    return 0;
+}
+
 int build_program(OpesciContext* c, const OpesciBcTerm* terms, const OpesciBcDTerm* dterms, int ndterms,
                   int nterms) {
     // derivative programs per term (contiguous, ordered by term)
@@ -297,6 +427,7 @@ int build_program(OpesciContext* c, const OpesciBcTerm* terms, const OpesciBcDTe
     if ((int64_t)g.nx * g.sx >= ((int64_t)1 << 31)) return fail(OPESCI_EUNSUPPORTED, "grid too large for int32 offsets");
     const int64_t stride[3] = {g.sx, g.sy, 1};
     std::vector<BcDesc> descs;
+    std::vector<const OpesciBcStmt*> src;    // the statement of each descriptor
     const int n = (int)c->stmts.size();
     for (int i = 0; i < n;) {
         const OpesciBcStmt& L = c->stmts[i];
@@ -341,6 +472,7 @@ int build_program(OpesciContext* c, const OpesciBcTerm* terms, const OpesciBcDTe
                 c->pool_elems += (int64_t)nslot * d.npts;
             }
             descs.push_back(d);
+            src.push_back(&a);
             lv.maxpts = std::max(lv.maxpts, d.npts);
         }
         lv.count = (int)descs.size() - lv.first;
@@ -348,6 +480,7 @@ int build_program(OpesciContext* c, const OpesciBcTerm* terms, const OpesciBcDTe
         if (lv.count > 0) c->levels[L.phase].push_back(lv);
         i = j;
     }
+    if (int e = build_step_launches(c, src, descs)) return e;
     if (int e = upload(&c->d_desc, descs.data(), descs.size(), c->stream)) return e;
     c->h_desc = std::move(descs);
     return 0;
@@ -627,10 +760,25 @@ bool fused_step(const OpesciContext* c) {
     return c->fused_F > 0 && c->cfg.variant == 0 && zfaces_in_sweep(c);
 }
 
-int run_bc_phase(OpesciContext* c, int phase, int t0, int t1) {
-    for (const BcLevel& lv : c->levels[phase])
+int run_bc_launches(OpesciContext* c, const std::vector<BcLevel>& launches, int t0, int t1) {
+    for (const BcLevel& lv : launches)
         OPESCI_HIP_TRY(launch_bc(c->g, c->real_bytes, c->storage, c->fptr, c->d_desc, c->d_pool, lv, t0, t1, c->stream));
     return 0;
+}
+int run_bc_phase(OpesciContext* c, int phase, int t0, int t1) {
+    return run_bc_launches(c, c->levels[phase], t0, t1);
+}
+
+// whether a step runs every statement (the simple variant always does)
+bool full_step(const OpesciContext* c) { return c->cfg.variant == 1 || c->full_steps > 0; }
+// planes of zeros the velocity sweep of a step stores
+int step_zero_last(const OpesciContext* c) { return full_step(c) || fused_step(c) ? 0 : c->zero_last; }
+// the boundary launches of phase 2 or 3 of a step
+const std::vector<BcLevel>& step_launches(const OpesciContext* c, int phase) {
+    return full_step(c) ? c->levels[phase] : (step_zero_last(c) ? c->runs_sweep[phase] : c->runs[phase]);
+}
+int step_bc(OpesciContext* c, int phase, int t0, int t1) {
+    return run_bc_launches(c, step_launches(c, phase), t0, t1);
 }
 
 int step_once(OpesciContext* c, int t0) {
@@ -639,10 +787,10 @@ int step_once(OpesciContext* c, int t0) {
         OPESCI_HIP_TRY(launch_step_fused(c->g, c->storage, c->fptr, c->coefs(), t0, t1, c->zf, c->fbox, 0, c->stream));
         OPESCI_HIP_TRY(launch_stress(c->g, c->real_bytes, c->storage, c->het, c->fptr, c->mptr, c->coefs(), t0, t1,
                                      c->cfg, c->stream, &c->zf, c->d_pool, &c->frame));
-        if (int e = run_bc_phase(c, 2, t0, t1)) return e;
+        if (int e = step_bc(c, 2, t0, t1)) return e;
         OPESCI_HIP_TRY(launch_velocity(c->g, c->real_bytes, c->storage, c->het, c->fptr, c->mptr, c->coefs(), t0, t1,
                                        c->cfg, c->stream, &c->frame));
-        if (int e = run_bc_phase(c, 3, t0, t1)) return e;
+        if (int e = step_bc(c, 3, t0, t1)) return e;
         if (c->nrec > 0 || c->src_ntr)
             OPESCI_HIP_TRY(launch_record_source(c->g, c->real_bytes, c->storage, c->fptr, t1, c->nrec, c->d_rec,
                                                 c->d_trace, c->src_ntr, c->src_idx, c->d_wavelet, c->d_step,
@@ -654,10 +802,10 @@ int step_once(OpesciContext* c, int t0) {
                                  c->cfg, c->stream, zin ? &c->zf : nullptr, c->d_pool));
     if (!zin)
         if (int e = run_bc_phase(c, 4, t0, t1)) return e;
-    if (int e = run_bc_phase(c, 2, t0, t1)) return e;
+    if (int e = step_bc(c, 2, t0, t1)) return e;
     OPESCI_HIP_TRY(launch_velocity(c->g, c->real_bytes, c->storage, c->het, c->fptr, c->mptr, c->coefs(), t0, t1,
-                                   c->cfg, c->stream));
-    if (int e = run_bc_phase(c, 3, t0, t1)) return e;
+                                   c->cfg, c->stream, nullptr, step_zero_last(c)));
+    if (int e = step_bc(c, 3, t0, t1)) return e;
     if (c->nrec > 0 || c->src_ntr)
         OPESCI_HIP_TRY(launch_record_source(c->g, c->real_bytes, c->storage, c->fptr, t1, c->nrec, c->d_rec,
                                             c->d_trace, c->src_ntr, c->src_idx, c->d_wavelet, c->d_step,
@@ -836,6 +984,7 @@ int ctx_init(OpesciContext* c) {
     if (c->d_step) OPESCI_HIP_TRY(launch_zero(c->d_step, 256, c->stream));
     OPESCI_HIP_TRY(hipStreamSynchronize(c->stream));
     c->steps = 0;
+    c->full_steps = 0;
     c->initialised = true;
     return 0;
 }
@@ -845,7 +994,11 @@ int ctx_run(OpesciContext* c, int n, double* seconds) {
     c->grad_every = 0;
     if (n < 0) return fail(OPESCI_EINVAL, "negative step count");
     if (c->desc.use_graph && n >= 2) {
-        if (int e = build_graph(c)) return e;
+        const int full = c->full_steps;   // these run ahead of the graph
+        c->full_steps = 0;
+        const int e = build_graph(c);
+        c->full_steps = full;
+        if (e) return e;
     }
     hipEvent_t e0, e1;
     OPESCI_HIP_TRY(hipEventCreate(&e0));
@@ -853,10 +1006,11 @@ int ctx_run(OpesciContext* c, int n, double* seconds) {
     OPESCI_HIP_TRY(hipEventRecord(e0, c->stream));
     int left = n;
     int rc = 0;
-    if (c->steps % 2 == 1 && left > 0) {
-        rc = step_once(c, 1);
+    while (!rc && left > 0 && (c->steps % 2 == 1 || c->full_steps > 0)) {
+        rc = step_once(c, c->steps % 2);
         --left;
         ++c->steps;
+        if (c->full_steps > 0) --c->full_steps;
     }
     while (!rc && left >= 2 && c->graph) {
         hipError_t he = hipGraphLaunch(c->graph, c->stream);
@@ -903,6 +1057,7 @@ int ctx_download(OpesciContext* c, int f, int level, void* host) {
 int ctx_upload(OpesciContext* c, int f, int level, const void* host) {
     if (f < 0 || f >= NF || level < 0 || level > 1 || !host) return fail(OPESCI_EINVAL, "bad upload arguments");
     c->grad_every = 0;
+    c->full_steps = 2;   // both levels' ghosts may hold anything now
     const size_t dense = (size_t)c->g.nx * c->g.ny * c->g.nz;
     OPESCI_HIP_TRY(hipMemcpyAsync(c->d_stage, host, dense * c->real_bytes, hipMemcpyHostToDevice, c->stream));
     OPESCI_HIP_TRY(launch_pack(c->g, c->real_bytes, c->storage, c->d_stage, c->fptr[f][level], c->stream));
@@ -1102,18 +1257,19 @@ int opesci_ctx_kernel_times(OpesciContext* ctx, int32_t nsteps, double out_ms[3]
             OPESCI_HIP_TRY(launch_stress(ctx->g, ctx->real_bytes, ctx->storage, ctx->het, ctx->fptr, ctx->mptr,
                                          ctx->coefs(), t0, t1, ctx->cfg, ctx->stream, &ctx->zf, ctx->d_pool, &ctx->frame));
             OPESCI_HIP_TRY(hipEventRecord(e[2], ctx->stream));
-            rc = run_bc_phase(ctx, 2, t0, t1);
+            rc = step_bc(ctx, 2, t0, t1);
             OPESCI_HIP_TRY(hipEventRecord(e[3], ctx->stream));
             OPESCI_HIP_TRY(launch_velocity(ctx->g, ctx->real_bytes, ctx->storage, ctx->het, ctx->fptr, ctx->mptr,
                                            ctx->coefs(), t0, t1, ctx->cfg, ctx->stream, &ctx->frame));
             OPESCI_HIP_TRY(hipEventRecord(e[4], ctx->stream));
-            if (!rc) rc = run_bc_phase(ctx, 3, t0, t1);
+            if (!rc) rc = step_bc(ctx, 3, t0, t1);
             if (!rc && (ctx->nrec > 0 || ctx->src_ntr))
                 OPESCI_HIP_TRY(launch_record_source(ctx->g, ctx->real_bytes, ctx->storage, ctx->fptr, t1, ctx->nrec,
                                                     ctx->d_rec, ctx->d_trace, ctx->src_ntr, ctx->src_idx,
                                                     ctx->d_wavelet, ctx->d_step, ctx->desc.ntsteps, ctx->stream));
             OPESCI_HIP_TRY(hipEventRecord(e[5], ctx->stream));
             ++ctx->steps;
+            if (ctx->full_steps > 0) --ctx->full_steps;
         }
         for (int s = 0; s < nsteps && !rc && !fused; ++s) {
             const int t0 = ctx->steps % 2, t1 = 1 - t0;
@@ -1125,18 +1281,20 @@ int opesci_ctx_kernel_times(OpesciContext* ctx, int32_t nsteps, double out_ms[3]
                                          ctx->d_pool));
             OPESCI_HIP_TRY(hipEventRecord(e[1], ctx->stream));
             if (!zin) rc = run_bc_phase(ctx, 4, t0, t1);
-            if (!rc) rc = run_bc_phase(ctx, 2, t0, t1);
+            if (!rc) rc = step_bc(ctx, 2, t0, t1);
             OPESCI_HIP_TRY(hipEventRecord(e[2], ctx->stream));
             OPESCI_HIP_TRY(launch_velocity(ctx->g, ctx->real_bytes, ctx->storage, ctx->het, ctx->fptr, ctx->mptr,
-                                           ctx->coefs(), t0, t1, ctx->cfg, ctx->stream));
+                                           ctx->coefs(), t0, t1, ctx->cfg, ctx->stream, nullptr,
+                                           step_zero_last(ctx)));
             OPESCI_HIP_TRY(hipEventRecord(e[3], ctx->stream));
-            if (!rc) rc = run_bc_phase(ctx, 3, t0, t1);
+            if (!rc) rc = step_bc(ctx, 3, t0, t1);
             if (!rc && (ctx->nrec > 0 || ctx->src_ntr))
                 OPESCI_HIP_TRY(launch_record_source(ctx->g, ctx->real_bytes, ctx->storage, ctx->fptr, t1, ctx->nrec,
                                                     ctx->d_rec, ctx->d_trace, ctx->src_ntr, ctx->src_idx,
                                                     ctx->d_wavelet, ctx->d_step, ctx->desc.ntsteps, ctx->stream));
             OPESCI_HIP_TRY(hipEventRecord(e[4], ctx->stream));
             ++ctx->steps;
+            if (ctx->full_steps > 0) --ctx->full_steps;
         }
         OPESCI_HIP_TRY(hipStreamSynchronize(ctx->stream));
         double acc[3] = {0, 0, 0};
@@ -1175,7 +1333,8 @@ int opesci_ctx_stats(OpesciContext* ctx, int32_t out[5]) {
         int n4 = 0;
         for (const BcLevel& lv : ctx->levels[4]) n4 += lv.count;
         const bool zin = zfaces_in_sweep(ctx);
-        out[0] = (int)(ctx->levels[2].size() + ctx->levels[3].size() + (zin ? 0 : ctx->levels[4].size()));
+        out[0] = (int)(step_launches(ctx, 2).size() + step_launches(ctx, 3).size() +
+                       (zin ? 0 : ctx->levels[4].size()));
         out[1] = n4;
         out[2] = zin ? 0 : (int)ctx->levels[4].size();
         out[3] = zin ? 1 : 0;
@@ -1961,7 +2120,13 @@ int opesci_batch_run(OpesciBatch* b, int32_t nsteps, double* seconds) {
         // the graph holds an even/odd step pair: bring an odd start to even first
         int left = nsteps;
         double extra = 0;
-        if (s0 % 2 == 1 && left > 0) {
+        // (and uploaded states past their steps with every statement)
+        auto ahead = [&]() {
+            for (const OpesciContext* c : b->ctx)
+                if (c->steps % 2 == 1 || c->full_steps > 0) return true;
+            return false;
+        };
+        while (left > 0 && ahead()) {
             for (OpesciContext* c : b->ctx) {
                 double s = 0;
                 if (int e = ctx_run(c, 1, &s)) return e;

@@ -29,7 +29,7 @@ struct VelocityPtrs {
 
 template <typename R, typename S, int M, bool HET>
 __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void velocity_flat(
-    Geom g, VelocityPtrs<R, S> P, VelocityCoefs<R> c, SweepTile T, int nblocks, Boxes B) {
+    Geom g, VelocityPtrs<R, S> P, VelocityCoefs<R> c, SweepTile T, int nblocks, Boxes B, int zero_last) {
     using C = Conv<S, R>;
     constexpr int Q = 2 * M;
     // planes: Tyy and Txy (y halo), Tzz and Txz (z halo), Tyz (both)
@@ -98,6 +98,7 @@ __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void vel
     };
     fetch();
     const int pitch = s.pitch;
+    const bool zero_v = (zero_last & 2) && s.y == g.ny - M - 1, zero_w = (zero_last & 4) && s.z == g.nz - M - 1;
     auto step = [&](auto phase, int x) __attribute__((always_inline)) {
         constexpr int PH = decltype(phase)::value, b = PH & 1;
         auto q = [](int i) constexpr { return (PH + i) % Q; };
@@ -175,9 +176,12 @@ __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void vel
             for (int k = 0; k < M; ++k)
                 sw = fma(c.cv[2][2][k], LZZ[s.me + 1 + k] - (k == 0 ? oZZ : LZZ[s.me - k]), sw);
             const R sum[3] = {su, sv, sw};
+            const bool zero[3] = {(zero_last & 1) && x == g.nx - M - 1, zero_v, zero_w};
 #pragma unroll
-            for (int i = 0; i < 3; ++i)
-                C::stnt(at_byte(b1[i], here), HET ? fma(md[i], sum[i], v0[i]) : v0[i] + sum[i]);
+            for (int i = 0; i < 3; ++i) {
+                const R v = HET ? fma(md[i], sum[i], v0[i]) : v0[i] + sum[i];
+                C::stnt(at_byte(b1[i], here), zero[i] ? (R)0 : v);
+            }
         }
     };
     sweep_planes(s.xb, s.xe, step, std::make_integer_sequence<int, Q>{});
@@ -186,7 +190,8 @@ __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void vel
 // ------------------------------------------------------------------ launch
 template <typename R, typename S, int M, bool HET>
 static hipError_t run_velocity(const Geom& g, const FieldPtrs<S>& F, const MediaPtrs<R>& md, const Coefs<R>& c, int t0,
-                               int t1, const InteriorLaunch& cfg, hipStream_t s, const Boxes* boxes) {
+                               int t1, const InteriorLaunch& cfg, hipStream_t s, const Boxes* boxes,
+                               int zero_last) {
     static std::atomic<int> occ[SWEEP_THREADS / 64 + 1] = {};
     // 9 reads and 3 writes of the storage type, 3 media
     const SweepShape sh = sweep_shape<M>(
@@ -205,20 +210,20 @@ static hipError_t run_velocity(const Geom& g, const FieldPtrs<S>& F, const Media
         for (int j = 0; j < 3; ++j)
             for (int a = 0; a < M; ++a) k.cv[i][j][a] = c.cv[i][j][a];
     hipLaunchKernelGGL((velocity_flat<R, S, M, HET>), dim3((unsigned)((sh.nb + 7) / 8 * 8)), dim3((unsigned)sh.threads),
-                       0, s, g, P, k, sh.tile, sh.nb, sh.boxes);
+                       0, s, g, P, k, sh.tile, sh.nb, sh.boxes, zero_last);
     return hipGetLastError();
 }
 
 template <typename R, typename S>
 static hipError_t velocity_m(const Geom& g, bool het, const void* fields, const void* media, const void* coefs, int t0,
-                             int t1, const InteriorLaunch& cfg, hipStream_t s, const Boxes* boxes) {
+                             int t1, const InteriorLaunch& cfg, hipStream_t s, const Boxes* boxes, int zero_last) {
     const FieldPtrs<S>& F = *static_cast<const FieldPtrs<S>*>(fields);
     const MediaPtrs<R>& md = *static_cast<const MediaPtrs<R>*>(media);
     const Coefs<R>& c = *static_cast<const Coefs<R>*>(coefs);
 #define OPESCI_CASE(MM)                                                                       \
     case MM:                                                                                  \
-        return het ? run_velocity<R, S, MM, true>(g, F, md, c, t0, t1, cfg, s, boxes)         \
-                   : run_velocity<R, S, MM, false>(g, F, md, c, t0, t1, cfg, s, boxes);
+        return het ? run_velocity<R, S, MM, true>(g, F, md, c, t0, t1, cfg, s, boxes, zero_last)         \
+                   : run_velocity<R, S, MM, false>(g, F, md, c, t0, t1, cfg, s, boxes, zero_last);
     switch (g.m) {
         OPESCI_CASE(1)
         OPESCI_CASE(2)
@@ -232,13 +237,14 @@ static hipError_t velocity_m(const Geom& g, bool het, const void* fields, const 
 
 hipError_t launch_velocity_sweep(const Geom& g, int real_bytes, int storage, bool het, const void* fields,
                                  const void* media, const void* coefs, int t0, int t1, const InteriorLaunch& cfg,
-                                 hipStream_t s, const Boxes* boxes) {
-    if (real_bytes == 8) return velocity_m<double, double>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
+                                 hipStream_t s, const Boxes* boxes, int zero_last) {
+    if (real_bytes == 8)
+        return velocity_m<double, double>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes, zero_last);
     if (storage == OPESCI_STORE_F16)
-        return velocity_m<float, _Float16>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
+        return velocity_m<float, _Float16>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes, zero_last);
     if (storage == OPESCI_STORE_BF16)
-        return velocity_m<float, bf16_t>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
-    return velocity_m<float, float>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes);
+        return velocity_m<float, bf16_t>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes, zero_last);
+    return velocity_m<float, float>(g, het, fields, media, coefs, t0, t1, cfg, s, boxes, zero_last);
 }
 
 }  // namespace opesci

@@ -135,6 +135,12 @@ typedef struct OpesciBcDTerm {
  * same double operations in the same order, so the values are bit for bit
  * those of this flag, at a fraction of the cost. */
 #define OPESCI_FLAG_POINTWISE_SOLUTION 2
+/* OpesciModelDesc.flags: statements of phase 4 (deep z-face rows of the
+ * stress phase) are applied by the stress sweep for every type, medium and
+ * z size.  Without it only by the FP32 sweep on constant media with the high
+ * face at least space_order / 2 points past a multiple of 128; elsewhere
+ * they are one launch after the sweep.  The results are the same bits. */
+#define OPESCI_FLAG_ZFACES_IN_SWEEP 4
 
 typedef struct OpesciModelDesc {
     int32_t abi_version;

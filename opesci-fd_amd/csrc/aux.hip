@@ -48,6 +48,16 @@ __global__ __launch_bounds__(256) void bc_coef_kernel(Geom g, MediaPtrs<R> md, c
                 (R)((double)D->t[k].coef * vm_eval<R>(code + D->t[k].prog, D->prog_len[k], c0, 0.0, md, g, ax, ay, az));
 }
 
+// item (face, point, term): one thread each
+template <typename R>
+__global__ __launch_bounds__(256) void zpool_kernel(ZFaceArgs zf, const R* __restrict__ pool, R* __restrict__ zpool) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (int64_t)2 * ZPOOL_TERMS * zf.npts) return;
+    const int e = (int)(i % ZPOOL_TERMS), face = i >= (int64_t)ZPOOL_TERMS * zf.npts ? 1 : 0;
+    const int64_t p = i / ZPOOL_TERMS - (face ? zf.npts : 0);
+    zpool[i] = pool[zf.cpool[face][e >> 3] + (int64_t)(e & 7) * zf.npts + p];
+}
+
 struct SolTable {
     double dx[3];
     double t[NF];
@@ -349,6 +359,17 @@ hipError_t launch_bc_coef(const Geom& g, int real_bytes, const void* media, cons
 
 #define OPESCI_TYPED(RB, ST, CALL_F, CALL_D, CALL_H, CALL_B) \
     ((RB) == 8 ? (CALL_D) : (ST) == OPESCI_STORE_F16 ? (CALL_H) : (ST) == OPESCI_STORE_BF16 ? (CALL_B) : (CALL_F))
+
+hipError_t launch_zpool(int real_bytes, const ZFaceArgs& zf, const void* pool, void* zpool, hipStream_t s) {
+    const dim3 grid((unsigned)(((int64_t)2 * ZPOOL_TERMS * zf.npts + 255) / 256));
+    if (real_bytes == 8)
+        hipLaunchKernelGGL((zpool_kernel<double>), grid, dim3(256), 0, s, zf, static_cast<const double*>(pool),
+                           static_cast<double*>(zpool));
+    else
+        hipLaunchKernelGGL((zpool_kernel<float>), grid, dim3(256), 0, s, zf, static_cast<const float*>(pool),
+                           static_cast<float*>(zpool));
+    return hipGetLastError();
+}
 
 hipError_t launch_bc(const Geom& g, int real_bytes, int storage, void* fields, const BcDesc* d_desc, const void* pool,
                      const BcLevel& lvl, int t0, int t1, hipStream_t s) {

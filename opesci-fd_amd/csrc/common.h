@@ -232,7 +232,7 @@ struct Boxes {
 
 
 // Free-surface statements of the stress phase on the z faces, applied by the
-// FP32 stress sweep in place, for the deep rows x, y in [F, dim - F)
+// stress sweep in place, for the deep rows x, y in [F, dim - F)
 // (where they commute with every other statement of the phase, so they may
 // follow the interior update directly).  Per face (b = m low, dim - m - 1
 // high) the statements have three fixed forms, which the host checks
@@ -242,7 +242,8 @@ struct Boxes {
 //             Tyz, Txz(b - 1 - k) = c T(b + k) (low),  T(b + k) = c T(b - 1 - k) (high), k = 0..M-1
 //   recompute Txx, Tyy(b) = sum of 9 terms in the canonical order
 //             U(x-2..x+1), V(y-2..y+1), T(t0) (Levander, half order 2),
-//             literal coefficients (constant media).
+//             literal coefficients on constant media, else one per point for
+//             the first eight terms, from the coefficient pool.
 // Values, term order and fma accumulation equal bc_point's, so the fields
 // are those of the boundary launches bit for bit.
 // coefficient block in device memory
@@ -265,7 +266,11 @@ struct ZFaceArgs {
     int n1 = 0, npts = 0;
     const ZCoef* coef = nullptr;
     ZRecompute rc = {};
+    const void* zpool = nullptr;   // read path: the recompute's coefficients [low, high][point][Txx, Tyy][term]
+    int32_t cpool[2][2] = {};      // their places in the coefficient pool [low, high][Txx, Tyy] (term-major there)
 };
+constexpr int ZPOOL_TERMS = 16;    // coefficients of a surface point: eight each for Txx and Tyy
+constexpr int ZPOOL_ITEMS = 512;   // of a tile's plane at most (16 rows, both faces)
 
 // `boxes` (x0..y1 and n set) restricts the update to those rows (sweeps only)
 hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
@@ -283,7 +288,7 @@ hipError_t launch_velocity_sweep(const Geom& g, int real_bytes, int storage, boo
                                  const void* media, const void* coefs, int t0, int t1, const InteriorLaunch& cfg,
                                  hipStream_t s, const Boxes* boxes, int zero_last);
 // whether launch_stress applies ZFaceArgs for this configuration
-bool stress_applies_zfaces(int real_bytes, bool het, const InteriorLaunch& cfg);
+bool stress_applies_zfaces(const InteriorLaunch& cfg);
 hipError_t launch_velocity(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                            const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
                            const Boxes* boxes = nullptr, int zero_last = 0);
@@ -330,6 +335,9 @@ struct BcLevel {
 // type R), and the step launches read them from there.
 hipError_t launch_bc(const Geom& g, int real_bytes, int storage, void* fields, const BcDesc* d_desc, const void* pool,
                      const BcLevel& lvl, int t0, int t1, hipStream_t s);
+// the z faces' recompute coefficients (ZFaceArgs) from the coefficient pool
+// into `zpool`: the lines a stress sweep tile reads per plane are then its own
+hipError_t launch_zpool(int real_bytes, const ZFaceArgs& zf, const void* pool, void* zpool, hipStream_t s);
 hipError_t launch_bc_coef(const Geom& g, int real_bytes, const void* media, const BcDesc* d_desc,
                           const OpesciExprOp* d_code, void* pool, int first, int count, int maxpts, hipStream_t s);
 // adjoint (adjoint.hip); native storage, compute type given by real_bytes

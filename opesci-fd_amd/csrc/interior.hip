@@ -927,10 +927,8 @@ hipError_t launch_step_fused(const Geom& g, int storage, void* fields, const voi
     return fused_m<float>(g, fields, coefs, t0, t1, zf, box, x_chunk, s);
 }
 
-bool stress_applies_zfaces(int real_bytes, bool het, const InteriorLaunch& cfg) {
-    // FP32 arithmetic on constant media (on the read path the surface
-    // recompute takes per-point coefficients)
-    return real_bytes == 4 && !het && cfg.variant == 0;
+bool stress_applies_zfaces(const InteriorLaunch& cfg) {
+    return cfg.variant != 1;
 }
 
 hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
@@ -938,7 +936,7 @@ hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, v
                          const ZFaceArgs* zf, const void* pool, const Boxes* boxes) {
     (void)pool;
     const bool sweep = cfg.variant != 1 && stress_sweep_applies(real_bytes, het, coefs, g.m);
-    if (zf && zf->F > 0 && !(sweep && stress_applies_zfaces(real_bytes, het, cfg))) return hipErrorInvalidValue;
+    if (zf && zf->F > 0 && !(sweep && stress_applies_zfaces(cfg))) return hipErrorInvalidValue;
     if (sweep)
         return launch_stress_sweep(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, zf, boxes);
     if (boxes) return hipErrorInvalidValue;

@@ -50,6 +50,7 @@ struct OpesciContext {
     Coefs<float> cf;
     Coefs<double> cd;
     std::vector<OpesciBcStmt> stmts;  // sorted by (phase, sched, axis, ranges)
+    std::vector<uint32_t> pool_media[5];  // media (bits) the coefficients of each level read
     std::vector<BcLevel> levels[5];    // phases 0..3 + 4 (deep z-face rows of the stress phase, one launch)
     // launches of a step's phases 2 and 3 (build_step_launches), and those
     // left beside a velocity sweep that stores the zero_last planes
@@ -60,6 +61,7 @@ struct OpesciContext {
     std::vector<BcDesc> h_desc;       // host copy of the descriptors (adjoint cell lists)
     void* d_pool = nullptr;           // precomputed media-dependent boundary coefficients (compute type)
     int64_t pool_elems = 0;
+    void* d_zpool = nullptr;          // those of the z faces' recompute in the order the stress sweep reads
     OpesciBcDTerm* d_dterms = nullptr;  // derivative programs of those coefficients (adjoint)
     // adjoint state (allocated by the first opesci_ctx_gradient)
     void* abase[NF][2] = {};
@@ -579,17 +581,19 @@ int alloc_zero(OpesciContext* c, void** p, size_t bytes) {
 // The deep z-face statements (phase 4, one launch level) when they have the
 // fixed forms the stress sweep applies in place: zero and images of
 // Tzz, images of Tyz/Txz, and the Levander recompute of Txx/Tyy with its
-// terms in the canonical order.  Anything else leaves zf.F = 0 and the
-// statements run as their own launch.
+// terms in the canonical order and coefficients that are all literals
+// (constant media) or, but for the last, all pool slots in term order (read
+// path).  Anything else leaves zf.F = 0 and the statements run as their own
+// launch.
 int build_zfaces(OpesciContext* c) {
     c->zf = ZFaceArgs();
     const Geom& g = c->g;
     const int M = g.m;
     if (c->levels[4].size() != 1 || !stress_sweep_applies(c->real_bytes, c->het, c->coefs(), M)) return 0;
     const int blo = M, bhi = g.nz - M - 1;
-    // image sources within the wave that holds the face: 2M interior points
-    // on either side, and the high face at least M points into its tile
-    if (bhi - blo < 2 * M || (bhi - M) % 128 < M) return 0;
+    if (bhi - blo < 2 * M) return 0;   // the faces' image sources are distinct points
+    if (!(c->desc.flags & OPESCI_FLAG_ZFACES_IN_SWEEP) && (c->real_bytes != 4 || c->het || (bhi - M) % 128 < M))
+        return 0;
     ZFaceArgs z;
     ZCoef zc;
     memset(&zc, 0, sizeof(zc));
@@ -634,11 +638,16 @@ int build_zfaces(OpesciContext* c) {
                 const BcTermDev& t = d.t[k];
                 const int want_fl = k < 4 ? 0 : (k < 8 ? 2 : f * 2);
                 const int64_t want_disp = k < 4 ? (k - 2) * g.sx : (k < 8 ? (k - 6) * g.sy : 0);
-                // literal coefficients only (constant media)
-                if (t.fl != want_fl || t.disp != want_disp || t.cslot >= 0) return 0;
+                if (t.fl != want_fl || t.disp != want_disp) return 0;
+                if (c->het && k < 8) {
+                    if (t.cslot != k) return 0;
+                    continue;
+                }
+                if (t.cslot >= 0) return 0;
                 if (face == 1 && rec[0][f - 3] && zc.rc[k][f - 3] != t.coef) return 0;
                 zc.rc[k][f - 3] = t.coef;
             }
+            z.cpool[face][f - 3] = d.cpool;
             rec[face][f - 3] = true;
         } else {
             return 0;
@@ -660,12 +669,12 @@ int build_zfaces(OpesciContext* c) {
                 if (zc.zc[face][fi][k] != -1.0f) return 0;
     if (z.rec)
         for (int i = 0; i < 2; ++i) {
-            for (int k = 0; k < 2; ++k) {
+            if (zc.rc[8][i] != 1.0f) return 0;
+            for (int k = 0; k < 2 && !c->het; ++k) {
                 z.rc.x[k][i] = zc.rc[2 + k][i];
                 z.rc.y[k][i] = zc.rc[6 + k][i];
                 if (zc.rc[1 - k][i] != -z.rc.x[k][i] || zc.rc[5 - k][i] != -z.rc.y[k][i]) return 0;
             }
-            if (zc.rc[8][i] != 1.0f) return 0;
         }
     z.F = F;
     z.n1 = g.ny - 2 * F;
@@ -678,7 +687,7 @@ int build_zfaces(OpesciContext* c) {
 
 // whether this step's stress launch applies the deep z-face statements
 bool zfaces_in_sweep(const OpesciContext* c) {
-    return c->zf.F > 0 && stress_applies_zfaces(c->real_bytes, c->het, c->cfg);
+    return c->zf.F > 0 && stress_applies_zfaces(c->cfg);
 }
 
 // The fused step's box: the largest [F, dim - F) in x and y such that no
@@ -694,6 +703,9 @@ int build_fused(OpesciContext* c) {
     c->frame = Boxes();
     const Geom& g = c->g;
     const int M = g.m;
+    // its lanes exchange the images: the high face at least M points into its
+    // 128-point tile
+    if ((g.nz - 2 * M - 1) % 128 < M) return 0;
     if (!(c->desc.flags & OPESCI_FLAG_FUSED_STEP) || c->real_bytes != 4 || c->het || c->zf.F <= 0 ||
         !fused_step_builds(M))
         return 0;
@@ -846,7 +858,7 @@ void destroy(OpesciContext* c) {
     void* ptrs[] = {c->d_desc,  c->d_code,    c->d_sol,  c->d_solslots, c->d_soltab, c->d_partial, c->d_stage, c->d_rec,
                     c->d_trace, c->d_wavelet, c->d_step, c->d_pool,    c->d_dterms, c->d_gpool,
                     c->d_log,   c->d_ckpt,    c->d_seg,  c->d_obs,     c->d_srclog, c->d_tcells,
-                    c->d_vcells, c->d_scells, c->d_zcoef, c->d_gather, c->d_abuf};
+                    c->d_vcells, c->d_scells, c->d_zcoef, c->d_zpool, c->d_gather, c->d_abuf};
     for (int f = 0; f < NF; ++f)
         for (int l = 0; l < 2; ++l)
             if (c->abase[f][l]) (void)hipFree(c->abase[f][l]);
@@ -858,6 +870,21 @@ void destroy(OpesciContext* c) {
         if (p) (void)hipFree(p);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
+}
+
+// The media-dependent coefficients of the levels that read any of `media`
+// (bits), and their copy for the stress sweep.
+int fill_pool(OpesciContext* c, uint32_t media) {
+    if (!c->d_pool) return 0;
+    for (int ph = 0; ph < 5; ++ph)
+        for (size_t L = 0; L < c->levels[ph].size(); ++L) {
+            const BcLevel& lv = c->levels[ph][L];
+            if (c->pool_media[ph][L] & media)
+                OPESCI_HIP_TRY(launch_bc_coef(c->g, c->real_bytes, c->mptr, c->d_desc, c->d_code, c->d_pool, lv.first,
+                                              lv.count, lv.maxpts, c->stream));
+        }
+    if (c->d_zpool) OPESCI_HIP_TRY(launch_zpool(c->real_bytes, c->zf, c->d_pool, c->d_zpool, c->stream));
+    return 0;
 }
 
 int create(const OpesciModelDesc* d, OpesciContext** out) {
@@ -935,10 +962,22 @@ int create(const OpesciModelDesc* d, OpesciContext** out) {
     // time-invariant media-dependent coefficients, once (the media are ready)
     if (c->pool_elems > 0) {
         OPESCI_HIP_TRY(hipMalloc(&c->d_pool, (size_t)c->pool_elems * c->real_bytes));
+        if (c->het && c->zf.F > 0 && c->zf.rec) {
+            OPESCI_HIP_TRY(hipMalloc(&c->d_zpool, (size_t)2 * ZPOOL_TERMS * c->zf.npts * c->real_bytes));
+            c->zf.zpool = c->d_zpool;
+        }
         for (int ph = 0; ph < 5; ++ph)
-            for (const BcLevel& lv : c->levels[ph])
-                OPESCI_HIP_TRY(launch_bc_coef(c->g, c->real_bytes, c->mptr, c->d_desc, c->d_code, c->d_pool, lv.first,
-                                              lv.count, lv.maxpts, c->stream));
+            for (const BcLevel& lv : c->levels[ph]) {
+                uint32_t media = 0;
+                for (int di = lv.first; di < lv.first + lv.count; ++di)
+                    for (int k = 0; k < c->h_desc[di].nterms; ++k)
+                        for (int i = 0; c->h_desc[di].t[k].cslot >= 0 && i < c->h_desc[di].prog_len[k]; ++i) {
+                            const OpesciExprOp& o = d->bc_code[c->h_desc[di].t[k].prog + i];
+                            if (o.op == OPESCI_OP_MEDIA) media |= 1u << o.a[0];
+                        }
+                c->pool_media[ph].push_back(media);
+            }
+        if (int e = fill_pool(c.get(), ~0u)) return e;
         OPESCI_HIP_TRY(hipStreamSynchronize(c->stream));
     }
     if (int e = build_solution(c.get(), d)) return e;
@@ -2016,11 +2055,7 @@ int opesci_ctx_upload_media(OpesciContext* c, int32_t media, const void* host) {
         const size_t dense = (size_t)c->g.nx * c->g.ny * c->g.nz;
         OPESCI_HIP_TRY(hipMemcpyAsync(c->d_stage, host, dense * c->real_bytes, hipMemcpyDefault, c->stream));
         OPESCI_HIP_TRY(launch_pack_media(c->g, c->real_bytes, c->d_stage, c->mptr[media], c->stream));
-        if (c->d_pool)
-            for (int ph = 0; ph < 5; ++ph)
-                for (const BcLevel& lv : c->levels[ph])
-                    OPESCI_HIP_TRY(launch_bc_coef(c->g, c->real_bytes, c->mptr, c->d_desc, c->d_code, c->d_pool, lv.first,
-                                                  lv.count, lv.maxpts, c->stream));
+        if (int e = fill_pool(c, 1u << media)) return e;
         OPESCI_HIP_TRY(hipStreamSynchronize(c->stream));
         return 0;
     });

@@ -18,6 +18,17 @@
 // 4th order FP32 with the z faces 223 -> 204, read path 253 -> 239, FP16 278
 // -> 128; 128^3 4th order FP64 read path 82 -> 57; 160^3 FP32 107 -> 61; 161
 // x 129 x 193 8th order BF16 read path 103 -> 79; 16^3 26 -> 7.
+//
+// The z-face statements of the deep rows are done here for every type and
+// medium: as launches they touch a line per point and statement.  Sweep +
+// other launches of a step before -> after (us): 256^3 4th order read path
+// 231 + 191 -> 255 + 132, 512^3 8th order read path 2090 + 274 -> 2212 + 100,
+// 161 x 129 x 193 8th order BF16 78 + 42 -> 86 + 27.  The sweep's share is
+// 6 us image stores and 10 us coefficients at 256^3 4th order, all image
+// stores (partial lines) at 512^3.  The coefficients in the pool's term-major
+// order cost 262 instead of 255 us; non-temporal image stores 261; the high
+// surface's images taken from the lane below (one whole store per line) 201
+// instead of 187 us on constant media, the exchange costs more than the line.
 #include "sweep.h"
 
 namespace opesci {
@@ -51,10 +62,11 @@ __device__ __forceinline__ R stored(R v) {
 template <typename R, typename S, int M, bool HET, bool ZF>
 __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void stress_flat(
     Geom g, StressPtrs<R, S> P, StressCoefs<R> c, SweepTile T, int nblocks, Boxes B, ZFaceArgs zf) {
-    static_assert(!ZF || (!HET && sizeof(R) == 4), "z faces in the sweep: FP32 arithmetic, constant media");
     using C = Conv<S, R>;
     constexpr int Q = 2 * M;
+    constexpr bool ZPOOL = ZF && HET && M == 2;   // the surface recompute takes per-point coefficients
     __shared__ R lds[2][3][SweepPlane<M>::SIZE];
+    __shared__ R zlds[2][ZPOOL ? ZPOOL_ITEMS : 1];
     const int l = sweep_block(nblocks);
     if (l < 0) return;
     const SweepLane s = sweep_lane<M>(g, B, l, T);
@@ -90,6 +102,22 @@ __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void str
     // where its images go (bytes from the point itself)
     bool deep = false, image_s = false, image_n = false, surface = false, high = false;
     uint32_t to_s = 0, to_n = 0;
+    // read path: the recompute's coefficients of a plane, ZPOOL_TERMS per
+    // surface point of the tile, staged through LDS one per thread: item
+    // (face, row, term)
+    const R* pz = nullptr;
+    int zitem = 0;
+    R nz = 0;
+    if constexpr (ZPOOL) {
+        const int per = ZPOOL_TERMS * s.rows, t = (int)threadIdx.x;
+        if (zf.rec && t < ((s.low ? 1 : 0) + (s.high ? 1 : 0)) * per) {
+            const int face = (s.low ? 0 : 1) + t / per, e = t % per, y = s.y0 + e / ZPOOL_TERMS;
+            if (y >= zf.F && y < g.ny - zf.F)
+                pz = static_cast<const R*>(zf.zpool) + (int64_t)face * ZPOOL_TERMS * zf.npts +
+                     (int64_t)ZPOOL_TERMS * (y - zf.F - zf.F * zf.n1) + e % ZPOOL_TERMS;
+        }
+        zitem = ((s.low && s.z == M) || !s.low ? 0 : per) + ZPOOL_TERMS * (s.y - s.y0);
+    }
     if constexpr (ZF) {
         const int k = s.z - M, j = g.nz - M - 1 - s.z;   // points above the low and below the high surface
         deep = s.on && s.y >= zf.F && s.y < g.ny - zf.F;
@@ -105,7 +133,10 @@ __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void str
     const S* aU = bU + (int64_t)(M - 1) * g.sx;
     const S* aV = bV + (int64_t)M * g.sx;
     const S* aW = bW + (int64_t)M * g.sx;
-    auto fetch = [&]() __attribute__((always_inline)) {
+    auto fetch = [&](int x) __attribute__((always_inline)) {
+        if constexpr (ZPOOL) {
+            if (pz && x >= zf.F && x < g.nx - zf.F) nz = pz[(int64_t)x * (ZPOOL_TERMS * zf.n1)];
+        }
         // halos, then the point's own loads in one block (the order in which
         // they are waited for)
         if (s.hy) {
@@ -133,7 +164,7 @@ __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void str
             for (int k = 0; k < 5; ++k) nm[k] = Conv<R, R>::ldnt(at_byte(bm[k], om));
         }
     };
-    fetch();
+    fetch(s.xb);
     const int pitch = s.pitch;
     auto step = [&](auto phase, int x) __attribute__((always_inline)) {
         constexpr int PH = decltype(phase)::value, b = PH & 1;
@@ -171,6 +202,9 @@ __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void str
             LV[s.lz] = zV;
             LW[s.lz] = zW;
         }
+        if constexpr (ZPOOL) {
+            if (pz) zlds[b][threadIdx.x] = nz;
+        }
         const uint32_t here = own;
         if (x + 1 < s.xe) {
             own += plane;
@@ -178,7 +212,7 @@ __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void str
             oz += plane;
             ox += plane;
             om += (uint32_t)g.sx * sizeof(R);
-            fetch();
+            fetch(x + 1);
         }
         lds_barrier();
         if (s.on) {
@@ -248,14 +282,22 @@ __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void str
                                 const R qx[4] = {qU[q(0)], qU[q(1)], qU[q(2)], qU[q(3)]};
 #pragma unroll
                                 for (int i = 0; i < 2; ++i) {
-                                    R r = fma(-zf.rc.x[1][i], qx[0], (R)0);
-                                    r = fma(-zf.rc.x[0][i], qx[1], r);
-                                    r = fma(zf.rc.x[0][i], qx[2], r);
-                                    r = fma(zf.rc.x[1][i], qx[3], r);
-                                    r = fma(-zf.rc.y[1][i], vy[0], r);
-                                    r = fma(-zf.rc.y[0][i], vy[1], r);
-                                    r = fma(zf.rc.y[0][i], vy[2], r);
-                                    r = fma(zf.rc.y[1][i], vy[3], r);
+                                    R r = 0;
+                                    if constexpr (HET) {
+                                        const R* zc = zlds[b] + zitem + 8 * i;
+#pragma unroll
+                                        for (int k = 0; k < 8; ++k)
+                                            r = fma(zc[k], k < 4 ? qx[k] : vy[k - 4], r);
+                                    } else {
+                                        r = fma((R)-zf.rc.x[1][i], qx[0], r);
+                                        r = fma((R)-zf.rc.x[0][i], qx[1], r);
+                                        r = fma((R)zf.rc.x[0][i], qx[2], r);
+                                        r = fma((R)zf.rc.x[1][i], qx[3], r);
+                                        r = fma((R)-zf.rc.y[1][i], vy[0], r);
+                                        r = fma((R)-zf.rc.y[0][i], vy[1], r);
+                                        r = fma((R)zf.rc.y[0][i], vy[2], r);
+                                        r = fma((R)zf.rc.y[1][i], vy[3], r);
+                                    }
                                     out[i] = r + T0[i];
                                 }
                             }
@@ -281,15 +323,15 @@ template <typename R, typename S, int M, bool HET>
 static hipError_t run_stress(const Geom& g, const FieldPtrs<S>& F, const MediaPtrs<R>& md, const Coefs<R>& c, int t0,
                              int t1, const InteriorLaunch& cfg, hipStream_t s, const ZFaceArgs* zf,
                              const Boxes* boxes) {
-    const bool in_sweep = !HET && sizeof(R) == 4 && zf && zf->F > 0;
-    constexpr bool CAN_ZF = !HET && sizeof(R) == 4;
+    const bool in_sweep = zf && zf->F > 0;
     static std::atomic<int> occ[2][SWEEP_THREADS / 64 + 1] = {};
     // 9 reads and 6 writes of the storage type, 5 media
     const SweepShape sh = sweep_shape<M>(
         g, cfg, boxes, 15 * (int)sizeof(S) + (HET ? 5 * (int)sizeof(R) : 0), sizeof(S), [&](int threads) {
-            return in_sweep ? sweep_blocks_per_cu(stress_flat<R, S, M, HET, CAN_ZF>, occ[1], threads)
+            return in_sweep ? sweep_blocks_per_cu(stress_flat<R, S, M, HET, true>, occ[1], threads)
                             : sweep_blocks_per_cu(stress_flat<R, S, M, HET, false>, occ[0], threads);
-        });
+        },
+        in_sweep && HET && M == 2 && zf->rec ? ZPOOL_TERMS : 0);
     if (sh.nb == 0) return hipSuccess;
     StressPtrs<R, S> P;
     for (int i = 0; i < 3; ++i) P.v[i] = F.f[i][t0];
@@ -313,7 +355,7 @@ static hipError_t run_stress(const Geom& g, const FieldPtrs<S>& F, const MediaPt
             for (int i = 0; i < M; ++i) k.cs[a][b][i] = c.cs[a][b][i];
     const dim3 grid((unsigned)((sh.nb + 7) / 8 * 8)), block((unsigned)sh.threads);
     if (in_sweep)
-        hipLaunchKernelGGL((stress_flat<R, S, M, HET, CAN_ZF>), grid, block, 0, s, g, P, k, sh.tile, sh.nb, sh.boxes,
+        hipLaunchKernelGGL((stress_flat<R, S, M, HET, true>), grid, block, 0, s, g, P, k, sh.tile, sh.nb, sh.boxes,
                            *zf);
     else
         hipLaunchKernelGGL((stress_flat<R, S, M, HET, false>), grid, block, 0, s, g, P, k, sh.tile, sh.nb, sh.boxes,

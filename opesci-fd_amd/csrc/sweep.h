@@ -73,6 +73,8 @@ struct SweepLane {
     bool hy, hz, hx;     // has a y-halo / z-halo / second y-halo item
     int ly, lz, lx;      // their places in an LDS plane
     uint32_t gy, gz, gx; // their element offsets
+    bool low, high;      // the tile holds the first / last interior z
+    int y0, rows;        // the tile's rows
 };
 // whether a tile can have more y-halo points than the block has threads
 // (order 8 with more than 64 columns): a second item for the first threads
@@ -130,6 +132,10 @@ __device__ __forceinline__ SweepLane sweep_lane(const Geom& g, const Boxes& B, i
         s.lx = lr2 * s.pitch + M + c2;
         s.gx = (uint32_t)((y0 - M + lr2) * (int)g.sy + z0 + c2);
     }
+    s.low = bz == 0;
+    s.high = bz == T.ntz - 1;
+    s.y0 = y0;
+    s.rows = rows;
     if (!s.on) r = c = 0;
     s.z = z0 + c;
     s.y = y0 + r;
@@ -209,10 +215,12 @@ int sweep_blocks_per_cu(K kernel, std::atomic<int>* cache, int threads) {
     return n;
 }
 
-// `bytes`: per point and plane; `blocks_per_cu(threads)`: of the kernel.
+// `bytes`: per point and plane; `blocks_per_cu(threads)`: of the kernel;
+// `row_items`: values a tile that holds a z face stages per row and face, one
+// per thread.
 template <int M, typename F>
 SweepShape sweep_shape(const Geom& g, const InteriorLaunch& cfg, const Boxes* boxes, int bytes, int elem,
-                       F&& blocks_per_cu) {
+                       F&& blocks_per_cu, int row_items = 0) {
     SweepShape s;
     const int nzi = g.nz - 2 * M;
     s.tile.ntz = std::max(1, (nzi - (SWEEP_LAST - SWEEP_COLS) + SWEEP_COLS - 1) / SWEEP_COLS);
@@ -233,7 +241,8 @@ SweepShape sweep_shape(const Geom& g, const InteriorLaunch& cfg, const Boxes* bo
     const int most_rows = std::min(ny, cfg.tile_y > 0 ? std::min(cap, cfg.tile_y) : cap);
     const int tiles = (ny + most_rows - 1) / most_rows;
     s.tile.rows = (ny + tiles - 1) / tiles;
-    const int need = std::max(cols * s.tile.rows, std::max(2 * M * cols, 2 * M * s.tile.rows));
+    const int items = row_items * (s.tile.ntz == 1 ? 2 : 1) * s.tile.rows;
+    const int need = std::max(std::max(cols * s.tile.rows, items), std::max(2 * M * cols, 2 * M * s.tile.rows));
     s.threads = std::min(SWEEP_THREADS, (need + 63) / 64 * 64);
     long long columns = 0;
     int nx = 1;

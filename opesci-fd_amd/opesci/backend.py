@@ -18,6 +18,7 @@ from .compilation import library_path
 ABI_VERSION = 2
 FLAG_FUSED_STEP = 1
 FLAG_POINTWISE_SOLUTION = 2
+FLAG_ZFACES_IN_SWEEP = 4
 FIELDS = ('U', 'V', 'W', 'Txx', 'Tyy', 'Tzz', 'Txy', 'Tyz', 'Txz')
 MEDIA_IDS = {'rho': 0, 'vp': 1, 'vs': 2, 'beta': 3, 'lambda': 4, 'mu': 5, 'beta1': 6, 'beta2': 7, 'beta3': 8,
              'mu12': 9, 'mu13': 10, 'mu23': 11}
@@ -168,7 +169,8 @@ def make_desc(plan):
     d.storage = plan.storage_code
     d.media_arrays = 1 if plan.media_arrays else 0
     d.flags = ((FLAG_FUSED_STEP if getattr(plan, 'fuse_step', False) else 0) |
-               (FLAG_POINTWISE_SOLUTION if getattr(plan, 'pointwise_solution', False) else 0))
+               (FLAG_POINTWISE_SOLUTION if getattr(plan, 'pointwise_solution', False) else 0) |
+               (FLAG_ZFACES_IN_SWEEP if getattr(plan, 'zfaces_in_sweep', False) else 0))
     d.dt = plan.dt
     d.spacing[:] = plan.spacing
     d.media_const[:] = [float(v) for v in plan.media_const]

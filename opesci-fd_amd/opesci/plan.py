@@ -526,9 +526,10 @@ def _build_bc(grid, slots):
     b.op_of_stmt = [b.op_of_stmt[i] for i in order]
     b.seq = list(range(len(b.stmts)))
     b.fused_frame = 0
-    # split by default where the FP32 pair stress sweep applies the deep rows
-    # in place (constant media); elsewhere they would only add a launch
-    if getattr(grid, 'fuse_boundary', not grid.read and not grid.double):
+    # split by default: the stress sweep applies the deep rows in place
+    # (fuse_boundary True splits too, but off FP32 arithmetic on constant media
+    # leaves the rows to a launch of their own, which tests compare with)
+    if getattr(grid, 'fuse_boundary', True):
         dims = [d.value for d in grid.dim]
         b.fused_frame = b.fuse_z(2, 4, dims, grid.margin.value)
     b.schedule()
@@ -658,6 +659,7 @@ def build_plan(grid):
     p.stmts, p.terms, p.bc_code, p.dterms = b.arrays()
     p.stmt_seq = np.asarray(b.seq, dtype=np.int64)
     p.fused_frame = b.fused_frame
+    p.zfaces_in_sweep = getattr(grid, 'fuse_boundary', None) is None
     p.nlaunches_step = int(sum(len(set(p.stmts['sched'][p.stmts['phase'] == ph])) for ph in (2, 3)))
     p.sol_code, p.sol_off, p.sol_len = _solutions(grid, slots)
     p.src_wavelet, p.src_idx, p.rec_idx = _sources(grid, p)

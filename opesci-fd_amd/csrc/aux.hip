@@ -27,6 +27,194 @@ __global__ __launch_bounds__(256) void bc_kernel(Geom g, FieldPtrs<S> F, const B
     bc_point<R, S>(g, F, D, pool, p, D->lo0 + p / n1, D->lo1 + p % n1, t0, t1);
 }
 
+// One boundary launch of a step: a block takes the points its entry of the
+// block list names, so pieces of any size share a launch without idle blocks.
+// What bounds it on small grids and edges is the chain of dependent cache
+// misses (the fields have passed through the caches since the last step):
+// block entry, descriptor, values, store.  The descriptor comes to LDS in
+// one load of the whole block, the field pointers next to it.  On large
+// grids it is the z faces, where every value is a line of its own: a group
+// touches a line once per plane it reads or writes.
+template <typename R, typename S>
+__device__ __forceinline__ void bc_piece(const Geom& g, S* const* field, const BcPieceDesc& D,
+                                         const R* __restrict__ pool, int p0, int points) {
+    using C = Conv<S, R>;
+    int p = p0 + (int)threadIdx.x;
+    auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    const int nt = uniform(D.nterms), axis = uniform(D.axis), n1 = uniform(D.n1), end = uniform(D.npts);
+    const int64_t so0 = axis == 0 ? g.sy : g.sx, so1 = axis == 2 ? g.sy : 1;
+    S* const to = field[uniform(D.fl)];
+    auto place = [&](int q, int& pp) {
+        const int i0 = D.lo0 + q / n1, i1 = D.lo1 + q % n1;
+        pp = (i0 - D.plo0) * D.pn1 + (i1 - D.plo1);
+        return (int64_t)i0 * so0 + (int64_t)i1 * so1 + D.disp;
+    };
+    if (nt <= 1) {
+        // images and zeros, most points of all: several per thread
+        const BcPieceTerm T = D.t[0];
+        const S* from = field[T.fl] + T.disp;
+        const R* coef = nt && uniform(T.cslot) >= 0 ? pool + D.cpool : nullptr;
+        for (const int last = min(p0 + points, end); p < last; p += BC_FEW * BC_BLOCK) {
+            R v[BC_FEW];
+            int64_t dst[BC_FEW];
+#pragma unroll
+            for (int k = 0; k < BC_FEW; ++k) {
+                const int q = p + k * BC_BLOCK;
+                v[k] = (R)0;
+                if (q < last) {
+                    int pp;
+                    dst[k] = place(q, pp);
+                    if (nt) v[k] = fma(coef ? coef[pp] : (R)T.coef, C::ld(from + dst[k]), v[k]);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < BC_FEW; ++k)
+                if (p + k * BC_BLOCK < last) C::st(to + dst[k], v[k]);
+        }
+        return;
+    }
+    if (p >= end) return;
+    int pp;
+    const int64_t dst = place(p, pp);
+    // terms loaded independently, summed in term order
+    R v[BC_MAXT], c[BC_MAXT];
+#pragma unroll
+    for (int k = 0; k < BC_MAXT; ++k)
+        if (k < nt) {
+            const BcPieceTerm T = D.t[k];
+            c[k] = (R)T.coef;
+            if (uniform(T.cslot) >= 0) c[k] = pool[D.cpool + (int64_t)T.cslot * D.pnpts + pp];
+            v[k] = C::ld(field[T.fl] + dst + T.disp);
+        }
+    R acc = (R)0;
+#pragma unroll
+    for (int k = 0; k < BC_MAXT; ++k)
+        if (k < nt) acc = fma(c[k], v[k], acc);
+    C::st(to + dst, acc);
+}
+
+template <typename R, typename S, int T1>
+__device__ __forceinline__ void bc_group(const Geom& g, S* const* field, const BcGroupDesc& D,
+                                         const R* __restrict__ pool, int tile, R* slot) {
+    using C = Conv<S, R>;
+    auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    constexpr int T0 = BC_BLOCK / T1, W = T1 + 2, H = T0 + 2, P = (H * W + BC_BLOCK - 1) / BC_BLOCK;
+    static_assert(H * W <= BC_TILE_ROWS, "tile");
+    const int t = (int)threadIdx.x, axis = uniform(D.axis);
+    const int n0 = axis == 0 ? g.ny : g.nx, n1 = axis == 2 ? g.ny : g.nz;
+    const int64_t so0 = axis == 0 ? g.sy : g.sx, so1 = axis == 2 ? g.sy : 1;
+    const int tiles1 = uniform(D.tiles1);
+    const int a0 = uniform(D.lo0) + tile / tiles1 * T0, a1 = uniform(D.lo1) + tile % tiles1 * T1;
+    const int e0 = min(a0 + T0, uniform(D.hi0)), e1 = min(a1 + T1, uniform(D.hi1));   // the tile's end
+    const int ns = uniform(D.nslots), own = uniform(D.own_slot), nq = uniform(D.nstmts);
+    const BcGroupStmt& N = D.s[0];
+    // the first statement's box and the points of it the tile takes
+    const int b0 = uniform(N.plo0), c0 = b0 + uniform(N.pn0), b1 = uniform(N.plo1), c1 = b1 + uniform(N.pn1);
+    const int x0 = max(a0 + uniform(D.min0), b0), y0 = min(e0 + uniform(D.max0), c0),
+              x1 = max(a1 + uniform(D.min1), b1), y1 = min(e1 + uniform(D.max1), c1);
+    const S* from[BC_SLOTS];
+#pragma unroll
+    for (int k = 0; k < BC_SLOTS; ++k) from[k] = field[D.slot_fl[k]] + D.slot_disp[k];
+    R v[P][BC_SLOTS];
+    bool in[P];
+#pragma unroll
+    for (int r = 0; r < P; ++r) {
+        const int i = t + r * BC_BLOCK, i0 = a0 - 1 + i / W, i1 = a1 - 1 + i % W;
+        in[r] = i < H * W && i0 >= 0 && i0 < n0 && i0 <= e0 && i1 >= 0 && i1 < n1 && i1 <= e1;
+        if (!in[r]) continue;
+        const int64_t at = (int64_t)i0 * so0 + (int64_t)i1 * so1;
+        const bool computed = i0 >= b0 && i0 < c0 && i1 >= b1 && i1 < c1;
+#pragma unroll
+        for (int k = 0; k < BC_SLOTS; ++k)
+            if (k < ns && !(k == own && computed)) v[r][k] = C::ld(from[k] + at);
+    }
+#pragma unroll
+    for (int r = 0; r < P; ++r)
+        if (in[r])
+#pragma unroll
+            for (int k = 0; k < BC_SLOTS; ++k)
+                if (k < ns) slot[k * BC_TILE_ROWS + t + r * BC_BLOCK] = v[r][k];
+    __syncthreads();
+    // sum of statement q's terms at the point (i0, i1), place i of the tile
+    auto eval = [&](const BcGroupTerm* T, int q, int i0, int i1, int i) __attribute__((always_inline)) {
+        const BcGroupStmt& s = D.s[q];
+        const int nt = uniform(s.nterms);
+        R c[BC_GTERMS], x[BC_GTERMS];
+#pragma unroll
+        for (int k = 0; k < BC_GTERMS; ++k) x[k] = slot[i + T[k].at];
+#pragma unroll
+        for (int k = 0; k < BC_GTERMS; ++k) c[k] = (R)T[k].coef;
+        if (uniform(s.pooled)) {
+            const int64_t pp = s.cpool + (int64_t)(i0 - s.plo0) * s.pn1 + (i1 - s.plo1);
+            const int64_t npts = (int64_t)s.pn0 * s.pn1;
+#pragma unroll
+            for (int k = 0; k < BC_GTERMS; ++k)
+                if (k < nt && uniform(T[k].cslot) >= 0) c[k] = pool[pp + T[k].cslot * npts];
+        }
+        R acc = (R)0;
+#pragma unroll
+        for (int k = 0; k < BC_GTERMS; ++k)
+            if (k < nt) acc = fma(c[k], x[k], acc);
+        return acc;
+    };
+    BcGroupTerm T[BC_GTERMS];
+#pragma unroll
+    for (int k = 0; k < BC_GTERMS; ++k) T[k] = D.t[0][k];
+#pragma unroll
+    for (int r = 0; r < P; ++r) {
+        const int i = t + r * BC_BLOCK, i0 = a0 - 1 + i / W, i1 = a1 - 1 + i % W;
+        if (i0 < x0 || i0 >= y0 || i1 < x1 || i1 >= y1) continue;
+        const R v = stored<S, R>(eval(T, 0, i0, i1, i));
+        slot[own * BC_TILE_ROWS + i] = v;
+        if (i0 >= a0 && i0 < e0 && i1 >= a1 && i1 < e1)
+            C::st(field[uniform(N.fl)] + (int64_t)i0 * so0 + (int64_t)i1 * so1 + N.disp, v);
+    }
+    __syncthreads();
+    const int i0 = a0 + t / T1, i1 = a1 + t % T1, i = (t / T1 + 1) * W + t % T1 + 1;
+    if (i0 >= e0 || i1 >= e1) return;
+#pragma unroll
+    for (int q = 1; q < BC_GROUP; ++q)
+        if (q < nq) {
+            const BcGroupStmt& s = D.s[q];
+#pragma unroll
+            for (int k = 0; k < BC_GTERMS; ++k) T[k] = D.t[q][k];
+            if (i0 >= s.lo0 && i0 < s.hi0 && i1 >= s.lo1 && i1 < s.hi1)
+                C::st(field[uniform(s.fl)] + (int64_t)i0 * so0 + (int64_t)i1 * so1 + s.disp, eval(T, q, i0, i1, i));
+        }
+}
+
+// GROUPS: some entry of the launch is a group
+template <typename R, typename S, bool GROUPS>
+__global__ __launch_bounds__(BC_BLOCK) void bc_run_kernel(Geom g, FieldPtrs<S> F, const BcPieceAny* __restrict__ pieces,
+                                                          const R* __restrict__ pool,
+                                                          const BcBlock* __restrict__ blocks, int points, int t0,
+                                                          int t1) {
+    __shared__ __align__(16) int raw[BC_WORDS];
+    __shared__ S* field[2 * NF];   // by field * 2 + level, as the terms name it
+    __shared__ R slot[GROUPS ? BC_SLOTS * BC_TILE_ROWS : 1];
+    const BcBlock e = blocks[blockIdx.x];
+    const int t = (int)threadIdx.x;
+    if (t < BC_WORDS) {
+        raw[t] = reinterpret_cast<const int*>(pieces + e.piece)[t];
+    } else {
+        S* p = nullptr;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) {
+            if (t == BC_WORDS + 2 * f) p = t0 ? F.f[f][1] : F.f[f][0];
+            if (t == BC_WORDS + 2 * f + 1) p = t1 ? F.f[f][1] : F.f[f][0];
+        }
+        if (t < BC_WORDS + 2 * NF) field[t - BC_WORDS] = p;
+    }
+    __syncthreads();
+    const int group = __builtin_amdgcn_readfirstlane(raw[0]);   // 1 + face axis, 0: a piece
+    if (GROUPS && group == 3)
+        bc_group<R, S, BC_TILE1[2]>(g, field, *reinterpret_cast<const BcGroupDesc*>(raw), pool, e.p0, slot);
+    else if (GROUPS && group)
+        bc_group<R, S, BC_TILE1[0]>(g, field, *reinterpret_cast<const BcGroupDesc*>(raw), pool, e.p0, slot);
+    else
+        bc_piece<R, S>(g, field, *reinterpret_cast<const BcPieceDesc*>(raw), pool, e.p0, points);
+}
+
 // Per-point media-dependent coefficients of the statements [first,
 // first+count): coef * program, rounded to R exactly as bc_point does.
 template <typename R>
@@ -341,6 +529,22 @@ static hipError_t bc_t(const Geom& g, void* fields, const BcDesc* desc, const vo
     return hipGetLastError();
 }
 
+template <typename R, typename S>
+static hipError_t bc_run_t(const Geom& g, void* fields, const BcPieceAny* pieces, const void* pool, const BcBlock* blocks,
+                           const BcRun& run, int t0, int t1, hipStream_t s) {
+    if (run.count <= 0) return hipSuccess;
+    const dim3 grid((unsigned)run.count), block(BC_BLOCK);
+    const FieldPtrs<S>& F = *static_cast<const FieldPtrs<S>*>(fields);
+    const R* coef = static_cast<const R*>(pool);
+    if (run.groups)
+        hipLaunchKernelGGL((bc_run_kernel<R, S, true>), grid, block, 0, s, g, F, pieces, coef, blocks + run.first,
+                           run.points, t0, t1);
+    else
+        hipLaunchKernelGGL((bc_run_kernel<R, S, false>), grid, block, 0, s, g, F, pieces, coef, blocks + run.first,
+                           run.points, t0, t1);
+    return hipGetLastError();
+}
+
 template <typename R>
 static hipError_t bc_coef_t(const Geom& g, const void* media, const BcDesc* desc, const OpesciExprOp* code,
                             void* pool, int first, int count, int maxpts, hipStream_t s) {
@@ -377,6 +581,14 @@ hipError_t launch_bc(const Geom& g, int real_bytes, int storage, void* fields, c
                         (bc_t<double, double>(g, fields, d_desc, pool, lvl, t0, t1, s)),
                         (bc_t<float, _Float16>(g, fields, d_desc, pool, lvl, t0, t1, s)),
                         (bc_t<float, bf16_t>(g, fields, d_desc, pool, lvl, t0, t1, s)));
+}
+
+hipError_t launch_bc_run(const Geom& g, int real_bytes, int storage, void* fields, const BcPieceAny* d_pieces,
+                         const void* pool, const BcBlock* blocks, const BcRun& run, int t0, int t1, hipStream_t s) {
+    return OPESCI_TYPED(real_bytes, storage, (bc_run_t<float, float>(g, fields, d_pieces, pool, blocks, run, t0, t1, s)),
+                        (bc_run_t<double, double>(g, fields, d_pieces, pool, blocks, run, t0, t1, s)),
+                        (bc_run_t<float, _Float16>(g, fields, d_pieces, pool, blocks, run, t0, t1, s)),
+                        (bc_run_t<float, bf16_t>(g, fields, d_pieces, pool, blocks, run, t0, t1, s)));
 }
 
 static SolTable make_tab(const double* dx) {

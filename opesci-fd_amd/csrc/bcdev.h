@@ -216,4 +216,10 @@ __device__ __forceinline__ void bc_point(const Geom& g, const FieldPtrs<S>& F, c
     C::st(F.f[fl >> 1][(fl & 1) ? t1 : t0] + dst, acc);
 }
 
+// v as a statement reading it back from memory sees it
+template <typename S, typename R>
+__device__ __forceinline__ R stored(R v) {
+    return Conv<S, R>::from(Conv<S, R>::to(v));
+}
+
 }  // namespace opesci

@@ -330,9 +330,74 @@ struct BcDesc {
 struct BcLevel {
     int first, count, maxpts;   // descriptors [first, first+count)
 };
+// A piece of a statement as a step's boundary launches run it: the part
+// [lo0, ..) x [lo1, ..) of its box.  Coefficients in the pool are numbered
+// over the boxes of the whole statements (plo, pn1, pnpts).  A block copies
+// its descriptor to LDS at once: read as scalars, each line of terms is a
+// cache miss that waits for the one before it.
+constexpr int BC_BLOCK = 256;   // threads of a block
+constexpr int BC_FEW = 4;       // points of a thread at a time, of statements of at most one term
+struct BcPieceTerm {
+    int32_t fl, disp, cslot;
+    float coef;
+};
+struct BcPieceDesc {
+    int32_t group, fl, disp, nterms;   // group: 0
+    int32_t lo0, lo1, n1, npts;
+    int32_t cpool, plo0, plo1, pn1;
+    int32_t pnpts, axis, pad[2];
+    BcPieceTerm t[BC_MAXT];
+};
+// A statement and up to two on the same axis that read what it writes (a
+// velocity along the axis and those across it), over the rectangle [lo0,
+// hi0) x [lo1, hi1): a block stages the planes they read (`slots`) for a
+// tile of points and one point around it, evaluates the first statement
+// there (for the points min .. max around the tile that the others read),
+// then the others.  The same sums, rounded as the stores would.
+constexpr int BC_GROUP = 3, BC_GTERMS = 8, BC_SLOTS = 8;
+constexpr int BC_TILE1[3] = {64, 64, 32};   // points of a tile along the second axis, by face axis
+constexpr int BC_TILE_ROWS = 396;           // of a tile with the points around it at most
+struct BcGroupStmt {
+    int32_t fl, disp, nterms, cpool;
+    int32_t plo0, plo1, pn0, pn1;           // its whole box
+    int32_t lo0, hi0, lo1, hi1;             // the points it writes
+    int32_t pooled, pad[3];                 // some coefficient is in the pool
+};
+struct BcGroupTerm {
+    int32_t at, cslot;                      // slot * BC_TILE_ROWS + offset in tile points
+    float coef;
+    int32_t pad;
+};
+struct BcGroupDesc {
+    int32_t group, axis, nslots, nstmts;    // group: 1 + axis
+    int32_t lo0, lo1, hi0, hi1;
+    int32_t tiles1, own_slot, min0, max0;   // own_slot: what the first statement writes
+    int32_t min1, max1, pad[2];
+    int32_t slot_fl[BC_SLOTS], slot_disp[BC_SLOTS];
+    BcGroupStmt s[BC_GROUP];
+    BcGroupTerm t[BC_GROUP][BC_GTERMS];
+};
+union BcPieceAny {
+    BcPieceDesc piece;
+    BcGroupDesc group;
+};
+constexpr int BC_WORDS = (int)(sizeof(BcPieceAny) / 4);
+static_assert(BC_WORDS + 2 * NF <= BC_BLOCK, "a descriptor and the field pointers: one word per thread");
+// One boundary launch of a step: blocks [first, first+count) of a block
+// list, each a tile of a group or the first of up to BC_BLOCK points of a
+// piece, of up to `points` if its statement has at most one term.
+struct BcBlock {
+    int32_t piece, p0;
+};
+struct BcRun {
+    int first, count, points;
+    bool groups;
+};
 // Media-dependent coefficients are time-invariant: bc_coef evaluates every
 // program once into the pool (pool[cpool + cslot*npts + point], compute
 // type R), and the step launches read them from there.
+hipError_t launch_bc_run(const Geom& g, int real_bytes, int storage, void* fields, const BcPieceAny* d_pieces,
+                         const void* pool, const BcBlock* blocks, const BcRun& run, int t0, int t1, hipStream_t s);
 hipError_t launch_bc(const Geom& g, int real_bytes, int storage, void* fields, const BcDesc* d_desc, const void* pool,
                      const BcLevel& lvl, int t0, int t1, hipStream_t s);
 // the z faces' recompute coefficients (ZFaceArgs) from the coefficient pool

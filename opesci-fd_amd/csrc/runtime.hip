@@ -54,7 +54,9 @@ struct OpesciContext {
     std::vector<BcLevel> levels[5];    // phases 0..3 + 4 (deep z-face rows of the stress phase, one launch)
     // launches of a step's phases 2 and 3 (build_step_launches), and those
     // left beside a velocity sweep that stores the zero_last planes
-    std::vector<BcLevel> runs[4], runs_sweep[4];
+    std::vector<BcRun> runs[4], runs_sweep[4];
+    BcPieceAny* d_pieces = nullptr;
+    BcBlock* d_blocks = nullptr;       // their block lists
     int zero_last = 0;
     int full_steps = 0;                // steps that still run every statement (after an upload)
     BcDesc* d_desc = nullptr;
@@ -318,8 +320,8 @@ CellBox read_by(const OpesciBcStmt& s, const OpesciBcTerm& t) {
     return stmt_box(s, t.field * 2 + t.level, t.plane, t.off[0], t.off[1]);
 }
 
-// The launches of a step: the hazard levels without the statements that write
-// what is already there, and levels that no hazard separates any more joined.
+// The launches of a step: the statements without those that write what is
+// already there, as pieces (schedule_pieces).
 //   * A statement without terms writes zeros.  In ghost cells that nothing
 //     else writes, those cells hold zeros from the second step after an init
 //     (which clears both levels) or an upload (whose two next steps run every
@@ -352,7 +354,282 @@ bool zero_stays(const OpesciContext* c, const OpesciBcStmt& s, bool last_plane) 
     return s.field < 3;   // (a source may add to any stress cell)
 }
 
-int build_step_launches(OpesciContext* c, const std::vector<const OpesciBcStmt*>& src, std::vector<BcDesc>& descs) {
+// A statement is cut into rectangles so that what only its rim depends on
+// does not hold up the rest, and a piece's launch is one past the last of the
+// earlier pieces it conflicts with.  Statements of the lowest hazard level
+// stay whole; the others are cut `cuts` points from either end of both axes.
+// Statements that read what one of the level before them on their axis
+// writes (velocities across the axis, after the one along it) form a group
+// with it (BcGroupDesc) and share its launches, when
+//   * no statement between the two writes what the first reads or writes (the
+//     value computed in place is then the value in the cell) or conflicts
+//     with the second;
+//   * the tile holds what they read: at most one point away along either
+//     axis, in at most BC_SLOTS planes.
+// A boundary launch takes 4 to 5 us at any size; 4th order has 3 launches of
+// the stress phase and 6 of the velocity phase as levels, and 2 and 3 as
+// pieces, of which all but the first of a phase hold edges only.
+constexpr int BC_ROUND = 8 * 256;      // blocks that fit the chip
+constexpr int BC_MOST = 8;
+struct BcPiece {
+    std::vector<int> stmts;            // descriptors, the group's first one first
+    int lo[2], hi[2];
+    int run = 0;
+    std::vector<CellBox> w, r;
+    BcGroupDesc group;                 // of several statements, but for the rectangle
+};
+
+// The group of statements `ids` (descriptors), false when a tile cannot hold it.
+bool build_group(const OpesciContext* c, const std::vector<const OpesciBcStmt*>& src, const std::vector<BcDesc>& descs,
+                 const std::vector<int>& ids, BcGroupDesc& out) {
+    memset(&out, 0, sizeof(out));
+    const OpesciBcStmt& a = *src[ids[0]];
+    const int W = BC_TILE1[a.axis] + 2;
+    const int64_t stride[3] = {c->g.sx, c->g.sy, 1};
+    out.group = 1 + a.axis;
+    out.axis = a.axis;
+    out.nstmts = (int)ids.size();
+    auto slot = [&](int fl, int plane) {
+        const int32_t disp = (int32_t)(plane * stride[a.axis]);
+        for (int k = 0; k < out.nslots; ++k)
+            if (out.slot_fl[k] == fl && out.slot_disp[k] == disp) return k;
+        if (out.nslots == BC_SLOTS) return -1;
+        out.slot_fl[out.nslots] = fl;
+        out.slot_disp[out.nslots] = disp;
+        return out.nslots++;
+    };
+    out.own_slot = slot(a.field * 2 + a.level, a.plane);
+    int32_t* lo[2] = {&out.min0, &out.min1};
+    int32_t* hi[2] = {&out.max0, &out.max1};
+    for (int q = (int)ids.size() - 1; q >= 0; --q) {
+        const OpesciBcStmt& s = *src[ids[q]];
+        const BcDesc& d = descs[ids[q]];
+        if (s.nterms > BC_GTERMS) return false;
+        BcGroupStmt& o = out.s[q];
+        o.fl = d.fl;
+        o.disp = d.disp;
+        o.nterms = d.nterms;
+        o.cpool = d.cpool;
+        o.plo0 = d.lo0;
+        o.plo1 = d.lo1;
+        o.pn0 = d.npts / d.n1;
+        o.pn1 = d.n1;
+        for (int k = 0; k < s.nterms; ++k) {
+            const OpesciBcTerm& t = c->h_terms[s.term0 + k];
+            const int sl = slot(t.field * 2 + t.level, t.plane);
+            if (sl < 0 || (q == 0 && sl == out.own_slot)) return false;
+            for (int d2 = 0; d2 < 2; ++d2) {
+                // reads of the first statement's values widen the points it
+                // takes, whose own reads stay within one point of the tile
+                if (q > 0 && sl == out.own_slot) {
+                    *lo[d2] = std::min(*lo[d2], t.off[d2]);
+                    *hi[d2] = std::max(*hi[d2], t.off[d2]);
+                }
+                const int l = q == 0 ? *lo[d2] : 0, h = q == 0 ? *hi[d2] : 0;
+                if (t.off[d2] + l < -1 || t.off[d2] + h > 1) return false;
+            }
+            out.t[q][k] = {sl * BC_TILE_ROWS + t.off[0] * W + t.off[1], d.t[k].cslot, d.t[k].coef, 0};
+            if (d.t[k].cslot >= 0) o.pooled = 1;
+        }
+    }
+    return true;
+}
+
+void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& src, const std::vector<int>& order,
+                     const std::vector<int>& cuts, const std::vector<BcDesc>& descs,
+                     std::vector<BcPieceAny>& out_pieces, std::vector<BcBlock>& blocks, std::vector<BcRun>& out) {
+    const Geom& g = c->g;
+    const int n[3] = {g.nx, g.ny, g.nz};
+    auto terms = [&](const OpesciBcStmt& s) { return c->h_terms.data() + s.term0; };
+    auto conflict = [&](const OpesciBcStmt& a, const OpesciBcStmt& b) {
+        const CellBox wa = written_by(a), wb = written_by(b);
+        if (wa.meets(wb)) return true;
+        for (int k = 0; k < b.nterms; ++k)
+            if (wa.meets(read_by(b, terms(b)[k]))) return true;
+        for (int k = 0; k < a.nterms; ++k)
+            if (wb.meets(read_by(a, terms(a)[k]))) return true;
+        return false;
+    };
+    // groups, in the place of their first statement
+    std::vector<std::vector<int>> units;
+    std::vector<int> unit_of(order.size());
+    for (int at = 0; at < (int)order.size(); ++at) {
+        const OpesciBcStmt& s = *src[order[at]];
+        int with = -1;
+        for (int b = at - 1; b >= 0 && with < 0 && s.sched > 0; --b) {
+            const OpesciBcStmt& a = *src[order[b]];
+            if (a.axis != s.axis || a.sched != s.sched - 1 || units[unit_of[b]][0] != order[b]) continue;
+            for (int k = 0; k < s.nterms; ++k) {
+                const OpesciBcTerm& t = terms(s)[k];
+                if (t.field == a.field && t.level == a.level && t.plane == a.plane) with = b;
+            }
+        }
+        if (with >= 0) {
+            const OpesciBcStmt& a = *src[order[with]];
+            std::vector<int> ids = units[unit_of[with]];
+            ids.push_back(order[at]);
+            BcGroupDesc d;
+            bool ok = (int)ids.size() <= BC_GROUP && build_group(c, src, descs, ids, d);
+            for (int b = with + 1; b <= at && ok; ++b) {
+                const OpesciBcStmt& x = *src[order[b]];
+                const CellBox w = written_by(x);
+                ok = !w.meets(written_by(a)) && (b == at || unit_of[b] == unit_of[with] || !conflict(x, s));
+                for (int k = 0; k < a.nterms && ok; ++k) ok = !w.meets(read_by(a, terms(a)[k]));
+            }
+            if (!ok) with = -1;
+        }
+        if (with >= 0) {
+            unit_of[at] = unit_of[with];
+            units[unit_of[at]].push_back(order[at]);
+        } else {
+            unit_of[at] = (int)units.size();
+            units.push_back({order[at]});
+        }
+    }
+    std::vector<BcPiece> pieces;
+    // pieces by what they write, and reads by what they read (piece, box)
+    std::vector<std::pair<int, CellBox>> writes[2 * NF], reads[2 * NF];
+    for (const std::vector<int>& u : units) {
+        const OpesciBcStmt& s = *src[u[0]];
+        const int o[2] = {s.axis == 0 ? 1 : 0, s.axis == 2 ? 1 : 2};
+        std::vector<int> cut[2];
+        for (int d = 0; d < 2; ++d) {
+            int lo = s.lo[d], hi = s.hi[d];
+            for (int id : u) {
+                lo = std::min(lo, src[id]->lo[d]);
+                hi = std::max(hi, src[id]->hi[d]);
+            }
+            cut[d] = {lo, hi};
+            if (s.sched > 0)
+                for (int f : cuts)
+                    for (int v : {f, n[o[d]] - f})
+                        if (v > lo && v < hi) cut[d].push_back(v);
+            std::sort(cut[d].begin(), cut[d].end());
+            cut[d].erase(std::unique(cut[d].begin(), cut[d].end()), cut[d].end());
+        }
+        const size_t first = pieces.size();
+        for (size_t i = 0; i + 1 < cut[0].size(); ++i)
+            for (size_t j = 0; j + 1 < cut[1].size(); ++j) {
+                BcPiece p;
+                p.stmts = u;
+                p.lo[0] = cut[0][i], p.hi[0] = cut[0][i + 1];
+                p.lo[1] = cut[1][j], p.hi[1] = cut[1][j + 1];
+                for (size_t q = 0; q < u.size(); ++q) {
+                    OpesciBcStmt part = *src[u[q]];
+                    for (int d = 0; d < 2; ++d) {
+                        part.lo[d] = std::max(part.lo[d], p.lo[d]);
+                        part.hi[d] = std::min(part.hi[d], p.hi[d]);
+                    }
+                    if (part.lo[0] >= part.hi[0] || part.lo[1] >= part.hi[1]) continue;
+                    p.w.push_back(written_by(part));
+                    for (int k = 0; k < part.nterms; ++k) {
+                        const OpesciBcTerm& t = terms(part)[k];
+                        OpesciBcStmt a = s;
+                        bool out_of_box = false;
+                        for (int d = 0; d < 2; ++d) {
+                            a.lo[d] = std::max(s.lo[d], part.lo[d] + t.off[d]);
+                            a.hi[d] = std::min(s.hi[d], part.hi[d] + t.off[d]);
+                            out_of_box |= part.lo[d] + t.off[d] < s.lo[d] || part.hi[d] + t.off[d] > s.hi[d];
+                        }
+                        const bool computed = q > 0 && t.field == s.field && t.level == s.level && t.plane == s.plane;
+                        if (!computed || out_of_box) p.r.push_back(read_by(part, t));
+                        if (computed && a.lo[0] < a.hi[0] && a.lo[1] < a.hi[1])
+                            for (int x = 0; x < a.nterms; ++x) p.r.push_back(read_by(a, terms(a)[x]));
+                    }
+                }
+                for (const CellBox& w : p.w) {
+                    for (const auto& q : writes[w.fl])
+                        if (pieces[q.first].run >= p.run && q.second.meets(w)) p.run = pieces[q.first].run + 1;
+                    for (const auto& q : reads[w.fl])
+                        if (pieces[q.first].run >= p.run && q.second.meets(w)) p.run = pieces[q.first].run + 1;
+                }
+                for (const CellBox& r : p.r)
+                    for (const auto& q : writes[r.fl])
+                        if (pieces[q.first].run >= p.run && q.second.meets(r)) p.run = pieces[q.first].run + 1;
+                // joined with the piece before it along the second axis
+                if (pieces.size() > first) {
+                    BcPiece& l = pieces.back();
+                    if (l.run == p.run && l.lo[0] == p.lo[0] && l.hi[0] == p.hi[0] && l.hi[1] == p.lo[1]) {
+                        l.hi[1] = p.hi[1];
+                        l.w.insert(l.w.end(), p.w.begin(), p.w.end());
+                        l.r.insert(l.r.end(), p.r.begin(), p.r.end());
+                        continue;
+                    }
+                }
+                if (u.size() > 1) (void)build_group(c, src, descs, u, p.group);
+                pieces.push_back(std::move(p));
+            }
+        for (size_t q = first; q < pieces.size(); ++q) {
+            for (const CellBox& w : pieces[q].w) writes[w.fl].push_back({(int)q, w});
+            for (const CellBox& r : pieces[q].r) reads[r.fl].push_back({(int)q, r});
+        }
+    }
+    int runs = 0;
+    for (const BcPiece& p : pieces) runs = std::max(runs, p.run + 1);
+    // z planes first: a line per point, the longest blocks
+    std::stable_sort(pieces.begin(), pieces.end(), [&](const BcPiece& a, const BcPiece& b) {
+        return (src[a.stmts[0]]->axis == 2) > (src[b.stmts[0]]->axis == 2);
+    });
+    for (int run = 0; run < runs; ++run) {
+        // points of a block, where a point costs little: as many as keep the
+        // launch within one round of the chip (8 blocks on a CU), so that a
+        // block fetches its descriptor for more than one round of loads
+        BcRun r{(int)blocks.size(), 0, BC_BLOCK, false};
+        int64_t all = 0;
+        for (const BcPiece& p : pieces)
+            if (p.run == run && p.stmts.size() == 1) all += (int64_t)(p.hi[0] - p.lo[0]) * (p.hi[1] - p.lo[1]);
+        while (r.points < BC_MOST * BC_BLOCK && all > (int64_t)BC_ROUND * r.points) r.points *= 2;
+        for (const BcPiece& p : pieces) {
+            if (p.run != run) continue;
+            r.groups |= p.stmts.size() > 1;
+            BcPieceAny any;
+            memset(&any, 0, sizeof(any));
+            const int n0 = p.hi[0] - p.lo[0], n1 = p.hi[1] - p.lo[1];
+            int nb, each = 1;
+            if (p.stmts.size() > 1) {
+                BcGroupDesc& d = any.group;
+                d = p.group;
+                d.lo0 = p.lo[0], d.hi0 = p.hi[0];
+                d.lo1 = p.lo[1], d.hi1 = p.hi[1];
+                const int T1 = BC_TILE1[d.axis], T0 = BC_BLOCK / T1;
+                d.tiles1 = (n1 + T1 - 1) / T1;
+                nb = (n0 + T0 - 1) / T0 * d.tiles1;
+                for (int q = 0; q < d.nstmts; ++q) {
+                    const OpesciBcStmt& s = *src[p.stmts[q]];
+                    d.s[q].lo0 = std::max(s.lo[0], p.lo[0]), d.s[q].hi0 = std::min(s.hi[0], p.hi[0]);
+                    d.s[q].lo1 = std::max(s.lo[1], p.lo[1]), d.s[q].hi1 = std::min(s.hi[1], p.hi[1]);
+                }
+            } else {
+                const BcDesc& o = descs[p.stmts[0]];
+                BcPieceDesc& d = any.piece;
+                d.fl = o.fl;
+                d.disp = o.disp;
+                d.nterms = o.nterms;
+                d.axis = o.axis;
+                d.lo0 = p.lo[0];
+                d.lo1 = p.lo[1];
+                d.n1 = n1;
+                d.npts = n0 * n1;
+                d.cpool = o.cpool;
+                d.plo0 = o.lo0;
+                d.plo1 = o.lo1;
+                d.pn1 = o.n1;
+                d.pnpts = o.npts;
+                for (int k = 0; k < o.nterms; ++k) d.t[k] = {o.t[k].fl, o.t[k].disp, o.t[k].cslot, o.t[k].coef};
+                each = o.nterms <= 1 ? r.points : BC_BLOCK;
+                nb = (d.npts + each - 1) / each;
+            }
+            for (int b = 0; b < nb; ++b)
+                blocks.push_back(BcBlock{(int32_t)out_pieces.size(), b * each});
+            out_pieces.push_back(any);
+        }
+        r.count = (int)blocks.size() - r.first;
+        out.push_back(r);
+    }
+}
+
+int build_step_launches(OpesciContext* c, const std::vector<const OpesciBcStmt*>& src,
+                        const std::vector<BcDesc>& descs) {
     const Geom& g = c->g;
     const int n[3] = {g.nx, g.ny, g.nz}, m = g.m;
     bool zeros = true;                    // every velocity statement stores constant zeros
@@ -373,45 +650,25 @@ int build_step_launches(OpesciContext* c, const std::vector<const OpesciBcStmt*>
         }
     for (int a = 0; a < 3; ++a)
         if (zeros && last[a]) c->zero_last |= 1 << a;
+    std::vector<BcPieceAny> pieces;
+    std::vector<BcBlock> blocks;
     for (int ph = 2; ph < 4; ++ph)
         for (int sweep = 0; sweep < 2; ++sweep) {
             // sweep 1: the launches beside a velocity sweep that stores zero_last
-            std::vector<BcLevel>& out = sweep ? c->runs_sweep[ph] : c->runs[ph];
-            std::vector<const OpesciBcStmt*> prev;
-            for (const BcLevel& lv : c->levels[ph]) {
-                BcLevel r{(int)descs.size(), 0, 0};
-                std::vector<const OpesciBcStmt*> live;
-                for (int i = lv.first; i < lv.first + lv.count; ++i) {
-                    if (zero_stays(c, *src[i], false) || (sweep && c->zero_last && on_last(*src[i]))) continue;
-                    live.push_back(src[i]);
-                    descs.push_back(BcDesc(descs[i]));
-                    r.maxpts = std::max(r.maxpts, descs.back().npts);
-                }
-                r.count = (int)descs.size() - r.first;
-                if (r.count == 0) continue;
-                // joined with the launch before when neither reads or writes
-                // what the other writes
-                bool join = !out.empty() && out.back().count + r.count <= 65535;
-                for (const OpesciBcStmt* a : prev)
-                    for (const OpesciBcStmt* b : live) {
-                        if (!join) break;
-                        join = !written_by(*a).meets(written_by(*b));
-                        for (int k = 0; join && k < b->nterms; ++k)
-                            join = !written_by(*a).meets(read_by(*b, c->h_terms[b->term0 + k]));
-                        for (int k = 0; join && k < a->nterms; ++k)
-                            join = !written_by(*b).meets(read_by(*a, c->h_terms[a->term0 + k]));
-                    }
-                if (join) {
-                    out.back().count += r.count;
-                    out.back().maxpts = std::max(out.back().maxpts, r.maxpts);
-                    prev.insert(prev.end(), live.begin(), live.end());
-                } else {
-                    out.push_back(r);
-                    prev = live;
-                }
+            std::vector<BcRun>& out = sweep ? c->runs_sweep[ph] : c->runs[ph];
+            if (sweep && (ph == 2 || !c->zero_last)) {
+                out = c->runs[ph];
+                continue;
             }
+            std::vector<int> live;
+            for (const BcLevel& lv : c->levels[ph])
+                for (int i = lv.first; i < lv.first + lv.count; ++i)
+                    if (!zero_stays(c, *src[i], false) && !(sweep && on_last(*src[i]))) live.push_back(i);
+            schedule_pieces(c, src, live, ph == 2 ? std::vector<int>{m + 1, 2 * m + 1} : std::vector<int>{2 * m}, descs,
+                            pieces, blocks, out);
         }
-    return 0;
+    if (int e = upload(&c->d_pieces, pieces.data(), pieces.size(), c->stream)) return e;
+    return upload(&c->d_blocks, blocks.data(), blocks.size(), c->stream);
 }
 
 int build_program(OpesciContext* c, const OpesciBcTerm* terms, const OpesciBcDTerm* dterms, int ndterms,
@@ -772,25 +1029,29 @@ bool fused_step(const OpesciContext* c) {
     return c->fused_F > 0 && c->cfg.variant == 0 && zfaces_in_sweep(c);
 }
 
-int run_bc_launches(OpesciContext* c, const std::vector<BcLevel>& launches, int t0, int t1) {
-    for (const BcLevel& lv : launches)
+int run_bc_phase(OpesciContext* c, int phase, int t0, int t1) {
+    for (const BcLevel& lv : c->levels[phase])
         OPESCI_HIP_TRY(launch_bc(c->g, c->real_bytes, c->storage, c->fptr, c->d_desc, c->d_pool, lv, t0, t1, c->stream));
     return 0;
-}
-int run_bc_phase(OpesciContext* c, int phase, int t0, int t1) {
-    return run_bc_launches(c, c->levels[phase], t0, t1);
 }
 
 // whether a step runs every statement (the simple variant always does)
 bool full_step(const OpesciContext* c) { return c->cfg.variant == 1 || c->full_steps > 0; }
 // planes of zeros the velocity sweep of a step stores
 int step_zero_last(const OpesciContext* c) { return full_step(c) || fused_step(c) ? 0 : c->zero_last; }
-// the boundary launches of phase 2 or 3 of a step
-const std::vector<BcLevel>& step_launches(const OpesciContext* c, int phase) {
-    return full_step(c) ? c->levels[phase] : (step_zero_last(c) ? c->runs_sweep[phase] : c->runs[phase]);
+// the boundary launches of phase 2 or 3 of a step that does not run every statement
+const std::vector<BcRun>& step_runs(const OpesciContext* c, int phase) {
+    return step_zero_last(c) ? c->runs_sweep[phase] : c->runs[phase];
+}
+int step_launch_count(const OpesciContext* c, int phase) {
+    return (int)(full_step(c) ? c->levels[phase].size() : step_runs(c, phase).size());
 }
 int step_bc(OpesciContext* c, int phase, int t0, int t1) {
-    return run_bc_launches(c, step_launches(c, phase), t0, t1);
+    if (full_step(c)) return run_bc_phase(c, phase, t0, t1);
+    for (const BcRun& r : step_runs(c, phase))
+        OPESCI_HIP_TRY(launch_bc_run(c->g, c->real_bytes, c->storage, c->fptr, c->d_pieces, c->d_pool, c->d_blocks, r, t0,
+                                     t1, c->stream));
+    return 0;
 }
 
 int step_once(OpesciContext* c, int t0) {
@@ -855,7 +1116,7 @@ void destroy(OpesciContext* c) {
             if (c->base[f][l]) (void)hipFree(c->base[f][l]);
     for (int i = 0; i < OPESCI_M_COUNT; ++i)
         if (c->mbase[i]) (void)hipFree(c->mbase[i]);
-    void* ptrs[] = {c->d_desc,  c->d_code,    c->d_sol,  c->d_solslots, c->d_soltab, c->d_partial, c->d_stage, c->d_rec,
+    void* ptrs[] = {c->d_pieces, c->d_blocks, c->d_desc,  c->d_code,    c->d_sol,  c->d_solslots, c->d_soltab, c->d_partial, c->d_stage, c->d_rec,
                     c->d_trace, c->d_wavelet, c->d_step, c->d_pool,    c->d_dterms, c->d_gpool,
                     c->d_log,   c->d_ckpt,    c->d_seg,  c->d_obs,     c->d_srclog, c->d_tcells,
                     c->d_vcells, c->d_scells, c->d_zcoef, c->d_zpool, c->d_gather, c->d_abuf};
@@ -1372,8 +1633,7 @@ int opesci_ctx_stats(OpesciContext* ctx, int32_t out[5]) {
         int n4 = 0;
         for (const BcLevel& lv : ctx->levels[4]) n4 += lv.count;
         const bool zin = zfaces_in_sweep(ctx);
-        out[0] = (int)(step_launches(ctx, 2).size() + step_launches(ctx, 3).size() +
-                       (zin ? 0 : ctx->levels[4].size()));
+        out[0] = step_launch_count(ctx, 2) + step_launch_count(ctx, 3) + (zin ? 0 : (int)ctx->levels[4].size());
         out[1] = n4;
         out[2] = zin ? 0 : (int)ctx->levels[4].size();
         out[3] = zin ? 1 : 0;

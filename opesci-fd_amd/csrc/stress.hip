@@ -29,6 +29,7 @@
 // order cost 262 instead of 255 us; non-temporal image stores 261; the high
 // surface's images taken from the lane below (one whole store per line) 201
 // instead of 187 us on constant media, the exchange costs more than the line.
+#include "bcdev.h"
 #include "sweep.h"
 
 namespace opesci {
@@ -52,12 +53,6 @@ struct StressPtrs {
     const R* mu;
     const R* ms[3];
 };
-
-// v as a boundary statement reading it back from memory sees it
-template <typename S, typename R>
-__device__ __forceinline__ R stored(R v) {
-    return Conv<S, R>::from(Conv<S, R>::to(v));
-}
 
 template <typename R, typename S, int M, bool HET, bool ZF>
 __global__ __launch_bounds__(SWEEP_THREADS, sizeof(R) * M <= 8 ? 5 : 2) void stress_flat(

@@ -555,7 +555,8 @@ __global__ void adj_receiver_kernel(FieldPtrs<R> F, AdjPtrs<R> B, int t1, int ng
     }
 }
 
-__global__ void set_step_kernel(int* step, int value) { *step = value; }
+// the step counter of both levels (record_source_kernel)
+__global__ void set_step_kernel(int* step, int value) { step[threadIdx.x] = value; }
 
 // Txx, Tyy, Tzz of one cell at level t: read into buf (mode 0) or written
 // from it (mode 1); brackets the point source in the reverse sweep.
@@ -864,7 +865,7 @@ hipError_t launch_copy_cells(int real_bytes, void* dst, int td, void* src, int t
 }
 
 hipError_t launch_set_step(int* step, int value, hipStream_t s) {
-    hipLaunchKernelGGL(set_step_kernel, dim3(1), dim3(1), 0, s, step, value);
+    hipLaunchKernelGGL(set_step_kernel, dim3(1), dim3(2), 0, s, step, value);
     return hipGetLastError();
 }
 

@@ -96,6 +96,8 @@ struct OpesciContext {
     int partial_cap = 0;
     void* d_stage = nullptr;          // dense staging buffer (one field level, real_t)
     int32_t* d_rec = nullptr;
+    int32_t* d_at_src = nullptr;      // the receivers in the source's cell
+    int nat_src = 0;
     void* d_trace = nullptr;          // [ntsteps][nrec][4] of the arithmetic type
     float* d_wavelet = nullptr;
     int* d_step = nullptr;
@@ -1054,6 +1056,14 @@ int step_bc(OpesciContext* c, int phase, int t0, int t1) {
     return 0;
 }
 
+// receivers (the first nrec), source and step counter of a step into level t1
+int record_source(OpesciContext* c, void* fp, int t1, int nrec) {
+    OPESCI_HIP_TRY(launch_record_source(c->g, c->real_bytes, c->storage, fp, t1, nrec, nrec > 0 ? c->nat_src : 0,
+                                        c->d_rec, c->d_at_src, c->d_trace, c->src_ntr, c->src_idx, c->d_wavelet,
+                                        c->d_step, c->desc.ntsteps, c->stream));
+    return 0;
+}
+
 int step_once(OpesciContext* c, int t0) {
     const int t1 = 1 - t0;
     if (fused_step(c)) {
@@ -1065,9 +1075,7 @@ int step_once(OpesciContext* c, int t0) {
                                        c->cfg, c->stream, &c->frame));
         if (int e = step_bc(c, 3, t0, t1)) return e;
         if (c->nrec > 0 || c->src_ntr)
-            OPESCI_HIP_TRY(launch_record_source(c->g, c->real_bytes, c->storage, c->fptr, t1, c->nrec, c->d_rec,
-                                                c->d_trace, c->src_ntr, c->src_idx, c->d_wavelet, c->d_step,
-                                                c->desc.ntsteps, c->stream));
+            if (int e = record_source(c, c->fptr, t1, c->nrec)) return e;
         return 0;
     }
     const bool zin = zfaces_in_sweep(c);
@@ -1080,9 +1088,7 @@ int step_once(OpesciContext* c, int t0) {
                                    c->cfg, c->stream, nullptr, step_zero_last(c)));
     if (int e = step_bc(c, 3, t0, t1)) return e;
     if (c->nrec > 0 || c->src_ntr)
-        OPESCI_HIP_TRY(launch_record_source(c->g, c->real_bytes, c->storage, c->fptr, t1, c->nrec, c->d_rec,
-                                            c->d_trace, c->src_ntr, c->src_idx, c->d_wavelet, c->d_step,
-                                            c->desc.ntsteps, c->stream));
+        if (int e = record_source(c, c->fptr, t1, c->nrec)) return e;
     return 0;
 }
 
@@ -1116,7 +1122,7 @@ void destroy(OpesciContext* c) {
             if (c->base[f][l]) (void)hipFree(c->base[f][l]);
     for (int i = 0; i < OPESCI_M_COUNT; ++i)
         if (c->mbase[i]) (void)hipFree(c->mbase[i]);
-    void* ptrs[] = {c->d_pieces, c->d_blocks, c->d_desc,  c->d_code,    c->d_sol,  c->d_solslots, c->d_soltab, c->d_partial, c->d_stage, c->d_rec,
+    void* ptrs[] = {c->d_pieces, c->d_blocks, c->d_desc,  c->d_code,    c->d_sol,  c->d_solslots, c->d_soltab, c->d_partial, c->d_stage, c->d_rec, c->d_at_src,
                     c->d_trace, c->d_wavelet, c->d_step, c->d_pool,    c->d_dterms, c->d_gpool,
                     c->d_log,   c->d_ckpt,    c->d_seg,  c->d_obs,     c->d_srclog, c->d_tcells,
                     c->d_vcells, c->d_scells, c->d_zcoef, c->d_zpool, c->d_gather, c->d_abuf};
@@ -1258,6 +1264,11 @@ int create(const OpesciModelDesc* d, OpesciContext** out) {
             if (int e = upload(&c->d_wavelet, d->src_wavelet, (size_t)std::max(d->ntsteps, 1) * c->src_ntr, c->stream))
                 return e;
             for (int a = 0; a < 3; ++a) c->src_idx[a] = d->src_idx[a];
+            std::vector<int32_t> at;
+            for (int r = 0; r < c->nrec; ++r)
+                if (std::equal(c->src_idx, c->src_idx + 3, c->h_rec.data() + 3 * r)) at.push_back(r);
+            c->nat_src = (int)at.size();
+            if (int e = upload(&c->d_at_src, at.data(), at.size(), c->stream)) return e;
         }
     }
     // pointers into the caller's arrays are not kept
@@ -1564,9 +1575,7 @@ int opesci_ctx_kernel_times(OpesciContext* ctx, int32_t nsteps, double out_ms[3]
             OPESCI_HIP_TRY(hipEventRecord(e[4], ctx->stream));
             if (!rc) rc = step_bc(ctx, 3, t0, t1);
             if (!rc && (ctx->nrec > 0 || ctx->src_ntr))
-                OPESCI_HIP_TRY(launch_record_source(ctx->g, ctx->real_bytes, ctx->storage, ctx->fptr, t1, ctx->nrec,
-                                                    ctx->d_rec, ctx->d_trace, ctx->src_ntr, ctx->src_idx,
-                                                    ctx->d_wavelet, ctx->d_step, ctx->desc.ntsteps, ctx->stream));
+                rc = rc ? rc : record_source(ctx, ctx->fptr, t1, ctx->nrec);
             OPESCI_HIP_TRY(hipEventRecord(e[5], ctx->stream));
             ++ctx->steps;
             if (ctx->full_steps > 0) --ctx->full_steps;
@@ -1589,9 +1598,7 @@ int opesci_ctx_kernel_times(OpesciContext* ctx, int32_t nsteps, double out_ms[3]
             OPESCI_HIP_TRY(hipEventRecord(e[3], ctx->stream));
             if (!rc) rc = step_bc(ctx, 3, t0, t1);
             if (!rc && (ctx->nrec > 0 || ctx->src_ntr))
-                OPESCI_HIP_TRY(launch_record_source(ctx->g, ctx->real_bytes, ctx->storage, ctx->fptr, t1, ctx->nrec,
-                                                    ctx->d_rec, ctx->d_trace, ctx->src_ntr, ctx->src_idx,
-                                                    ctx->d_wavelet, ctx->d_step, ctx->desc.ntsteps, ctx->stream));
+                rc = rc ? rc : record_source(ctx, ctx->fptr, t1, ctx->nrec);
             OPESCI_HIP_TRY(hipEventRecord(e[4], ctx->stream));
             ++ctx->steps;
             if (ctx->full_steps > 0) --ctx->full_steps;
@@ -2236,9 +2243,7 @@ int opesci_ctx_gradient_reverse(OpesciContext* c) {
                 if (c->src_ntr)
                     OPESCI_HIP_TRY(launch_src_cells(c->g, c->real_bytes, fp, t1, si[0], si[1], si[2], sl, 0, c->stream));
                 // source and step counter only (the traces are already recorded)
-                OPESCI_HIP_TRY(launch_record_source(c->g, c->real_bytes, c->storage, fp, t1, 0, c->d_rec, c->d_trace,
-                                                    c->src_ntr, c->src_idx, c->d_wavelet, c->d_step, c->desc.ntsteps,
-                                                    c->stream));
+                if (int e = record_source(c, fp, t1, 0)) return e;
                 if (c->src_ntr)
                     OPESCI_HIP_TRY(launch_src_cells(c->g, c->real_bytes, fp, t1, si[0], si[1], si[2], sl + 3 * rb, 0,
                                                     c->stream));

@@ -836,6 +836,38 @@ hipError_t launch_src_cells(const Geom& g, int real_bytes, void* fields, int t, 
     return hipGetLastError();
 }
 
+// The cells outside the interior of all nine fields at a level, from S to D:
+// whole rows in the x and y ghosts, m points at either end of the others, 32
+// lanes on a row.
+constexpr int GHOST_ROWS = 64;   // of a block
+template <typename R>
+__global__ __launch_bounds__(256) void copy_ghosts_kernel(Geom g, FieldPtrs<R> D, FieldPtrs<R> S, int t) {
+    const int f = blockIdx.y, lane = (int)threadIdx.x & 31, m = g.m;
+    R* d = t ? D.f[f][1] : D.f[f][0];
+    const R* s = t ? S.f[f][1] : S.f[f][0];
+    const int rows = g.nx * g.ny, r0 = (int)blockIdx.x * GHOST_ROWS;
+    for (int r = r0 + ((int)threadIdx.x >> 5); r < min(r0 + GHOST_ROWS, rows); r += 8) {
+        const int x = r / g.ny, y = r % g.ny;
+        const bool inner = x >= m && x < g.nx - m && y >= m && y < g.ny - m;
+        const int64_t at = g.at(x, y, 0);
+        for (int i = lane; i < (inner ? 2 * m : g.nz); i += 32) {
+            const int64_t q = at + (inner && i >= m ? g.nz - 2 * m + i : i);
+            d[q] = s[q];
+        }
+    }
+}
+
+hipError_t launch_copy_ghosts(const Geom& g, int real_bytes, void* dst, void* src, int t, hipStream_t s) {
+    const dim3 grid((unsigned)((g.nx * g.ny + GHOST_ROWS - 1) / GHOST_ROWS), NF);
+    if (real_bytes == 8)
+        hipLaunchKernelGGL((copy_ghosts_kernel<double>), grid, dim3(256), 0, s, g,
+                           *static_cast<const FieldPtrs<double>*>(dst), *static_cast<const FieldPtrs<double>*>(src), t);
+    else
+        hipLaunchKernelGGL((copy_ghosts_kernel<float>), grid, dim3(256), 0, s, g,
+                           *static_cast<const FieldPtrs<float>*>(dst), *static_cast<const FieldPtrs<float>*>(src), t);
+    return hipGetLastError();
+}
+
 // D.f[field][td][offset] = S.f[field][ts][offset] for a list of distinct
 // cells, each entry (offset << 4) | field.
 template <typename R>

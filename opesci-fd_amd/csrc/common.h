@@ -458,6 +458,8 @@ hipError_t launch_adj_receivers(const Geom& g, int real_bytes, void* fields, voi
                                 const int32_t* start, const int64_t* cell, const int32_t* order, const float* obs,
                                 hipStream_t s);
 hipError_t launch_set_step(int* step, int value, hipStream_t s);
+// non-interior cells of the nine fields at level t (FieldPtrs images)
+hipError_t launch_copy_ghosts(const Geom& g, int real_bytes, void* dst, void* src, int t, hipStream_t s);
 // dst level td := src level ts at a list of distinct cells ((offset << 4) |
 // field), both FieldPtrs images of the compute type
 hipError_t launch_copy_cells(int real_bytes, void* dst, int td, void* src, int ts, const int64_t* cells, int n,

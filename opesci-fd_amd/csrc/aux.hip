@@ -2,6 +2,7 @@
 // layout conversion and point source / receivers.
 #include "bcdev.h"
 
+#include <algorithm>
 #include <mutex>
 
 namespace opesci {
@@ -459,7 +460,12 @@ __global__ void unpack_kernel(Geom g, const S* __restrict__ field, R* __restrict
     }
 }
 
-__global__ void zero_kernel(uint4* __restrict__ p, size_t n16) {
+struct ZeroList {
+    uint4* p[2 * NF];
+};
+// n16 16-byte words of each array of the list (blockIdx.y)
+__global__ void zero_kernel(ZeroList list, size_t n16) {
+    uint4* p = list.p[blockIdx.y];
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += (size_t)gridDim.x * blockDim.x)
         p[i] = make_uint4(0, 0, 0, 0);
 }
@@ -793,9 +799,19 @@ hipError_t launch_pack_media(const Geom& g, int real_bytes, const void* dense, v
     return real_bytes == 8 ? pack_t<double, double>(g, dense, media, s) : pack_t<float, float>(g, dense, media, s);
 }
 
-hipError_t launch_zero(void* p, size_t bytes, hipStream_t s) {
+hipError_t launch_zero(void* p, size_t bytes, hipStream_t s) { return launch_zero_all(&p, 1, bytes, s); }
+
+// One launch for up to 2 * NF arrays of one size: an init clears 18, a reverse
+// sweep 30, and on small grids a launch costs what it clears (16^3: 18
+// launches 0.2 ms of an init's 0.4).
+hipError_t launch_zero_all(void* const* p, int n, size_t bytes, hipStream_t s) {
     const size_t n16 = bytes / 16;
-    if (n16) hipLaunchKernelGGL(zero_kernel, dim3(2048), dim3(256), 0, s, (uint4*)p, n16);
+    if (n <= 0 || n16 == 0) return hipSuccess;
+    if (n > 2 * NF) return hipErrorInvalidValue;
+    ZeroList list = {};
+    for (int i = 0; i < n; ++i) list.p[i] = static_cast<uint4*>(p[i]);
+    const unsigned blocks = (unsigned)std::min<size_t>(n > 1 ? 512 : 2048, (n16 + 255) / 256);
+    hipLaunchKernelGGL(zero_kernel, dim3(blocks, (unsigned)n), dim3(256), 0, s, list, n16);
     return hipGetLastError();
 }
 

@@ -509,6 +509,7 @@ hipError_t launch_pack(const Geom& g, int real_bytes, int storage, const void* d
 hipError_t launch_unpack(const Geom& g, int real_bytes, int storage, const void* field, void* dense, hipStream_t s);
 hipError_t launch_pack_media(const Geom& g, int real_bytes, const void* dense, void* media, hipStream_t s);
 hipError_t launch_zero(void* p, size_t bytes, hipStream_t s);
+hipError_t launch_zero_all(void* const* p, int n, size_t bytes, hipStream_t s);   // n <= 2 * NF
 hipError_t launch_record_source(const Geom& g, int real_bytes, int storage, void* fields, int t1, int nrec, int nat,
                                 const int32_t* d_rec, const int32_t* d_at_src, void* d_trace, int src_on,
                                 const int32_t* src_idx, const float* d_wavelet, int* d_step, int ntsteps,

@@ -1286,8 +1286,7 @@ int create(const OpesciModelDesc* d, OpesciContext** out) {
 
 int ctx_init(OpesciContext* c) {
     c->grad_every = 0;
-    for (int f = 0; f < NF; ++f)
-        for (int l = 0; l < 2; ++l) OPESCI_HIP_TRY(launch_zero(c->base[f][l], c->field_bytes, c->stream));
+    OPESCI_HIP_TRY(launch_zero_all(&c->base[0][0], 2 * NF, c->field_bytes, c->stream));
     OPESCI_HIP_TRY(launch_initial(c->g, c->real_bytes, c->storage, c->fptr, c->mptr, c->sol, c->desc.spacing,
                                   c->desc.dt, c->stream));
     if (int e = run_bc_phase(c, 0, 0, 0)) return e;
@@ -2175,10 +2174,9 @@ int opesci_ctx_gradient_reverse(OpesciContext* c) {
         const bool keep_t0 = c->grad_keep_t0;
         const size_t slot = keep_t0 ? (size_t)NF * c->field_bytes : state;
         // reverse sweep, segment by segment
-        for (int f = 0; f < NF; ++f)
-            for (int l = 0; l < 2; ++l) OPESCI_HIP_TRY(launch_zero(c->abase[f][l], c->field_bytes, c->stream));
+        OPESCI_HIP_TRY(launch_zero_all(&c->abase[0][0], 2 * NF, c->field_bytes, c->stream));
         const size_t mbytes = (size_t)c->g.total * c->real_bytes;
-        for (int i = 0; i < OPESCI_M_COUNT; ++i) OPESCI_HIP_TRY(launch_zero(c->gbase[i], mbytes, c->stream));
+        OPESCI_HIP_TRY(launch_zero_all(c->gbase, OPESCI_M_COUNT, mbytes, c->stream));
         if (c->d_gpool)
             OPESCI_HIP_TRY(launch_zero(c->d_gpool, ((size_t)c->pool_elems * c->real_bytes + 15) & ~size_t(15), c->stream));
         const size_t rb = c->real_bytes, zo = (size_t)c->g.zoff * rb;

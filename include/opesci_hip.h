@@ -194,7 +194,8 @@ typedef struct OpesciModelDesc {
     int32_t tile_y;
     int32_t x_chunk;
     int32_t kernel_variant;     /* 0 default (LDS/register-queue sweep), 1 plain gather, 2 sweep
-                                   without the z-face statements in the stress kernel */
+                                   without the z-face statements in the stress kernel (and so
+                                   without the fused step) */
     int32_t use_graph;          /* capture the time loop in a hipGraph */
     /* adjoint: derivative programs of the media-dependent boundary
      * coefficients (may be 0 / null when no gradient is asked for) */
@@ -278,7 +279,7 @@ int opesci_ctx_kernel_times(OpesciContext* ctx, int32_t nsteps, double out_ms[3]
 /* Execution plan of a context: out[0] = boundary launches per time step,
  * out[1] = phase-4 statements (deep z-face rows of the stress phase),
  * out[2] = launches they take (0 or 1), out[3] = 1 when the stress sweep
- * applies them in place (FP32 sweeps), else 0, out[4] = the fused
+ * applies them in place (kernel_variant 0), else 0, out[4] = the fused
  * step's margin F (its box is [F, dim - F) in x and y; 0: separate stress
  * and velocity launches).  No reference counterpart. */
 int opesci_ctx_stats(OpesciContext* ctx, int32_t out[5]);

@@ -207,7 +207,7 @@ int fail(int code, const std::string& msg);
     } while (0)
 
 // ---------------------------------------------------------------- launch wrappers
-// interior kernels; variant 0, 2 = flat-tile sweep, 1 = plain gather
+// interior kernels; variant 0, 2 = flat-tile sweep (2 without the z faces), 1 = plain gather
 struct InteriorLaunch {
     int variant;
     int tile_y;

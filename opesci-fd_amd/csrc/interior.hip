@@ -927,8 +927,9 @@ hipError_t launch_step_fused(const Geom& g, int storage, void* fields, const voi
     return fused_m<float>(g, fields, coefs, t0, t1, zf, box, x_chunk, s);
 }
 
+// 2 leaves them to their own launch, as 1 does
 bool stress_applies_zfaces(const InteriorLaunch& cfg) {
-    return cfg.variant != 1;
+    return cfg.variant == 0;
 }
 
 hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,

@@ -325,9 +325,10 @@ class Context(object):
         return int(out[4])
 
     def configure(self, kernel_variant=0, tile_y=0, x_chunk=0):
-        """Interior launch configuration: kernel_variant 0 or 2 sweep, 1 gather;
-        tile_y rows of a tile at most, x_chunk planes of a block (0: chosen);
-        results are the same for every one."""
+        """Interior launch configuration: kernel_variant 0 sweep, 1 gather, 2
+        sweep with the z-face statements of the stress phase in a launch of
+        their own; tile_y rows of a tile at most, x_chunk planes of a block (0:
+        chosen); results are the same for every one."""
         _check(self.lib.opesci_ctx_configure(self.h, kernel_variant, tile_y, x_chunk), 'opesci_ctx_configure')
 
     def _observed(self, observed):

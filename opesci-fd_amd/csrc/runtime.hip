@@ -58,6 +58,7 @@ struct OpesciContext {
     BcPieceAny* d_pieces = nullptr;
     BcBlock* d_blocks = nullptr;       // their block lists
     int zero_last = 0;
+    bool left_out = false;             // some statement is in none of the runs (zero_stays)
     int full_steps = 0;                // steps that still run every statement (after an upload)
     BcDesc* d_desc = nullptr;
     std::vector<BcDesc> h_desc;       // host copy of the descriptors (adjoint cell lists)
@@ -664,8 +665,11 @@ int build_step_launches(OpesciContext* c, const std::vector<const OpesciBcStmt*>
             }
             std::vector<int> live;
             for (const BcLevel& lv : c->levels[ph])
-                for (int i = lv.first; i < lv.first + lv.count; ++i)
-                    if (!zero_stays(c, *src[i], false) && !(sweep && on_last(*src[i]))) live.push_back(i);
+                for (int i = lv.first; i < lv.first + lv.count; ++i) {
+                    const bool stays = zero_stays(c, *src[i], false);
+                    c->left_out |= stays;
+                    if (!stays && !(sweep && on_last(*src[i]))) live.push_back(i);
+                }
             schedule_pieces(c, src, live, ph == 2 ? std::vector<int>{m + 1, 2 * m + 1} : std::vector<int>{2 * m}, descs,
                             pieces, blocks, out);
         }
@@ -1367,7 +1371,9 @@ int ctx_download(OpesciContext* c, int f, int level, void* host) {
 int ctx_upload(OpesciContext* c, int f, int level, const void* host) {
     if (f < 0 || f >= NF || level < 0 || level > 1 || !host) return fail(OPESCI_EINVAL, "bad upload arguments");
     c->grad_every = 0;
-    c->full_steps = 2;   // both levels' ghosts may hold anything now
+    // a velocity's ghosts may hold anything now, in both levels: the zeros
+    // that steps leave out are written once more (4th order leaves out none)
+    if (f < 3 && c->left_out) c->full_steps = 2;
     const size_t dense = (size_t)c->g.nx * c->g.ny * c->g.nz;
     OPESCI_HIP_TRY(hipMemcpyAsync(c->d_stage, host, dense * c->real_bytes, hipMemcpyHostToDevice, c->stream));
     OPESCI_HIP_TRY(launch_pack(c->g, c->real_bytes, c->storage, c->d_stage, c->fptr[f][level], c->stream));
@@ -2407,6 +2413,46 @@ int opesci_batch_destroy(OpesciBatch* b) {
     });
 }
 
+// Up to `most` single steps of every context, side by side on the contexts'
+// streams, while one is at an odd step or still runs every statement; the
+// steps taken and the GPU seconds from the first start to the last end.
+static int batch_ahead(OpesciBatch* b, int most, int* taken, double* seconds) {
+    auto ahead = [&]() {
+        for (const OpesciContext* c : b->ctx)
+            if (c->steps % 2 == 1 || c->full_steps > 0) return true;
+        return false;
+    };
+    *taken = 0;
+    *seconds = 0;
+    if (most <= 0 || !ahead()) return 0;
+    struct Events {
+        std::vector<hipEvent_t> e;
+        ~Events() {
+            for (hipEvent_t v : e)
+                if (v) (void)hipEventDestroy(v);
+        }
+    } ev{std::vector<hipEvent_t>(b->ctx.size() + 1, nullptr)};   // the start, then each context's end
+    for (hipEvent_t& v : ev.e) OPESCI_HIP_TRY(hipEventCreate(&v));
+    for (OpesciContext* c : b->ctx) OPESCI_HIP_TRY(hipStreamSynchronize(c->stream));
+    OPESCI_HIP_TRY(hipEventRecord(ev.e[0], b->ctx[0]->stream));
+    int rc = 0;
+    for (; *taken < most && !rc && ahead(); ++*taken)
+        for (OpesciContext* c : b->ctx) {
+            c->grad_every = 0;
+            if (!rc) rc = step_once(c, c->steps % 2);
+            ++c->steps;
+            if (c->full_steps > 0) --c->full_steps;
+        }
+    for (size_t i = 0; i < b->ctx.size(); ++i) OPESCI_HIP_TRY(hipEventRecord(ev.e[i + 1], b->ctx[i]->stream));
+    for (size_t i = 0; i < b->ctx.size(); ++i) {
+        float ms = 0;
+        OPESCI_HIP_TRY(hipEventSynchronize(ev.e[i + 1]));
+        OPESCI_HIP_TRY(hipEventElapsedTime(&ms, ev.e[0], ev.e[i + 1]));
+        *seconds = std::max(*seconds, ms * 1e-3);
+    }
+    return rc;
+}
+
 int opesci_batch_run(OpesciBatch* b, int32_t nsteps, double* seconds) {
     return guarded([&]() -> int {
         if (!b) return fail(OPESCI_EINVAL, "null batch");
@@ -2416,23 +2462,12 @@ int opesci_batch_run(OpesciBatch* b, int32_t nsteps, double* seconds) {
             if (!c->initialised) return fail(OPESCI_ESTATE, "every context of the batch must be initialised");
             if (c->steps != s0) return fail(OPESCI_ESTATE, "contexts of a batch must be at the same step");
         }
-        // the graph holds an even/odd step pair: bring an odd start to even first
-        int left = nsteps;
+        // the graph holds an even/odd step pair: bring an odd start to even
+        // first, and uploaded states past their steps with every statement
+        int left = nsteps, taken = 0;
         double extra = 0;
-        // (and uploaded states past their steps with every statement)
-        auto ahead = [&]() {
-            for (const OpesciContext* c : b->ctx)
-                if (c->steps % 2 == 1 || c->full_steps > 0) return true;
-            return false;
-        };
-        while (left > 0 && ahead()) {
-            for (OpesciContext* c : b->ctx) {
-                double s = 0;
-                if (int e = ctx_run(c, 1, &s)) return e;
-                extra += s;
-            }
-            --left;
-        }
+        if (int e = batch_ahead(b, left, &taken, &extra)) return e;
+        left -= taken;
         if (left >= 2)
             if (int e = batch_graph(b)) return e;
         hipEvent_t e0, e1;

@@ -276,12 +276,10 @@ constexpr int ZPOOL_ITEMS = 512;   // of a tile's plane at most (16 rows, both f
 hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                          const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
                          const ZFaceArgs* zf = nullptr, const void* pool = nullptr, const Boxes* boxes = nullptr);
-// the flat-tile stress sweep (stress.hip) and whether it takes these
-// coefficients
+// the flat-tile stress sweep (stress.hip)
 hipError_t launch_stress_sweep(const Geom& g, int real_bytes, int storage, bool het, const void* fields,
                                const void* media, const void* coefs, int t0, int t1, const InteriorLaunch& cfg,
                                hipStream_t s, const ZFaceArgs* zf, const Boxes* boxes);
-bool stress_sweep_applies(int real_bytes, bool het, const void* coefs, int m);
 // the flat-tile velocity sweep (velocity.hip); zero_last: bit a stores zeros
 // on the last interior plane of axis a for the velocity along it
 hipError_t launch_velocity_sweep(const Geom& g, int real_bytes, int storage, bool het, const void* fields,

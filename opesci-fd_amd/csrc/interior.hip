@@ -24,8 +24,7 @@
 //    what they share); 2 leaves the z-face statements of the stress phase to
 //    their own launch.
 //  * 1, gather (here): one thread per (y,z) column, every stencil operand
-//    loaded from global memory (caches only); the simple reference form, and
-//    the stress kernel of models whose off-axis normal coefficients differ.
+//    loaded from global memory (caches only); the simple reference form.
 // All keep one accumulation order, so their results agree bit for bit.
 //
 // Also here: the opt-in fused step.
@@ -936,12 +935,10 @@ hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, v
                          const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
                          const ZFaceArgs* zf, const void* pool, const Boxes* boxes) {
     (void)pool;
-    const bool sweep = cfg.variant != 1 && stress_sweep_applies(real_bytes, het, coefs, g.m);
-    if (zf && zf->F > 0 && !(sweep && stress_applies_zfaces(cfg))) return hipErrorInvalidValue;
-    if (sweep)
+    if (zf && zf->F > 0 && !stress_applies_zfaces(cfg)) return hipErrorInvalidValue;
+    if (cfg.variant != 1)
         return launch_stress_sweep(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, zf, boxes);
     if (boxes) return hipErrorInvalidValue;
-    // sums not shared by the normal stresses: the gather kernel takes any coefficients
     return launch_gather<false>(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg.x_chunk, s);
 }
 

@@ -852,7 +852,7 @@ int build_zfaces(OpesciContext* c) {
     c->zf = ZFaceArgs();
     const Geom& g = c->g;
     const int M = g.m;
-    if (c->levels[4].size() != 1 || !stress_sweep_applies(c->real_bytes, c->het, c->coefs(), M)) return 0;
+    if (c->levels[4].size() != 1) return 0;
     const int blo = M, bhi = g.nz - M - 1;
     if (bhi - blo < 2 * M) return 0;   // the faces' image sources are distinct points
     if (!(c->desc.flags & OPESCI_FLAG_ZFACES_IN_SWEEP) && (c->real_bytes != 4 || c->het || (bhi - M) % 128 < M))

@@ -246,7 +246,7 @@ struct Boxes {
 //             the first eight terms, from the coefficient pool.
 // Values, term order and fma accumulation equal bc_point's, so the fields
 // are those of the boundary launches bit for bit.
-// coefficient block in device memory
+// coefficient block of the fused step, in device memory
 struct ZCoef {
     float rc[9][2];        // recompute literals [term][Txx, Tyy], the same at both faces
     float zc[2][3][MAXM];  // image coefficients [low, high][Tzz, Tyz, Txz][k]

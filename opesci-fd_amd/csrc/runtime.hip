@@ -55,12 +55,13 @@ struct OpesciContext {
     // launches of a step's phases 2 and 3 (build_step_launches), and those
     // left beside a velocity sweep that stores the zero_last planes
     std::vector<BcRun> runs[4], runs_sweep[4];
-    BcPieceAny* d_pieces = nullptr;
-    BcBlock* d_blocks = nullptr;       // their block lists
+    const BcPieceAny* d_pieces = nullptr;
+    const BcBlock* d_blocks = nullptr; // their block lists
     int zero_last = 0;
     bool left_out = false;             // some statement is in none of the runs (zero_stays)
     int full_steps = 0;                // steps that still run every statement (after an upload)
-    BcDesc* d_desc = nullptr;
+    const BcDesc* d_desc = nullptr;
+    char* d_program = nullptr;         // all three
     std::vector<BcDesc> h_desc;       // host copy of the descriptors (adjoint cell lists)
     void* d_pool = nullptr;           // precomputed media-dependent boundary coefficients (compute type)
     int64_t pool_elems = 0;
@@ -89,8 +90,7 @@ struct OpesciContext {
     void* d_srclog = nullptr;         // Txx/Tyy/Tzz at the source before and after injection, per step
     float* d_obs = nullptr;
     OpesciExprOp* d_code = nullptr;
-    OpesciExprOp* d_sol = nullptr;    // the analytic programs, split (SolProg)
-    SolSlot* d_solslots = nullptr;
+    char* d_sol = nullptr;            // the analytic programs, split, and their slots (SolProg)
     double* d_soltab = nullptr;
     SolProg sol;
     double* d_partial = nullptr;
@@ -116,7 +116,7 @@ struct OpesciContext {
     Boxes fbox, frame;              // its box and the four boxes of rows around it
     int grad_every = 0;             // checkpoint interval of the last forward pass (0: none pending)
     bool grad_keep_t0 = false;
-    ZCoef* d_zcoef = nullptr;       // their coefficient block (device)
+    ZCoef* d_zcoef = nullptr;       // their coefficient block (device), of the fused step
     // adjoint: fixed-order gathers of the boundary transposes per level
     // (phases 2-4) and the receivers grouped by cell
     std::vector<OpesciBcDTerm> h_dterms;
@@ -342,8 +342,8 @@ CellBox read_by(const OpesciBcStmt& s, const OpesciBcTerm& t) {
 bool zero_stays(const OpesciContext* c, const OpesciBcStmt& s, bool last_plane) {
     const Geom& g = c->g;
     const int n[3] = {g.nx, g.ny, g.nz}, m = g.m;
+    if (s.nterms != 0 || s.field >= 3) return false;   // (a source may add to any stress cell)
     const CellBox w = written_by(s);
-    if (s.nterms != 0) return false;
     CellBox inner = w;
     for (int a = 0; a < 3; ++a) {
         inner.lo[a] = m;
@@ -351,10 +351,8 @@ bool zero_stays(const OpesciContext* c, const OpesciBcStmt& s, bool last_plane) 
     }
     if (!last_plane && w.meets(inner)) return false;
     for (const OpesciBcStmt& o : c->stmts)
-        for (int l = 0; l < 2; ++l)
-            if (o.nterms > 0 && o.field == s.field && stmt_box(o, s.field * 2 + s.level, o.plane, 0, 0).meets(w))
-                return false;
-    return s.field < 3;   // (a source may add to any stress cell)
+        if (o.nterms > 0 && o.field == s.field && stmt_box(o, w.fl, o.plane, 0, 0).meets(w)) return false;
+    return true;
 }
 
 // A statement is cut into rectangles so that what only its rim depends on
@@ -374,13 +372,69 @@ bool zero_stays(const OpesciContext* c, const OpesciBcStmt& s, bool last_plane) 
 // pieces, of which all but the first of a phase hold edges only.
 constexpr int BC_ROUND = 8 * 256;      // blocks that fit the chip
 constexpr int BC_MOST = 8;
-struct BcPiece {
+struct BcUnit {
     std::vector<int> stmts;            // descriptors, the group's first one first
-    int lo[2], hi[2];
-    int run = 0;
-    std::vector<CellBox> w, r;
     BcGroupDesc group;                 // of several statements, but for the rectangle
 };
+struct BcPiece {
+    int unit;
+    int lo[2], hi[2];
+    int run;
+};
+
+// the cells of b in q, where the two differ along one axis and meet or touch there
+bool take_in(CellBox& q, const CellBox& b) {
+    if (q.fl != b.fl) return false;
+    int differ = 0, axis = 0;
+    for (int a = 0; a < 3; ++a)
+        if (q.lo[a] != b.lo[a] || q.hi[a] != b.hi[a]) {
+            ++differ;
+            axis = a;
+        }
+    if (differ > 1 || q.lo[axis] > b.hi[axis] || b.lo[axis] > q.hi[axis]) return false;
+    q.lo[axis] = std::min(q.lo[axis], b.lo[axis]);
+    q.hi[axis] = std::max(q.hi[axis], b.hi[axis]);
+    return true;
+}
+// b into a list of boxes; the terms of a stencil become one
+void add_box(std::vector<CellBox>& list, const CellBox& b) {
+    for (CellBox& q : list)
+        if (take_in(q, b)) return;
+    list.push_back(b);
+}
+// cells that a piece of launch `run` writes or reads
+struct BcAccess {
+    int run;
+    CellBox box;
+};
+// (among those from `from` on)
+void add_box(std::vector<BcAccess>& list, size_t from, int run, const CellBox& b) {
+    for (size_t i = from; i < list.size(); ++i)
+        if (list[i].run == run && take_in(list[i].box, b)) return;
+    list.push_back(BcAccess{run, b});
+}
+// What a statement writes and reads.  `rel`: its reads relative to a point
+// along the loop's axes, planes as they are; `r`: of its whole box.
+struct BcCells {
+    CellBox w;
+    std::vector<CellBox> r, rel;
+};
+// the cells that the points of `box` read through `rel`
+CellBox reads_of(const CellBox& box, const CellBox& rel, int axis) {
+    CellBox b = rel;
+    for (int a = 0; a < 3; ++a)
+        if (a != axis) {
+            b.lo[a] = box.lo[a] + rel.lo[a];
+            b.hi[a] = box.hi[a] + rel.hi[a] - 1;
+        }
+    return b;
+}
+CellBox relative(const OpesciBcStmt& s, const OpesciBcTerm& t) {
+    OpesciBcStmt one = s;
+    one.lo[0] = one.lo[1] = 0;
+    one.hi[0] = one.hi[1] = 1;
+    return read_by(one, t);
+}
 
 // The group of statements `ids` (descriptors), false when a tile cannot hold it.
 bool build_group(const OpesciContext* c, const std::vector<const OpesciBcStmt*>& src, const std::vector<BcDesc>& descs,
@@ -439,62 +493,107 @@ bool build_group(const OpesciContext* c, const std::vector<const OpesciBcStmt*>&
 }
 
 void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& src, const std::vector<int>& order,
-                     const std::vector<int>& cuts, const std::vector<BcDesc>& descs,
+                     const std::vector<int>& cuts, const std::vector<BcDesc>& descs, const std::vector<BcCells>& cells,
                      std::vector<BcPieceAny>& out_pieces, std::vector<BcBlock>& blocks, std::vector<BcRun>& out) {
     const Geom& g = c->g;
     const int n[3] = {g.nx, g.ny, g.nz};
     auto terms = [&](const OpesciBcStmt& s) { return c->h_terms.data() + s.term0; };
-    auto conflict = [&](const OpesciBcStmt& a, const OpesciBcStmt& b) {
-        const CellBox wa = written_by(a), wb = written_by(b);
-        if (wa.meets(wb)) return true;
-        for (int k = 0; k < b.nterms; ++k)
-            if (wa.meets(read_by(b, terms(b)[k]))) return true;
-        for (int k = 0; k < a.nterms; ++k)
-            if (wb.meets(read_by(a, terms(a)[k]))) return true;
+    auto meets = [](const CellBox& w, const std::vector<CellBox>& boxes) {
+        for (const CellBox& b : boxes)
+            if (w.meets(b)) return true;
         return false;
     };
+    auto conflict = [&](const BcCells& a, const BcCells& b) {
+        return a.w.meets(b.w) || meets(a.w, b.r) || meets(b.w, a.r);
+    };
     // groups, in the place of their first statement
-    std::vector<std::vector<int>> units;
+    std::vector<BcUnit> units;
+    units.reserve(order.size());
     std::vector<int> unit_of(order.size());
     for (int at = 0; at < (int)order.size(); ++at) {
         const OpesciBcStmt& s = *src[order[at]];
         int with = -1;
         for (int b = at - 1; b >= 0 && with < 0 && s.sched > 0; --b) {
             const OpesciBcStmt& a = *src[order[b]];
-            if (a.axis != s.axis || a.sched != s.sched - 1 || units[unit_of[b]][0] != order[b]) continue;
+            if (a.axis != s.axis || a.sched != s.sched - 1 || units[unit_of[b]].stmts[0] != order[b]) continue;
             for (int k = 0; k < s.nterms; ++k) {
                 const OpesciBcTerm& t = terms(s)[k];
                 if (t.field == a.field && t.level == a.level && t.plane == a.plane) with = b;
             }
         }
+        BcGroupDesc group;
         if (with >= 0) {
-            const OpesciBcStmt& a = *src[order[with]];
-            std::vector<int> ids = units[unit_of[with]];
+            const BcCells& a = cells[order[with]];
+            std::vector<int> ids = units[unit_of[with]].stmts;
             ids.push_back(order[at]);
-            BcGroupDesc d;
-            bool ok = (int)ids.size() <= BC_GROUP && build_group(c, src, descs, ids, d);
+            bool ok = (int)ids.size() <= BC_GROUP && build_group(c, src, descs, ids, group);
             for (int b = with + 1; b <= at && ok; ++b) {
-                const OpesciBcStmt& x = *src[order[b]];
-                const CellBox w = written_by(x);
-                ok = !w.meets(written_by(a)) && (b == at || unit_of[b] == unit_of[with] || !conflict(x, s));
-                for (int k = 0; k < a.nterms && ok; ++k) ok = !w.meets(read_by(a, terms(a)[k]));
+                const BcCells& x = cells[order[b]];
+                ok = !x.w.meets(a.w) && !meets(x.w, a.r) &&
+                     (b == at || unit_of[b] == unit_of[with] || !conflict(x, cells[order[at]]));
             }
             if (!ok) with = -1;
         }
         if (with >= 0) {
             unit_of[at] = unit_of[with];
-            units[unit_of[at]].push_back(order[at]);
+            units[unit_of[at]].stmts.push_back(order[at]);
+            units[unit_of[at]].group = group;
         } else {
             unit_of[at] = (int)units.size();
-            units.push_back({order[at]});
+            units.emplace_back();
+            units.back().stmts.push_back(order[at]);
         }
     }
     std::vector<BcPiece> pieces;
-    // pieces by what they write, and reads by what they read (piece, box)
-    std::vector<std::pair<int, CellBox>> writes[2 * NF], reads[2 * NF];
-    for (const std::vector<int>& u : units) {
+    // what the pieces of earlier units write and read, by field and level
+    std::vector<BcAccess> writes[2 * NF], reads[2 * NF];
+    std::vector<BcAccess> unit_writes, unit_reads, near_writes, near_reads;
+    std::vector<CellBox> w, r, own[BC_GROUP], plain[BC_GROUP];
+    for (int ui = 0; ui < (int)units.size(); ++ui) {
+        const std::vector<int>& u = units[ui].stmts;
         const OpesciBcStmt& s = *src[u[0]];
         const int o[2] = {s.axis == 0 ? 1 : 0, s.axis == 2 ? 1 : 2};
+        // the reads of the first statement's cells, of the others: computed in
+        // place where it has a value there, which reads what it reads
+        for (size_t q = 1; q < u.size(); ++q) {
+            own[q].clear();
+            plain[q].clear();
+            for (int k = 0; k < src[u[q]]->nterms; ++k) {
+                const OpesciBcTerm& t = terms(*src[u[q]])[k];
+                const bool in_place = t.field == s.field && t.level == s.level && t.plane == s.plane;
+                add_box(in_place ? own[q] : plain[q], relative(*src[u[q]], t));
+            }
+        }
+        const CellBox& whole = cells[u[0]].w;
+        // the cells its part within a rectangle writes (w) and reads (r)
+        auto collect = [&](const int lo[2], const int hi[2]) {
+            w.clear();
+            r.clear();
+            for (size_t q = 0; q < u.size(); ++q) {
+                CellBox part = cells[u[q]].w;
+                for (int d = 0; d < 2; ++d) {
+                    part.lo[o[d]] = std::max(part.lo[o[d]], lo[d]);
+                    part.hi[o[d]] = std::min(part.hi[o[d]], hi[d]);
+                }
+                if (part.lo[o[0]] >= part.hi[o[0]] || part.lo[o[1]] >= part.hi[o[1]]) continue;
+                w.push_back(part);
+                for (const CellBox& rel : q == 0 ? cells[u[0]].rel : plain[q]) add_box(r, reads_of(part, rel, s.axis));
+                if (q == 0) continue;
+                for (const CellBox& rel : own[q]) {
+                    const CellBox b = reads_of(part, rel, s.axis);
+                    CellBox a = b;
+                    bool out_of_box = false;
+                    for (int d = 0; d < 2; ++d) {
+                        a.lo[o[d]] = std::max(whole.lo[o[d]], b.lo[o[d]]);
+                        a.hi[o[d]] = std::min(whole.hi[o[d]], b.hi[o[d]]);
+                        out_of_box |= a.lo[o[d]] != b.lo[o[d]] || a.hi[o[d]] != b.hi[o[d]];
+                    }
+                    if (out_of_box) add_box(r, b);
+                    if (a.lo[o[0]] < a.hi[o[0]] && a.lo[o[1]] < a.hi[o[1]])
+                        for (const CellBox& x : cells[u[0]].rel) add_box(r, reads_of(a, x, s.axis));
+                }
+            }
+        };
         std::vector<int> cut[2];
         for (int d = 0; d < 2; ++d) {
             int lo = s.lo[d], hi = s.hi[d];
@@ -510,100 +609,104 @@ void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& s
             std::sort(cut[d].begin(), cut[d].end());
             cut[d].erase(std::unique(cut[d].begin(), cut[d].end()), cut[d].end());
         }
+        // the earlier accesses that the unit as a whole conflicts with
+        near_writes.clear();
+        near_reads.clear();
+        {
+            const int lo[2] = {cut[0].front(), cut[1].front()}, hi[2] = {cut[0].back(), cut[1].back()};
+            collect(lo, hi);
+            for (const CellBox& b : w) {
+                for (const BcAccess& q : writes[b.fl])
+                    if (q.box.meets(b)) near_writes.push_back(q);
+                for (const BcAccess& q : reads[b.fl])
+                    if (q.box.meets(b)) near_writes.push_back(q);
+            }
+            for (const CellBox& b : r)
+                for (const BcAccess& q : writes[b.fl])
+                    if (q.box.meets(b)) near_reads.push_back(q);
+        }
+        // (nothing to wait for: the rectangles along the second axis join)
+        if (near_writes.empty() && near_reads.empty()) cut[1] = {cut[1].front(), cut[1].back()};
         const size_t first = pieces.size();
+        unit_writes.clear();
+        unit_reads.clear();
+        size_t from_w = 0, from_r = 0;
         for (size_t i = 0; i + 1 < cut[0].size(); ++i)
             for (size_t j = 0; j + 1 < cut[1].size(); ++j) {
-                BcPiece p;
-                p.stmts = u;
-                p.lo[0] = cut[0][i], p.hi[0] = cut[0][i + 1];
-                p.lo[1] = cut[1][j], p.hi[1] = cut[1][j + 1];
-                for (size_t q = 0; q < u.size(); ++q) {
-                    OpesciBcStmt part = *src[u[q]];
-                    for (int d = 0; d < 2; ++d) {
-                        part.lo[d] = std::max(part.lo[d], p.lo[d]);
-                        part.hi[d] = std::min(part.hi[d], p.hi[d]);
-                    }
-                    if (part.lo[0] >= part.hi[0] || part.lo[1] >= part.hi[1]) continue;
-                    p.w.push_back(written_by(part));
-                    for (int k = 0; k < part.nterms; ++k) {
-                        const OpesciBcTerm& t = terms(part)[k];
-                        OpesciBcStmt a = s;
-                        bool out_of_box = false;
-                        for (int d = 0; d < 2; ++d) {
-                            a.lo[d] = std::max(s.lo[d], part.lo[d] + t.off[d]);
-                            a.hi[d] = std::min(s.hi[d], part.hi[d] + t.off[d]);
-                            out_of_box |= part.lo[d] + t.off[d] < s.lo[d] || part.hi[d] + t.off[d] > s.hi[d];
-                        }
-                        const bool computed = q > 0 && t.field == s.field && t.level == s.level && t.plane == s.plane;
-                        if (!computed || out_of_box) p.r.push_back(read_by(part, t));
-                        if (computed && a.lo[0] < a.hi[0] && a.lo[1] < a.hi[1])
-                            for (int x = 0; x < a.nterms; ++x) p.r.push_back(read_by(a, terms(a)[x]));
-                    }
-                }
-                for (const CellBox& w : p.w) {
-                    for (const auto& q : writes[w.fl])
-                        if (pieces[q.first].run >= p.run && q.second.meets(w)) p.run = pieces[q.first].run + 1;
-                    for (const auto& q : reads[w.fl])
-                        if (pieces[q.first].run >= p.run && q.second.meets(w)) p.run = pieces[q.first].run + 1;
-                }
-                for (const CellBox& r : p.r)
-                    for (const auto& q : writes[r.fl])
-                        if (pieces[q.first].run >= p.run && q.second.meets(r)) p.run = pieces[q.first].run + 1;
+                BcPiece p{ui, {cut[0][i], cut[1][j]}, {cut[0][i + 1], cut[1][j + 1]}, 0};
+                collect(p.lo, p.hi);
+                for (const BcAccess& q : near_writes)
+                    if (q.run >= p.run && meets(q.box, w)) p.run = q.run + 1;
+                for (const BcAccess& q : near_reads)
+                    if (q.run >= p.run && meets(q.box, r)) p.run = q.run + 1;
+                // (into the boxes of the rectangle before it where they touch)
+                const size_t nw = unit_writes.size(), nr = unit_reads.size();
+                for (const CellBox& b : w) add_box(unit_writes, from_w, p.run, b);
+                for (const CellBox& b : r) add_box(unit_reads, from_r, p.run, b);
+                if (unit_writes.size() > nw) from_w = nw;
+                if (unit_reads.size() > nr) from_r = nr;
                 // joined with the piece before it along the second axis
                 if (pieces.size() > first) {
                     BcPiece& l = pieces.back();
                     if (l.run == p.run && l.lo[0] == p.lo[0] && l.hi[0] == p.hi[0] && l.hi[1] == p.lo[1]) {
                         l.hi[1] = p.hi[1];
-                        l.w.insert(l.w.end(), p.w.begin(), p.w.end());
-                        l.r.insert(l.r.end(), p.r.begin(), p.r.end());
                         continue;
                     }
                 }
-                if (u.size() > 1) (void)build_group(c, src, descs, u, p.group);
-                pieces.push_back(std::move(p));
+                pieces.push_back(p);
             }
-        for (size_t q = first; q < pieces.size(); ++q) {
-            for (const CellBox& w : pieces[q].w) writes[w.fl].push_back({(int)q, w});
-            for (const CellBox& r : pieces[q].r) reads[r.fl].push_back({(int)q, r});
-        }
+        for (const BcAccess& q : unit_writes) writes[q.box.fl].push_back(q);
+        for (const BcAccess& q : unit_reads) reads[q.box.fl].push_back(q);
     }
     int runs = 0;
     for (const BcPiece& p : pieces) runs = std::max(runs, p.run + 1);
-    // z planes first: a line per point, the longest blocks
-    std::stable_sort(pieces.begin(), pieces.end(), [&](const BcPiece& a, const BcPiece& b) {
-        return (src[a.stmts[0]]->axis == 2) > (src[b.stmts[0]]->axis == 2);
+    // by run, z planes first: a line per point, the longest blocks
+    auto on_z = [&](const BcPiece& p) { return src[units[p.unit].stmts[0]]->axis == 2; };
+    std::vector<int> sorted(pieces.size());
+    for (size_t i = 0; i < sorted.size(); ++i) sorted[i] = (int)i;
+    std::stable_sort(sorted.begin(), sorted.end(), [&](int a, int b) {
+        const BcPiece &x = pieces[a], &y = pieces[b];
+        return x.run != y.run ? x.run < y.run : on_z(x) > on_z(y);
     });
+    out_pieces.reserve(out_pieces.size() + pieces.size());
+    auto at = sorted.begin();
     for (int run = 0; run < runs; ++run) {
+        const auto end = std::find_if(at, sorted.end(), [&](int i) { return pieces[i].run != run; });
         // points of a block, where a point costs little: as many as keep the
         // launch within one round of the chip (8 blocks on a CU), so that a
         // block fetches its descriptor for more than one round of loads
         BcRun r{(int)blocks.size(), 0, BC_BLOCK, false};
         int64_t all = 0;
-        for (const BcPiece& p : pieces)
-            if (p.run == run && p.stmts.size() == 1) all += (int64_t)(p.hi[0] - p.lo[0]) * (p.hi[1] - p.lo[1]);
+        for (auto i = at; i != end; ++i) {
+            const BcPiece& p = pieces[*i];
+            if (units[p.unit].stmts.size() == 1) all += (int64_t)(p.hi[0] - p.lo[0]) * (p.hi[1] - p.lo[1]);
+        }
         while (r.points < BC_MOST * BC_BLOCK && all > (int64_t)BC_ROUND * r.points) r.points *= 2;
-        for (const BcPiece& p : pieces) {
-            if (p.run != run) continue;
-            r.groups |= p.stmts.size() > 1;
-            BcPieceAny any;
+        for (; at != end; ++at) {
+            const BcPiece& p = pieces[*at];
+            const std::vector<int>& stmts = units[p.unit].stmts;
+            r.groups |= stmts.size() > 1;
+            const int32_t index = (int32_t)out_pieces.size();
+            out_pieces.emplace_back();
+            BcPieceAny& any = out_pieces.back();
             memset(&any, 0, sizeof(any));
             const int n0 = p.hi[0] - p.lo[0], n1 = p.hi[1] - p.lo[1];
             int nb, each = 1;
-            if (p.stmts.size() > 1) {
+            if (stmts.size() > 1) {
                 BcGroupDesc& d = any.group;
-                d = p.group;
+                d = units[p.unit].group;
                 d.lo0 = p.lo[0], d.hi0 = p.hi[0];
                 d.lo1 = p.lo[1], d.hi1 = p.hi[1];
                 const int T1 = BC_TILE1[d.axis], T0 = BC_BLOCK / T1;
                 d.tiles1 = (n1 + T1 - 1) / T1;
                 nb = (n0 + T0 - 1) / T0 * d.tiles1;
                 for (int q = 0; q < d.nstmts; ++q) {
-                    const OpesciBcStmt& s = *src[p.stmts[q]];
+                    const OpesciBcStmt& s = *src[stmts[q]];
                     d.s[q].lo0 = std::max(s.lo[0], p.lo[0]), d.s[q].hi0 = std::min(s.hi[0], p.hi[0]);
                     d.s[q].lo1 = std::max(s.lo[1], p.lo[1]), d.s[q].hi1 = std::min(s.hi[1], p.hi[1]);
                 }
             } else {
-                const BcDesc& o = descs[p.stmts[0]];
+                const BcDesc& o = descs[stmts[0]];
                 BcPieceDesc& d = any.piece;
                 d.fl = o.fl;
                 d.disp = o.disp;
@@ -622,17 +725,16 @@ void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& s
                 each = o.nterms <= 1 ? r.points : BC_BLOCK;
                 nb = (d.npts + each - 1) / each;
             }
-            for (int b = 0; b < nb; ++b)
-                blocks.push_back(BcBlock{(int32_t)out_pieces.size(), b * each});
-            out_pieces.push_back(any);
+            for (int b = 0; b < nb; ++b) blocks.push_back(BcBlock{index, b * each});
         }
         r.count = (int)blocks.size() - r.first;
         out.push_back(r);
     }
 }
 
-int build_step_launches(OpesciContext* c, const std::vector<const OpesciBcStmt*>& src,
-                        const std::vector<BcDesc>& descs) {
+void build_step_launches(OpesciContext* c, const std::vector<const OpesciBcStmt*>& src,
+                         const std::vector<BcDesc>& descs, std::vector<BcPieceAny>& pieces,
+                         std::vector<BcBlock>& blocks) {
     const Geom& g = c->g;
     const int n[3] = {g.nx, g.ny, g.nz}, m = g.m;
     bool zeros = true;                    // every velocity statement stores constant zeros
@@ -644,17 +746,25 @@ int build_step_launches(OpesciContext* c, const std::vector<const OpesciBcStmt*>
             if (a != s.axis && (w.lo[a] > m || w.hi[a] < n[a] - m)) return false;
         return s.level == 1 && zero_stays(c, s, true);
     };
-    for (const BcLevel& lv : c->levels[3])
-        for (int i = lv.first; i < lv.first + lv.count; ++i) {
-            if (on_last(*src[i]))
-                last[src[i]->axis] = true;
-            else if (!zero_stays(c, *src[i], false))
-                zeros = false;
-        }
+    std::vector<char> stays(src.size(), 0), last_plane(src.size(), 0);
+    std::vector<BcCells> cells(src.size());
+    for (int ph = 2; ph < 4; ++ph)
+        for (const BcLevel& lv : c->levels[ph])
+            for (int i = lv.first; i < lv.first + lv.count; ++i) {
+                stays[i] = zero_stays(c, *src[i], false);
+                last_plane[i] = on_last(*src[i]);
+                cells[i].w = written_by(*src[i]);
+                for (int k = 0; k < src[i]->nterms; ++k)
+                    add_box(cells[i].rel, relative(*src[i], c->h_terms[src[i]->term0 + k]));
+                for (const CellBox& rel : cells[i].rel) cells[i].r.push_back(reads_of(cells[i].w, rel, src[i]->axis));
+                c->left_out |= stays[i] != 0;
+                if (ph == 3 && last_plane[i])
+                    last[src[i]->axis] = true;
+                else if (ph == 3 && !stays[i])
+                    zeros = false;
+            }
     for (int a = 0; a < 3; ++a)
         if (zeros && last[a]) c->zero_last |= 1 << a;
-    std::vector<BcPieceAny> pieces;
-    std::vector<BcBlock> blocks;
     for (int ph = 2; ph < 4; ++ph)
         for (int sweep = 0; sweep < 2; ++sweep) {
             // sweep 1: the launches beside a velocity sweep that stores zero_last
@@ -665,16 +775,11 @@ int build_step_launches(OpesciContext* c, const std::vector<const OpesciBcStmt*>
             }
             std::vector<int> live;
             for (const BcLevel& lv : c->levels[ph])
-                for (int i = lv.first; i < lv.first + lv.count; ++i) {
-                    const bool stays = zero_stays(c, *src[i], false);
-                    c->left_out |= stays;
-                    if (!stays && !(sweep && on_last(*src[i]))) live.push_back(i);
-                }
+                for (int i = lv.first; i < lv.first + lv.count; ++i)
+                    if (!stays[i] && !(sweep && last_plane[i])) live.push_back(i);
             schedule_pieces(c, src, live, ph == 2 ? std::vector<int>{m + 1, 2 * m + 1} : std::vector<int>{2 * m}, descs,
-                            pieces, blocks, out);
+                            cells, pieces, blocks, out);
         }
-    if (int e = upload(&c->d_pieces, pieces.data(), pieces.size(), c->stream)) return e;
-    return upload(&c->d_blocks, blocks.data(), blocks.size(), c->stream);
 }
 
 int build_program(OpesciContext* c, const OpesciBcTerm* terms, const OpesciBcDTerm* dterms, int ndterms,
@@ -745,8 +850,21 @@ int build_program(OpesciContext* c, const OpesciBcTerm* terms, const OpesciBcDTe
         if (lv.count > 0) c->levels[L.phase].push_back(lv);
         i = j;
     }
-    if (int e = build_step_launches(c, src, descs)) return e;
-    if (int e = upload(&c->d_desc, descs.data(), descs.size(), c->stream)) return e;
+    // descriptors, pieces and block lists in one allocation and one transfer
+    std::vector<BcPieceAny> pieces;
+    std::vector<BcBlock> blocks;
+    build_step_launches(c, src, descs, pieces, blocks);
+    auto padded = [](size_t bytes) { return (bytes + 255) & ~size_t(255); };
+    const size_t o_pieces = padded(descs.size() * sizeof(BcDesc)),
+                 o_blocks = o_pieces + padded(pieces.size() * sizeof(BcPieceAny));
+    std::vector<char> all(o_blocks + blocks.size() * sizeof(BcBlock));
+    if (!descs.empty()) memcpy(all.data(), descs.data(), descs.size() * sizeof(BcDesc));
+    if (!pieces.empty()) memcpy(all.data() + o_pieces, pieces.data(), pieces.size() * sizeof(BcPieceAny));
+    if (!blocks.empty()) memcpy(all.data() + o_blocks, blocks.data(), blocks.size() * sizeof(BcBlock));
+    if (int e = upload(&c->d_program, all.data(), all.size(), c->stream)) return e;
+    c->d_desc = reinterpret_cast<const BcDesc*>(c->d_program);
+    c->d_pieces = reinterpret_cast<const BcPieceAny*>(c->d_program + o_pieces);
+    c->d_blocks = reinterpret_cast<const BcBlock*>(c->d_program + o_blocks);
     c->h_desc = std::move(descs);
     return 0;
 }
@@ -824,11 +942,15 @@ int build_solution(OpesciContext* c, const OpesciModelDesc* d) {
     }
     for (SolSlot& s : slots) s.prog += (int32_t)pc.size();
     pc.insert(pc.end(), tc.begin(), tc.end());
-    if (int e = upload(&c->d_sol, pc.data(), pc.size(), c->stream)) return e;
-    if (int e = upload(&c->d_solslots, slots.data(), slots.size(), c->stream)) return e;
+    static_assert(alignof(SolSlot) <= alignof(OpesciExprOp) && sizeof(OpesciExprOp) % alignof(SolSlot) == 0,
+                  "slots follow the programs");
+    std::vector<char> all(pc.size() * sizeof(OpesciExprOp) + slots.size() * sizeof(SolSlot));
+    if (!pc.empty()) memcpy(all.data(), pc.data(), pc.size() * sizeof(OpesciExprOp));
+    if (!slots.empty()) memcpy(all.data() + pc.size() * sizeof(OpesciExprOp), slots.data(), slots.size() * sizeof(SolSlot));
+    if (int e = upload(&c->d_sol, all.data(), all.size(), c->stream)) return e;
     if (ntab > 0) OPESCI_HIP_TRY(hipMalloc((void**)&c->d_soltab, (size_t)ntab * sizeof(double)));
-    c->sol.code = c->d_sol;
-    c->sol.slots = c->d_solslots;
+    c->sol.code = reinterpret_cast<const OpesciExprOp*>(c->d_sol);
+    c->sol.slots = reinterpret_cast<const SolSlot*>(c->sol.code + pc.size());
     c->sol.nslots = (int)slots.size();
     c->sol.maxdim = std::max(dims[0], std::max(dims[1], dims[2]));
     c->sol.tab = c->d_soltab;
@@ -848,7 +970,7 @@ int alloc_zero(OpesciContext* c, void** p, size_t bytes) {
 // (constant media) or, but for the last, all pool slots in term order (read
 // path).  Anything else leaves zf.F = 0 and the statements run as their own
 // launch.
-int build_zfaces(OpesciContext* c) {
+int build_zfaces(OpesciContext* c, ZCoef& zc) {
     c->zf = ZFaceArgs();
     const Geom& g = c->g;
     const int M = g.m;
@@ -858,7 +980,6 @@ int build_zfaces(OpesciContext* c) {
     if (!(c->desc.flags & OPESCI_FLAG_ZFACES_IN_SWEEP) && (c->real_bytes != 4 || c->het || (bhi - M) % 128 < M))
         return 0;
     ZFaceArgs z;
-    ZCoef zc;
     memset(&zc, 0, sizeof(zc));
     bool zero[2] = {false, false}, img[2][3][MAXM] = {}, rec[2][2] = {};
     int F = -1;
@@ -942,8 +1063,6 @@ int build_zfaces(OpesciContext* c) {
     z.F = F;
     z.n1 = g.ny - 2 * F;
     z.npts = (g.nx - 2 * F) * z.n1;
-    if (int e = upload(&c->d_zcoef, &zc, 1, c->stream)) return e;
-    z.coef = c->d_zcoef;
     c->zf = z;
     return 0;
 }
@@ -960,7 +1079,7 @@ bool zfaces_in_sweep(const OpesciContext* c) {
 // written before it).  The box rows are then deep z-face rows at every halo
 // plane and row (F - M >= the z faces' F), and the x and y stencils of the
 // sweep stay inside the grid (F >= 2M).
-int build_fused(OpesciContext* c) {
+int build_fused(OpesciContext* c, const ZCoef& zc) {
     c->fused_F = 0;
     c->fbox = Boxes();
     c->frame = Boxes();
@@ -1025,6 +1144,8 @@ int build_fused(OpesciContext* c) {
             f.y0[i] = Y0[i];
             f.y1[i] = Y1[i];
         }
+        if (int e = upload(&c->d_zcoef, &zc, 1, c->stream)) return e;
+        c->zf.coef = c->d_zcoef;
         return 0;
     }
     return 0;
@@ -1126,7 +1247,7 @@ void destroy(OpesciContext* c) {
             if (c->base[f][l]) (void)hipFree(c->base[f][l]);
     for (int i = 0; i < OPESCI_M_COUNT; ++i)
         if (c->mbase[i]) (void)hipFree(c->mbase[i]);
-    void* ptrs[] = {c->d_pieces, c->d_blocks, c->d_desc,  c->d_code,    c->d_sol,  c->d_solslots, c->d_soltab, c->d_partial, c->d_stage, c->d_rec, c->d_at_src,
+    void* ptrs[] = {c->d_program, c->d_code,    c->d_sol, c->d_soltab, c->d_partial, c->d_stage, c->d_rec, c->d_at_src,
                     c->d_trace, c->d_wavelet, c->d_step, c->d_pool,    c->d_dterms, c->d_gpool,
                     c->d_log,   c->d_ckpt,    c->d_seg,  c->d_obs,     c->d_srclog, c->d_tcells,
                     c->d_vcells, c->d_scells, c->d_zcoef, c->d_zpool, c->d_gather, c->d_abuf};
@@ -1190,18 +1311,20 @@ int create(const OpesciModelDesc* d, OpesciContext** out) {
     c->field_bytes = (size_t)g.total * c->elem;
     for (int f = 0; f < NF; ++f)
         for (int l = 0; l < 2; ++l) {
-            if (int e = alloc_zero(c.get(), &c->base[f][l], c->field_bytes)) return e;
+            OPESCI_HIP_TRY(hipMalloc(&c->base[f][l], c->field_bytes));
             c->fptr[f][l] = (char*)c->base[f][l] + (size_t)g.zoff * c->elem;
         }
+    OPESCI_HIP_TRY(launch_zero_all(&c->base[0][0], 2 * NF, c->field_bytes, c->stream));
     const size_t rb = d->real_bytes;
     const size_t dense = (size_t)g.nx * g.ny * g.nz;
     OPESCI_HIP_TRY(hipMalloc(&c->d_stage, dense * std::max(rb, sizeof(float) * 3)));
     if (c->het) {
         const size_t mbytes = (size_t)g.total * rb;
         for (int i = 0; i < OPESCI_M_COUNT; ++i) {
-            if (int e = alloc_zero(c.get(), &c->mbase[i], mbytes)) return e;
+            OPESCI_HIP_TRY(hipMalloc(&c->mbase[i], mbytes));
             c->mptr[i] = (char*)c->mbase[i] + (size_t)g.zoff * rb;
         }
+        OPESCI_HIP_TRY(launch_zero_all(c->mbase, OPESCI_M_COUNT, mbytes, c->stream));
         float* st = (float*)c->d_stage;
         OPESCI_HIP_TRY(hipMemcpyAsync(st, d->rho, dense * 4, hipMemcpyHostToDevice, c->stream));
         OPESCI_HIP_TRY(hipMemcpyAsync(st + dense, d->vp, dense * 4, hipMemcpyHostToDevice, c->stream));
@@ -1225,8 +1348,9 @@ int create(const OpesciModelDesc* d, OpesciContext** out) {
     c->stmts.assign(d->stmts, d->stmts + d->nstmts);
     c->h_terms.assign(d->terms, d->terms + d->nterms);
     if (int e = build_program(c.get(), d->terms, d->dterms, d->ndterms, d->nterms)) return e;
-    if (int e = build_zfaces(c.get())) return e;
-    if (int e = build_fused(c.get())) return e;
+    ZCoef zc = {};
+    if (int e = build_zfaces(c.get(), zc)) return e;
+    if (int e = build_fused(c.get(), zc)) return e;
     if (int e = upload(&c->d_dterms, d->dterms, (size_t)d->ndterms, c->stream)) return e;
     c->h_dterms.assign(d->dterms, d->dterms + d->ndterms);
     if (int e = upload(&c->d_code, d->bc_code, (size_t)d->ncode, c->stream)) return e;

@@ -275,7 +275,7 @@ constexpr int ZPOOL_ITEMS = 512;   // of a tile's plane at most (16 rows, both f
 // `boxes` (x0..y1 and n set) restricts the update to those rows (sweeps only)
 hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                          const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
-                         const ZFaceArgs* zf = nullptr, const void* pool = nullptr, const Boxes* boxes = nullptr);
+                         const ZFaceArgs* zf = nullptr, const Boxes* boxes = nullptr);
 // the flat-tile stress sweep (stress.hip)
 hipError_t launch_stress_sweep(const Geom& g, int real_bytes, int storage, bool het, const void* fields,
                                const void* media, const void* coefs, int t0, int t1, const InteriorLaunch& cfg,

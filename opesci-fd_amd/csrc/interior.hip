@@ -205,10 +205,10 @@ __device__ __forceinline__ float lane_read(float v, int lane) {
 // A block owns a 128 (z) x TY (y) tile of an x chunk [xb, xe).  Its waves
 // hold rows y0 - M .. y0 + TY + M - 1: TY own rows between M halo rows on
 // either side.  At step xs of the sweep (xs = xb - M .. xe + M - 1) every
-// wave computes the stresses of its row at plane xs exactly as the pair
-// stress sweep does (velocity plane xs staged in LDS with 2M halo rows and
-// 2M z columns either side, x stencils in register queues), lanes 0 and 63
-// of the own waves add the z-halo pairs below and above the tile (Txz, Tyz,
+// wave computes the stresses of its row at plane xs exactly as the stress
+// sweep does, two z points per lane (velocity plane xs staged in LDS with 2M
+// halo rows and 2M z columns either side, x stencils in register queues),
+// lanes 0 and 63 of the own waves add the z-halo pairs below and above the tile (Txz, Tyz,
 // Tzz) where a neighbouring tile, not a face, lies there, and the z-face
 // statements replace the surface values and produce the ghost cells.  The
 // stresses go to an LDS plane (rounded to the storage type, as the separate
@@ -933,8 +933,7 @@ bool stress_applies_zfaces(const InteriorLaunch& cfg) {
 
 hipError_t launch_stress(const Geom& g, int real_bytes, int storage, bool het, void* fields, const void* media,
                          const void* coefs, int t0, int t1, const InteriorLaunch& cfg, hipStream_t s,
-                         const ZFaceArgs* zf, const void* pool, const Boxes* boxes) {
-    (void)pool;
+                         const ZFaceArgs* zf, const Boxes* boxes) {
     if (zf && zf->F > 0 && !stress_applies_zfaces(cfg)) return hipErrorInvalidValue;
     if (cfg.variant != 1)
         return launch_stress_sweep(g, real_bytes, storage, het, fields, media, coefs, t0, t1, cfg, s, zf, boxes);

@@ -1194,7 +1194,7 @@ int step_once(OpesciContext* c, int t0) {
     if (fused_step(c)) {
         OPESCI_HIP_TRY(launch_step_fused(c->g, c->storage, c->fptr, c->coefs(), t0, t1, c->zf, c->fbox, 0, c->stream));
         OPESCI_HIP_TRY(launch_stress(c->g, c->real_bytes, c->storage, c->het, c->fptr, c->mptr, c->coefs(), t0, t1,
-                                     c->cfg, c->stream, &c->zf, c->d_pool, &c->frame));
+                                     c->cfg, c->stream, &c->zf, &c->frame));
         if (int e = step_bc(c, 2, t0, t1)) return e;
         OPESCI_HIP_TRY(launch_velocity(c->g, c->real_bytes, c->storage, c->het, c->fptr, c->mptr, c->coefs(), t0, t1,
                                        c->cfg, c->stream, &c->frame));
@@ -1205,7 +1205,7 @@ int step_once(OpesciContext* c, int t0) {
     }
     const bool zin = zfaces_in_sweep(c);
     OPESCI_HIP_TRY(launch_stress(c->g, c->real_bytes, c->storage, c->het, c->fptr, c->mptr, c->coefs(), t0, t1,
-                                 c->cfg, c->stream, zin ? &c->zf : nullptr, c->d_pool));
+                                 c->cfg, c->stream, zin ? &c->zf : nullptr));
     if (!zin)
         if (int e = run_bc_phase(c, 4, t0, t1)) return e;
     if (int e = step_bc(c, 2, t0, t1)) return e;
@@ -1695,7 +1695,7 @@ int opesci_ctx_kernel_times(OpesciContext* ctx, int32_t nsteps, double out_ms[3]
                                              ctx->stream));
             OPESCI_HIP_TRY(hipEventRecord(e[1], ctx->stream));
             OPESCI_HIP_TRY(launch_stress(ctx->g, ctx->real_bytes, ctx->storage, ctx->het, ctx->fptr, ctx->mptr,
-                                         ctx->coefs(), t0, t1, ctx->cfg, ctx->stream, &ctx->zf, ctx->d_pool, &ctx->frame));
+                                         ctx->coefs(), t0, t1, ctx->cfg, ctx->stream, &ctx->zf, &ctx->frame));
             OPESCI_HIP_TRY(hipEventRecord(e[2], ctx->stream));
             rc = step_bc(ctx, 2, t0, t1);
             OPESCI_HIP_TRY(hipEventRecord(e[3], ctx->stream));
@@ -1704,7 +1704,7 @@ int opesci_ctx_kernel_times(OpesciContext* ctx, int32_t nsteps, double out_ms[3]
             OPESCI_HIP_TRY(hipEventRecord(e[4], ctx->stream));
             if (!rc) rc = step_bc(ctx, 3, t0, t1);
             if (!rc && (ctx->nrec > 0 || ctx->src_ntr))
-                rc = rc ? rc : record_source(ctx, ctx->fptr, t1, ctx->nrec);
+                rc = record_source(ctx, ctx->fptr, t1, ctx->nrec);
             OPESCI_HIP_TRY(hipEventRecord(e[5], ctx->stream));
             ++ctx->steps;
             if (ctx->full_steps > 0) --ctx->full_steps;
@@ -1715,8 +1715,7 @@ int opesci_ctx_kernel_times(OpesciContext* ctx, int32_t nsteps, double out_ms[3]
             OPESCI_HIP_TRY(hipEventRecord(e[0], ctx->stream));
             const bool zin = zfaces_in_sweep(ctx);
             OPESCI_HIP_TRY(launch_stress(ctx->g, ctx->real_bytes, ctx->storage, ctx->het, ctx->fptr, ctx->mptr,
-                                         ctx->coefs(), t0, t1, ctx->cfg, ctx->stream, zin ? &ctx->zf : nullptr,
-                                         ctx->d_pool));
+                                         ctx->coefs(), t0, t1, ctx->cfg, ctx->stream, zin ? &ctx->zf : nullptr));
             OPESCI_HIP_TRY(hipEventRecord(e[1], ctx->stream));
             if (!zin) rc = run_bc_phase(ctx, 4, t0, t1);
             if (!rc) rc = step_bc(ctx, 2, t0, t1);
@@ -1727,7 +1726,7 @@ int opesci_ctx_kernel_times(OpesciContext* ctx, int32_t nsteps, double out_ms[3]
             OPESCI_HIP_TRY(hipEventRecord(e[3], ctx->stream));
             if (!rc) rc = step_bc(ctx, 3, t0, t1);
             if (!rc && (ctx->nrec > 0 || ctx->src_ntr))
-                rc = rc ? rc : record_source(ctx, ctx->fptr, t1, ctx->nrec);
+                rc = record_source(ctx, ctx->fptr, t1, ctx->nrec);
             OPESCI_HIP_TRY(hipEventRecord(e[4], ctx->stream));
             ++ctx->steps;
             if (ctx->full_steps > 0) --ctx->full_steps;

@@ -48,7 +48,7 @@ def main():
     ap.add_argument('--storage', default='native')
     ap.add_argument('--no-cpu', action='store_true')
     ap.add_argument('--cpu-steps', type=int, default=100)
-    ap.add_argument('--variant', type=int, default=None, help='interior kernel variant (0 and 2 sweep, 1 gather)')
+    ap.add_argument('--variant', type=int, default=None, help='interior kernel variant (0 sweep, 1 gather, 2 sweep without the z faces)')
     ap.add_argument('--x-chunk', type=int, default=0)
     ap.add_argument('--tile-y', type=int, default=0)
     ap.add_argument('--copy-probe', type=int, default=0, help='MiB copied device-to-device 3x first')
@@ -100,10 +100,10 @@ def main():
         kt = ctx.kernel_times(10)   # per-launch averages, after the timed region
         bc_stats = ctx.stats(full=True)
         fused_F = ctx.fused_margin()
-    # the traffic record of the stress launch that ran: the pair sweep with
-    # or without the deep z-face statements
-    workload_key = 'stress_sweep %d^3 order %d %s%s%s' % (N, order, args.storage, ' hetero' if args.hetero else '',
-                                                         ' z-faces in sweep' if bc_stats[3] else '')
+    # the traffic record of the launch that ran: the stress sweep with or
+    # without the deep z-face statements (none for the fused step or the gather)
+    workload_key = workload(N, order, args.storage, args.hetero, bool(bc_stats[3]), plan.kernel_variant == 1,
+                            fused_F > 0)
     # flops per point-step: ADD + MUL of the stress and velocity kernels in the
     # reference's own operation count (get_*_kernel_ai)
     flops_pt = sum(ai[2] + ai[3] for ai in (g.get_stress_kernel_ai(), g.get_velocity_kernel_ai()))
@@ -188,16 +188,27 @@ def copy_probe(hip, nbytes):
     hip.hipFree(b)
 
 
-def committed_traffic(key):
-    """HBM bytes per launch from a committed PMC summary, or None."""
+def workload(N, order, storage, hetero, zfaces, gather=False, fused=False):
+    kernel = 'fused_step' if fused else 'stress_gather' if gather else 'stress_sweep'
+    return '%s %d^3 order %d %s%s%s' % (kernel, N, order, storage, ' hetero' if hetero else '',
+                                        ' z-faces in sweep' if zfaces else '')
+
+
+def traffic_records():
+    """The traffic lines of the committed PMC summaries."""
     import glob
+    out = []
     for path in sorted(glob.glob(os.path.join(PROFILES, '*_pmc.md'))):
         with open(path) as f:
-            for line in f:
-                if line.startswith('traffic:'):
-                    rec = json.loads(line[len('traffic:'):])
-                    if rec.get('workload') == key:
-                        return float(rec['bytes_per_launch'])
+            out += [json.loads(line[len('traffic:'):]) for line in f if line.startswith('traffic:')]
+    return out
+
+
+def committed_traffic(key):
+    """HBM bytes per launch from a committed PMC summary, or None."""
+    for rec in traffic_records():
+        if rec.get('workload') == key:
+            return float(rec['bytes_per_launch'])
     return None
 
 

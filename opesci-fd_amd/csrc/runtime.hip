@@ -97,7 +97,7 @@ struct OpesciContext {
     int partial_cap = 0;
     void* d_stage = nullptr;          // dense staging buffer (one field level, real_t)
     int32_t* d_rec = nullptr;
-    int32_t* d_at_src = nullptr;      // the receivers in the source's cell
+    const int32_t* d_at_src = nullptr;   // the receivers in the source's cell (behind d_rec's points)
     int nat_src = 0;
     void* d_trace = nullptr;          // [ntsteps][nrec][4] of the arithmetic type
     float* d_wavelet = nullptr;
@@ -372,9 +372,10 @@ bool zero_stays(const OpesciContext* c, const OpesciBcStmt& s, bool last_plane) 
 // pieces, of which all but the first of a phase hold edges only.
 constexpr int BC_ROUND = 8 * 256;      // blocks that fit the chip
 constexpr int BC_MOST = 8;
+constexpr int BC_CUTS = 2;             // distances from an end at which a rectangle is cut, at most
 struct BcUnit {
-    std::vector<int> stmts;            // descriptors, the group's first one first
-    BcGroupDesc group;                 // of several statements, but for the rectangle
+    int n, stmts[BC_GROUP];            // descriptors, the group's first one first
+    int group;                         // of several statements: its descriptor but for the rectangle
 };
 struct BcPiece {
     int unit;
@@ -438,14 +439,14 @@ CellBox relative(const OpesciBcStmt& s, const OpesciBcTerm& t) {
 
 // The group of statements `ids` (descriptors), false when a tile cannot hold it.
 bool build_group(const OpesciContext* c, const std::vector<const OpesciBcStmt*>& src, const std::vector<BcDesc>& descs,
-                 const std::vector<int>& ids, BcGroupDesc& out) {
+                 const BcUnit& ids, BcGroupDesc& out) {
     memset(&out, 0, sizeof(out));
-    const OpesciBcStmt& a = *src[ids[0]];
+    const OpesciBcStmt& a = *src[ids.stmts[0]];
     const int W = BC_TILE1[a.axis] + 2;
     const int64_t stride[3] = {c->g.sx, c->g.sy, 1};
     out.group = 1 + a.axis;
     out.axis = a.axis;
-    out.nstmts = (int)ids.size();
+    out.nstmts = ids.n;
     auto slot = [&](int fl, int plane) {
         const int32_t disp = (int32_t)(plane * stride[a.axis]);
         for (int k = 0; k < out.nslots; ++k)
@@ -458,9 +459,9 @@ bool build_group(const OpesciContext* c, const std::vector<const OpesciBcStmt*>&
     out.own_slot = slot(a.field * 2 + a.level, a.plane);
     int32_t* lo[2] = {&out.min0, &out.min1};
     int32_t* hi[2] = {&out.max0, &out.max1};
-    for (int q = (int)ids.size() - 1; q >= 0; --q) {
-        const OpesciBcStmt& s = *src[ids[q]];
-        const BcDesc& d = descs[ids[q]];
+    for (int q = ids.n - 1; q >= 0; --q) {
+        const OpesciBcStmt& s = *src[ids.stmts[q]];
+        const BcDesc& d = descs[ids.stmts[q]];
         if (s.nterms > BC_GTERMS) return false;
         BcGroupStmt& o = out.s[q];
         o.fl = d.fl;
@@ -493,7 +494,7 @@ bool build_group(const OpesciContext* c, const std::vector<const OpesciBcStmt*>&
 }
 
 void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& src, const std::vector<int>& order,
-                     const std::vector<int>& cuts, const std::vector<BcDesc>& descs, const std::vector<BcCells>& cells,
+                     const int* cuts, int ncuts, const std::vector<BcDesc>& descs, const std::vector<BcCells>& cells,
                      std::vector<BcPieceAny>& out_pieces, std::vector<BcBlock>& blocks, std::vector<BcRun>& out) {
     const Geom& g = c->g;
     const int n[3] = {g.nx, g.ny, g.nz};
@@ -508,6 +509,7 @@ void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& s
     };
     // groups, in the place of their first statement
     std::vector<BcUnit> units;
+    std::vector<BcGroupDesc> groups;
     units.reserve(order.size());
     std::vector<int> unit_of(order.size());
     for (int at = 0; at < (int)order.size(); ++at) {
@@ -522,11 +524,15 @@ void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& s
             }
         }
         BcGroupDesc group;
+        BcUnit grown;
         if (with >= 0) {
             const BcCells& a = cells[order[with]];
-            std::vector<int> ids = units[unit_of[with]].stmts;
-            ids.push_back(order[at]);
-            bool ok = (int)ids.size() <= BC_GROUP && build_group(c, src, descs, ids, group);
+            grown = units[unit_of[with]];
+            bool ok = grown.n < BC_GROUP;
+            if (ok) {
+                grown.stmts[grown.n++] = order[at];
+                ok = build_group(c, src, descs, grown, group);
+            }
             for (int b = with + 1; b <= at && ok; ++b) {
                 const BcCells& x = cells[order[b]];
                 ok = !x.w.meets(a.w) && !meets(x.w, a.r) &&
@@ -536,12 +542,15 @@ void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& s
         }
         if (with >= 0) {
             unit_of[at] = unit_of[with];
-            units[unit_of[at]].stmts.push_back(order[at]);
-            units[unit_of[at]].group = group;
+            if (grown.group < 0) {
+                grown.group = (int)groups.size();
+                groups.emplace_back();
+            }
+            groups[grown.group] = group;
+            units[unit_of[at]] = grown;
         } else {
             unit_of[at] = (int)units.size();
-            units.emplace_back();
-            units.back().stmts.push_back(order[at]);
+            units.push_back(BcUnit{1, {order[at]}, -1});
         }
     }
     std::vector<BcPiece> pieces;
@@ -550,12 +559,13 @@ void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& s
     std::vector<BcAccess> unit_writes, unit_reads, near_writes, near_reads;
     std::vector<CellBox> w, r, own[BC_GROUP], plain[BC_GROUP];
     for (int ui = 0; ui < (int)units.size(); ++ui) {
-        const std::vector<int>& u = units[ui].stmts;
+        const int* const u = units[ui].stmts;
+        const int nu = units[ui].n;
         const OpesciBcStmt& s = *src[u[0]];
         const int o[2] = {s.axis == 0 ? 1 : 0, s.axis == 2 ? 1 : 2};
         // the reads of the first statement's cells, of the others: computed in
         // place where it has a value there, which reads what it reads
-        for (size_t q = 1; q < u.size(); ++q) {
+        for (int q = 1; q < nu; ++q) {
             own[q].clear();
             plain[q].clear();
             for (int k = 0; k < src[u[q]]->nterms; ++k) {
@@ -569,7 +579,7 @@ void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& s
         auto collect = [&](const int lo[2], const int hi[2]) {
             w.clear();
             r.clear();
-            for (size_t q = 0; q < u.size(); ++q) {
+            for (int q = 0; q < nu; ++q) {
                 CellBox part = cells[u[q]].w;
                 for (int d = 0; d < 2; ++d) {
                     part.lo[o[d]] = std::max(part.lo[o[d]], lo[d]);
@@ -594,26 +604,31 @@ void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& s
                 }
             }
         };
-        std::vector<int> cut[2];
+        struct Cuts {
+            int v[2 + 2 * BC_CUTS], n;
+            int back() const { return v[n - 1]; }
+        } cut[2];
         for (int d = 0; d < 2; ++d) {
             int lo = s.lo[d], hi = s.hi[d];
-            for (int id : u) {
-                lo = std::min(lo, src[id]->lo[d]);
-                hi = std::max(hi, src[id]->hi[d]);
+            for (int q = 1; q < nu; ++q) {
+                lo = std::min(lo, src[u[q]]->lo[d]);
+                hi = std::max(hi, src[u[q]]->hi[d]);
             }
-            cut[d] = {lo, hi};
-            if (s.sched > 0)
-                for (int f : cuts)
-                    for (int v : {f, n[o[d]] - f})
-                        if (v > lo && v < hi) cut[d].push_back(v);
-            std::sort(cut[d].begin(), cut[d].end());
-            cut[d].erase(std::unique(cut[d].begin(), cut[d].end()), cut[d].end());
+            Cuts& k = cut[d];
+            k.v[0] = lo;
+            k.v[1] = hi;
+            k.n = 2;
+            for (int i = 0; i < ncuts && s.sched > 0; ++i)
+                for (int v : {cuts[i], n[o[d]] - cuts[i]})
+                    if (v > lo && v < hi) k.v[k.n++] = v;
+            std::sort(k.v, k.v + k.n);
+            k.n = (int)(std::unique(k.v, k.v + k.n) - k.v);
         }
         // the earlier accesses that the unit as a whole conflicts with
         near_writes.clear();
         near_reads.clear();
         {
-            const int lo[2] = {cut[0].front(), cut[1].front()}, hi[2] = {cut[0].back(), cut[1].back()};
+            const int lo[2] = {cut[0].v[0], cut[1].v[0]}, hi[2] = {cut[0].back(), cut[1].back()};
             collect(lo, hi);
             for (const CellBox& b : w) {
                 for (const BcAccess& q : writes[b.fl])
@@ -626,14 +641,14 @@ void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& s
                     if (q.box.meets(b)) near_reads.push_back(q);
         }
         // (nothing to wait for: the rectangles along the second axis join)
-        if (near_writes.empty() && near_reads.empty()) cut[1] = {cut[1].front(), cut[1].back()};
+        if (near_writes.empty() && near_reads.empty()) cut[1] = Cuts{{cut[1].v[0], cut[1].back()}, 2};
         const size_t first = pieces.size();
         unit_writes.clear();
         unit_reads.clear();
         size_t from_w = 0, from_r = 0;
-        for (size_t i = 0; i + 1 < cut[0].size(); ++i)
-            for (size_t j = 0; j + 1 < cut[1].size(); ++j) {
-                BcPiece p{ui, {cut[0][i], cut[1][j]}, {cut[0][i + 1], cut[1][j + 1]}, 0};
+        for (int i = 0; i + 1 < cut[0].n; ++i)
+            for (int j = 0; j + 1 < cut[1].n; ++j) {
+                BcPiece p{ui, {cut[0].v[i], cut[1].v[j]}, {cut[0].v[i + 1], cut[1].v[j + 1]}, 0};
                 collect(p.lo, p.hi);
                 for (const BcAccess& q : near_writes)
                     if (q.run >= p.run && meets(q.box, w)) p.run = q.run + 1;
@@ -679,22 +694,23 @@ void schedule_pieces(OpesciContext* c, const std::vector<const OpesciBcStmt*>& s
         int64_t all = 0;
         for (auto i = at; i != end; ++i) {
             const BcPiece& p = pieces[*i];
-            if (units[p.unit].stmts.size() == 1) all += (int64_t)(p.hi[0] - p.lo[0]) * (p.hi[1] - p.lo[1]);
+            if (units[p.unit].n == 1) all += (int64_t)(p.hi[0] - p.lo[0]) * (p.hi[1] - p.lo[1]);
         }
         while (r.points < BC_MOST * BC_BLOCK && all > (int64_t)BC_ROUND * r.points) r.points *= 2;
         for (; at != end; ++at) {
             const BcPiece& p = pieces[*at];
-            const std::vector<int>& stmts = units[p.unit].stmts;
-            r.groups |= stmts.size() > 1;
+            const int* const stmts = units[p.unit].stmts;
+            const bool group = units[p.unit].n > 1;
+            r.groups |= group;
             const int32_t index = (int32_t)out_pieces.size();
             out_pieces.emplace_back();
             BcPieceAny& any = out_pieces.back();
             memset(&any, 0, sizeof(any));
             const int n0 = p.hi[0] - p.lo[0], n1 = p.hi[1] - p.lo[1];
             int nb, each = 1;
-            if (stmts.size() > 1) {
+            if (group) {
                 BcGroupDesc& d = any.group;
-                d = units[p.unit].group;
+                d = groups[units[p.unit].group];
                 d.lo0 = p.lo[0], d.hi0 = p.hi[0];
                 d.lo1 = p.lo[1], d.hi1 = p.hi[1];
                 const int T1 = BC_TILE1[d.axis], T0 = BC_BLOCK / T1;
@@ -777,8 +793,9 @@ void build_step_launches(OpesciContext* c, const std::vector<const OpesciBcStmt*
             for (const BcLevel& lv : c->levels[ph])
                 for (int i = lv.first; i < lv.first + lv.count; ++i)
                     if (!stays[i] && !(sweep && last_plane[i])) live.push_back(i);
-            schedule_pieces(c, src, live, ph == 2 ? std::vector<int>{m + 1, 2 * m + 1} : std::vector<int>{2 * m}, descs,
-                            cells, pieces, blocks, out);
+            const int stress_cuts[BC_CUTS] = {m + 1, 2 * m + 1}, velocity_cuts[1] = {2 * m};
+            schedule_pieces(c, src, live, ph == 2 ? stress_cuts : velocity_cuts, ph == 2 ? BC_CUTS : 1, descs, cells,
+                            pieces, blocks, out);
         }
 }
 
@@ -1260,7 +1277,7 @@ void destroy(OpesciContext* c) {
             if (c->base[f][l]) (void)hipFree(c->base[f][l]);
     for (int i = 0; i < OPESCI_M_COUNT; ++i)
         if (c->mbase[i]) (void)hipFree(c->mbase[i]);
-    void* ptrs[] = {c->d_program, c->d_code,    c->d_sol, c->d_soltab, c->d_partial, c->d_stage, c->d_rec, c->d_at_src,
+    void* ptrs[] = {c->d_program, c->d_code,    c->d_sol, c->d_soltab, c->d_partial, c->d_stage, c->d_rec,
                     c->d_trace, c->d_wavelet, c->d_step, c->d_pool,    c->d_dterms, c->d_gpool,
                     c->d_log,   c->d_ckpt,    c->d_seg,  c->d_obs,     c->d_srclog, c->d_tcells,
                     c->d_vcells, c->d_scells, c->d_zcoef, c->d_zpool, c->d_gather, c->d_abuf};
@@ -1390,7 +1407,13 @@ int create(const OpesciModelDesc* d, OpesciContext** out) {
     if (c->nrec || c->src_ntr) {
         if (int e = alloc_zero(c.get(), (void**)&c->d_step, 256)) return e;
         if (c->nrec) {
-            if (int e = upload(&c->d_rec, d->rec_idx, (size_t)3 * c->nrec, c->stream)) return e;
+            // the receivers' points, then the numbers of those in the source's cell
+            std::vector<int32_t> rec(d->rec_idx, d->rec_idx + (size_t)3 * c->nrec);
+            for (int r = 0; r < c->nrec && c->src_ntr; ++r)
+                if (std::equal(d->src_idx, d->src_idx + 3, d->rec_idx + 3 * r)) rec.push_back(r);
+            c->nat_src = (int)rec.size() - 3 * c->nrec;
+            if (int e = upload(&c->d_rec, rec.data(), rec.size(), c->stream)) return e;
+            c->d_at_src = c->d_rec + (size_t)3 * c->nrec;
             c->h_rec.assign(d->rec_idx, d->rec_idx + (size_t)3 * c->nrec);
             const size_t tb = (size_t)std::max(d->ntsteps, 1) * c->nrec * 4 * d->real_bytes;
             if (int e = alloc_zero(c.get(), (void**)&c->d_trace, tb)) return e;
@@ -1399,11 +1422,6 @@ int create(const OpesciModelDesc* d, OpesciContext** out) {
             if (int e = upload(&c->d_wavelet, d->src_wavelet, (size_t)std::max(d->ntsteps, 1) * c->src_ntr, c->stream))
                 return e;
             for (int a = 0; a < 3; ++a) c->src_idx[a] = d->src_idx[a];
-            std::vector<int32_t> at;
-            for (int r = 0; r < c->nrec; ++r)
-                if (std::equal(c->src_idx, c->src_idx + 3, c->h_rec.data() + 3 * r)) at.push_back(r);
-            c->nat_src = (int)at.size();
-            if (int e = upload(&c->d_at_src, at.data(), at.size(), c->stream)) return e;
         }
     }
     // pointers into the caller's arrays are not kept

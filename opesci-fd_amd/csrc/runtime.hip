@@ -59,7 +59,7 @@ struct OpesciContext {
     const BcBlock* d_blocks = nullptr; // their block lists
     int zero_last = 0;
     bool left_out = false;             // some statement is in none of the runs (zero_stays)
-    int full_steps = 0;                // steps that still run every statement (after an upload)
+    int full_steps = 0;                // steps that still run every statement (after a velocity's upload)
     const BcDesc* d_desc = nullptr;
     char* d_program = nullptr;         // all three
     std::vector<BcDesc> h_desc;       // host copy of the descriptors (adjoint cell lists)
@@ -327,8 +327,8 @@ CellBox read_by(const OpesciBcStmt& s, const OpesciBcTerm& t) {
 // already there, as pieces (schedule_pieces).
 //   * A statement without terms writes zeros.  In ghost cells that nothing
 //     else writes, those cells hold zeros from the second step after an init
-//     (which clears both levels) or an upload (whose two next steps run every
-//     statement) on: dead.  At orders 2, 6 and 8 these are all velocity
+//     (which clears both levels) or a velocity's upload (whose two next steps
+//     run every statement) on: dead.  At orders 2, 6 and 8 these are all velocity
 //     statements but the ones of the next item.
 //   * When every velocity statement is of that kind, those on the staggered
 //     field's last interior plane (U at x = nx - m - 1, V and W alike) are the

@@ -14,10 +14,11 @@
 // per CU) measured 248 us against 239 on the 256^3 read path and 147 against
 // 128 us for FP16; loads two planes ahead instead of one, and blocks of 256
 // or 1024 threads, gained nothing; z tiles that do not start on a line cost
-// 81 us against 58 at 160^3.  Measured before -> after (events, us): 256^3
-// 4th order FP32 with the z faces 223 -> 204, read path 253 -> 239, FP16 278
-// -> 128; 128^3 4th order FP64 read path 82 -> 57; 160^3 FP32 107 -> 61; 161
-// x 129 x 193 8th order BF16 read path 103 -> 79; 16^3 26 -> 7.
+// 81 us against 58 at 160^3.  Measured before -> now (events, us), now with the
+// z faces in every one and rows of 9 lines at 256^3: 256^3 4th order FP32 223
+// (z faces in it) -> 190, read path 253 -> 258 (226 without the z faces), FP16
+// 278 -> 125; 128^3 4th order FP64 read path 82 -> 60; 160^3 FP32 107 -> 61; 161
+// x 129 x 193 8th order BF16 read path 103 -> 87; 16^3 26 -> 7.
 //
 // The z-face statements of the deep rows are done here for every type and
 // medium: as launches they touch a line per point and statement.  Sweep +

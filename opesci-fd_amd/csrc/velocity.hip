@@ -7,10 +7,10 @@
 // reads and 3 writes per point, 48 bytes in FP32), the chain of one plane on
 // small ones, instructions with 16-bit storage; 58-65 registers at 4th order
 // in FP32.  Measured before (two points per lane in 128-point tiles, FP64 one)
-// -> after (events, us): 256^3 4th order FP32 159 -> 160, read path 204 ->
-// 187, FP16 142 -> 89, 8th order read path 222 -> 206; 160^3 93 -> 44; 161 x
-// 129 x 193 8th order BF16 read path 89 -> 67; 61 x 47 x 53 8th order FP64 30
-// -> 13; 16^3 27 -> 8.
+// -> now (events, us; rows of 9 lines instead of 10 at 256^3): 256^3 4th order
+// FP32 159 -> 154, read path 204 -> 181, FP16 142 -> 84, 8th order read path
+// 222 -> 191; 160^3 93 -> 44; 161 x 129 x 193 8th order BF16 read path 89 ->
+// 66; 61 x 47 x 53 8th order FP64 30 -> 12; 16^3 27 -> 7.
 #include "sweep.h"
 
 namespace opesci {

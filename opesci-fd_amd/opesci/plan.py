@@ -527,8 +527,8 @@ def _build_bc(grid, slots):
     b.seq = list(range(len(b.stmts)))
     b.fused_frame = 0
     # split by default: the stress sweep applies the deep rows in place
-    # (fuse_boundary True splits too, but off FP32 arithmetic on constant media
-    # leaves the rows to a launch of their own, which tests compare with)
+    # (fuse_boundary True splits too, but without the description's flag: the
+    # library then keeps the older, narrower rule for them, which tests hold)
     if getattr(grid, 'fuse_boundary', True):
         dims = [d.value for d in grid.dim]
         b.fused_frame = b.fuse_z(2, 4, dims, grid.margin.value)
